@@ -638,8 +638,7 @@ template <typename T, int S, int ZS, bool PRE = false> struct EpiDuFinal {
       for (int i = 0; i < NSS; ++i) ss += (pt % LPC + i * LPC < h) ? ssv[i] : 0.f;
 #pragma unroll
       for (int j = 0; j < CPT; ++j) pv[ZS][j] = tile[r * LDT + c0 + j];
-#pragma unroll
-      for (int x = 1; x < LPC; x <<= 1) ss += __shfl_xor(ss, x, 64);
+      ss = lanes_sum<1, LPC / 2>(ss);
       const float rr = rsqrtf(ss * inv_d + eps);
       float g[CPT], dot = 0.f;
 #pragma unroll
@@ -652,8 +651,7 @@ template <typename T, int S, int ZS, bool PRE = false> struct EpiDuFinal {
         dot += g[j] * ov[j];
         tile[r * LDT + c0 + j] = m < M ? du * ov[j] * rr : 0.f;
       }
-#pragma unroll
-      for (int x = 1; x < LPC; x <<= 1) dot += __shfl_xor(dot, x, 64);
+      dot = lanes_sum<1, LPC / 2>(dot);
       if (m < M) {
         store_vec<float, CPT>(gw + (long)m * d + col, g);
         if (pt % LPC == 0) rowdot[(long)m * (d / DU_EPI_TN) + col / DU_EPI_TN] = dot;
@@ -830,8 +828,8 @@ DM_DEV void attn_bwd_body(const AttnBwdArgs<T>& a, int L, int nbh) {
       ss = sum_strided<MAX_HEADS / 4>(a.ssq + n * g.h, part, g.h, 4);
       dot = sum_strided<MAX_ROWDOT / 4>(a.rowdot + n * a.nrd, part, a.nrd, 4);
     }
-    ss += __shfl_xor(ss, 1, 64); ss += __shfl_xor(ss, 2, 64);
-    dot += __shfl_xor(dot, 1, 64); dot += __shfl_xor(dot, 2, 64);
+    ss = lanes_sum<1, 2>(ss);
+    dot = lanes_sum<1, 2>(dot);
     const float r = rsqrtf(ss * a.inv_d + a.eps);
     const float c3 = r * r * r * a.inv_d * dot;
     const float Mi = ok ? a.stat_m[(long)bh * c + i] : 0.f;
@@ -845,9 +843,9 @@ DM_DEV void attn_bwd_body(const AttnBwdArgs<T>& a, int L, int nbh) {
       sq += q[e] * ks[e];
       dov += dO[e] * vr[e];
     }
-    Dp += __shfl_xor(Dp, 1, 64); Dp += __shfl_xor(Dp, 2, 64);
-    sq += __shfl_xor(sq, 1, 64); sq += __shfl_xor(sq, 2, 64);
-    dov += __shfl_xor(dov, 1, 64); dov += __shfl_xor(dov, 2, 64);
+    Dp = lanes_sum<1, 2>(Dp);
+    sq = lanes_sum<1, 2>(sq);
+    dov = lanes_sum<1, 2>(dov);
     // raw self column: p_self = exp(s_self - M) / Z, dS_self = p_self (dO.v_raw - D)
     const float ps = ok ? __expf(sq * a.scale - Mi) / Zi : 0.f;
     const float dss = ps * (dov - Dp);

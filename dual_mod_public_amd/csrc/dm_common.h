@@ -124,6 +124,12 @@ template <typename V> DM_DEV void settle_raw(const V& v) {
   for (int i = 0; i < (int)(sizeof(V) / 4); ++i) asm volatile("" ::"v"(x.w[i]));
 }
 
+// settle_raw of one loaded vector (2 to 16 bytes)
+template <typename V> DM_DEV void settle_item(const V& v) {
+  if constexpr (sizeof(V) < 4) asm volatile("" ::"v"((uint32_t)v));
+  else settle_raw(v);
+}
+
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -160,6 +166,57 @@ template <typename T> DM_DEV void st4(T* p, const float* in) {
   } else {
     *reinterpret_cast<floatx4*>(p) = floatx4{in[0], in[1], in[2], in[3]};
   }
+}
+// V consecutive storage elements (V = 1, 2, 4, 8; at most 16 bytes) as one load / store, and V fp32
+template <typename T, int V> struct RawV {
+  static constexpr int W = (int)sizeof(T) * V / 4;
+  static_assert(W == 1 || W == 2 || W == 4, "4, 8 or 16 bytes");
+  typedef unsigned int type __attribute__((ext_vector_type(W)));
+};
+template <> struct RawV<bf16, 1> { typedef unsigned short type; };
+template <int V> struct FloatV { typedef float type __attribute__((ext_vector_type(V))); };
+template <> struct FloatV<1> { typedef float type; };
+template <typename T, int V> DM_DEV void unpackv(const typename RawV<T, V>::type& r, float (&out)[V]) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) out[i] = __uint_as_float(r[i]);
+  } else if constexpr (V == 1) {
+    out[0] = __uint_as_float((unsigned)r << 16);
+  } else {
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i) {
+      out[2 * i] = __uint_as_float(r[i] << 16);
+      out[2 * i + 1] = __uint_as_float(r[i] & 0xffff0000u);
+    }
+  }
+}
+template <int V> DM_DEV void unpackfv(const typename FloatV<V>::type& v, float (&out)[V]) {
+  if constexpr (V == 1) out[0] = v;
+  else {
+#pragma unroll
+    for (int i = 0; i < V; ++i) out[i] = v[i];
+  }
+}
+template <typename T, int V> DM_DEV typename RawV<T, V>::type packv(const float (&in)[V]) {
+  typename RawV<T, V>::type r;
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) r[i] = __float_as_uint(in[i]);
+  } else if constexpr (V == 1) {
+    r = __builtin_bit_cast(uint16_t, (bf16)in[0]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i)
+      r[i] = (uint32_t)__builtin_bit_cast(uint16_t, (bf16)in[2 * i]) |
+             ((uint32_t)__builtin_bit_cast(uint16_t, (bf16)in[2 * i + 1]) << 16);
+  }
+  return r;
+}
+template <typename T, int V> DM_DEV void stv(T* p, const float (&in)[V]) {
+  *reinterpret_cast<typename RawV<T, V>::type*>(p) = packv<T, V>(in);
+}
+template <typename T, int V> DM_DEV void stv_nt(T* p, const float (&in)[V]) {   // store_vec_nt's hint
+  __builtin_nontemporal_store(packv<T, V>(in), reinterpret_cast<typename RawV<T, V>::type*>(p));
 }
 // 8 consecutive storage elements: one 16-byte load of bf16, two of fp32
 template <typename T> struct Raw8 {
@@ -242,34 +299,64 @@ constexpr float HEAD_NORM_EPS = 1e-6f;
 DM_DEV float head_norm_r(float ss, float inv_dh) { return rsqrtf(ss * inv_dh + HEAD_NORM_EPS); }
 
 // ---- wave reductions (full 64-lane and within 16-lane groups) ----------------
+// One step of a butterfly: v combined with lane ^ O's. Inside a 16-lane row the partner comes by a
+// DPP move (xor 1, 2: quad permutations; 8: a rotation by 8; 4: the half-row mirror, xor 7, then a
+// quad reversal, xor 3), across rows by gfx950's lane swaps, which give both halves of the pair at
+// once. The LDS crossbar (ds_bpermute, what __shfl_xor compiles to) costs a round trip of over 100
+// clocks per step, and these reductions are chains of 2 to 6 steps on the critical path of every
+// attention and epilogue kernel. Every lane of the group is active where these are called.
+template <int CTRL> DM_DEV float dpp_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+struct LanePair {
+  float a, b;
+};
+template <int O> DM_DEV LanePair lane_pair(float v) {
+  if constexpr (O == 1) return {v, dpp_move<0xB1>(v)};           // quad_perm 1 0 3 2
+  else if constexpr (O == 2) return {v, dpp_move<0x4E>(v)};      // quad_perm 2 3 0 1
+  else if constexpr (O == 4) return {v, dpp_move<0x1B>(dpp_move<0x141>(v))};   // row_half_mirror, quad_perm 3 2 1 0
+  else if constexpr (O == 8) return {v, dpp_move<0x128>(v)};     // row_ror 8
+  else {
+    static_assert(O == 16 || O == 32, "butterfly step");
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    if constexpr (O == 16) {
+      const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+      return {__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1])};
+    } else {
+      const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      return {__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1])};
+    }
+  }
+}
+template <int O> DM_DEV float xor_sum(float v) {
+  const LanePair p = lane_pair<O>(v);
+  return p.a + p.b;
+}
+template <int O> DM_DEV float xor_max(float v) {
+  const LanePair p = lane_pair<O>(v);
+  return fmaxf(p.a, p.b);
+}
+// sum / max over lanes l, l ^ LO, ... up to xor HI (ascending powers of two from LO to HI)
+template <int LO, int HI> DM_DEV float lanes_sum(float v) {
+  if constexpr (LO <= HI) return lanes_sum<2 * LO, HI>(xor_sum<LO>(v));
+  else return v;
+}
+template <int LO, int HI> DM_DEV float lanes_max(float v) {
+  if constexpr (LO <= HI) return lanes_max<2 * LO, HI>(xor_max<LO>(v));
+  else return v;
+}
 // sum over aligned groups of G consecutive lanes (G a power of two <= 64)
 template <int G> DM_DEV float group_sum(float v) {
   static_assert(G >= 1 && G <= 64 && (G & (G - 1)) == 0, "lane group");
-#pragma unroll
-  for (int o = 1; o < G; o <<= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return lanes_sum<1, G / 2>(v);
 }
 DM_DEV float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return xor_sum<1>(xor_sum<2>(xor_sum<4>(xor_sum<8>(xor_sum<16>(xor_sum<32>(v))))));
 }
-DM_DEV float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
+DM_DEV float wave_max(float v) { return lanes_max<1, 32>(v); }
 // reduce across the 16 lanes that share lane>>4 (xor over the low 4 bits)
-DM_DEV float group16_max(float v) {
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-DM_DEV float group16_sum(float v) {
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
+DM_DEV float group16_max(float v) { return lanes_max<1, 8>(v); }
+DM_DEV float group16_sum(float v) { return xor_sum<1>(xor_sum<2>(xor_sum<4>(xor_sum<8>(v)))); }
 
 // ---- MFMA traits -------------------------------------------------------------
 // 16x16 output tile; lane l holds D[4*(l>>4) + r][l & 15], r = 0..3.

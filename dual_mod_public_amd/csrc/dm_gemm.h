@@ -93,7 +93,6 @@ template <typename T> struct SrcRowsRs {
     float v[MAX_HEADS / 2];   // the loaded partials (summed in prepare_store, so no wait here)
   };
   // 256 / R adjacent threads per row split its nparts (<= MAX_HEADS) partial sums
-  template <int R> static constexpr int prepare_loads() { return MAX_HEADS / (256 / R); }
   template <int R> DM_DEV Pre prepare_load(int r0, int) const {
     constexpr int P = 256 / R, Q = MAX_HEADS / P;
     static_assert(256 % R == 0 && P >= 2 && P <= 8, "rows per block");
@@ -101,7 +100,10 @@ template <typename T> struct SrcRowsRs {
     const float* row = ssq + (long)r * nparts;
     Pre pr;
 #pragma unroll
-    for (int i = 0; i < Q; ++i) pr.v[i] = row[min(part + i * P, nparts - 1)];
+    for (int i = 0; i < Q; ++i) {
+      pr.v[i] = 0.f;
+      if (i * P < nparts) pr.v[i] = row[min(part + i * P, nparts - 1)];   // uniform
+    }
     return pr;
   }
   template <int R> DM_DEV void prepare_store(const Pre& pr, float* rs_lds, T*, int) const {
@@ -110,8 +112,7 @@ template <typename T> struct SrcRowsRs {
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < Q; ++i) s += part + i * P < nparts ? pr.v[i] : 0.f;
-#pragma unroll
-    for (int o = 1; o < P; o <<= 1) s += __shfl_xor(s, o, 64);
+    s = lanes_sum<1, P / 2>(s);
     if (threadIdx.x % P == 0) rs_lds[threadIdx.x / P] = rsqrtf(s * inv_d + eps);
   }
   DM_DEV const T* ptr(int r, int k) const { return p + (long)min(r, rows - 1) * ld + k; }
@@ -137,11 +138,6 @@ template <class S> struct requires_prepare { static constexpr bool value = false
 template <typename T> struct requires_prepare<SrcRowsRs<T>> { static constexpr bool value = true; };
 struct NoPre {};
 template <class S> struct PrepOf { using type = NoPre; };
-// vector-memory loads of a source's prepare_load (row scales), 0 for plain sources
-template <class S, int BM> constexpr int prepare_loads_of() {
-  if constexpr (requires_prepare<S>::value) return S::template prepare_loads<BM>();
-  else return 0;
-}
 template <typename T> struct PrepOf<SrcRowsRs<T>> { using type = typename SrcRowsRs<T>::Pre; };
 
 // Tile epilogues: an EPI with a member type TilePre gathers its global inputs with
@@ -156,6 +152,20 @@ template <typename T> struct PrepOf<SrcRowsRs<T>> { using type = typename SrcRow
 // large for one LDS tile still store whole rows.
 template <class E, class = void> struct has_tile_epi { static constexpr bool value = false; };
 template <class E> struct has_tile_epi<E, std::void_t<typename E::TilePre>> { static constexpr bool value = true; };
+// An EPI with a static KINDS has its tile epilogue in KINDS forms, one per block (epi.kind(n0), uniform):
+// KindEpi<E, KD> is form KD as a tile epilogue of its own.
+template <class E, class = void> struct kinds_of { static constexpr int value = 0; };
+template <class E> struct kinds_of<E, std::void_t<decltype(E::KINDS)>> { static constexpr int value = E::KINDS; };
+template <class E, int KD> struct KindEpi {
+  const E& e;
+  typedef typename E::template TilePre<KD> TilePre;
+  static constexpr int LATE_GATHERS = E::template late_gathers<KD>();
+  DM_DEV TilePre tile_prefetch(int m0, int n0) const { return e.template tile_prefetch<KD>(m0, n0); }
+  template <int BM, int BN, int LDT>
+  DM_DEV void tile_apply(const float* tile, int m0, int n0, const float* rs, const TilePre& pre, int) const {
+    e.template tile_apply<KD, BM, BN, LDT>(tile, m0, n0, rs, pre);
+  }
+};
 template <class E, class = void> struct tile_rows_of { static constexpr int value = 1 << 30; };
 // An EPI with a static LATE_GATHERS = the exact number of vector-memory load instructions its
 // tile_prefetch issues gets them issued late in the direct-to-LDS k-loop (gemm_mainloop_dma).
@@ -663,6 +673,14 @@ constexpr int gemm_block_lds() {
 // 1024-byte aligned).
 template <typename T, int BM, int BN, int WM, int WN, int D, class SA, class SB, class EPI>
 DM_DEV void gemm_block_at(const SA& sa, const SB& sb, int K, const EPI& epi, int bx, int by, int bz, char* smem) {
+  if constexpr (kinds_of<EPI>::value > 0) {
+    static_assert(kinds_of<EPI>::value == 4, "four kinds");
+    const int kd = epi.kind(bx * BN);   // uniform
+    if (kd == 0) gemm_block_at<T, BM, BN, WM, WN, D>(sa, sb, K, KindEpi<EPI, 0>{epi}, bx, by, bz, smem);
+    else if (kd == 1) gemm_block_at<T, BM, BN, WM, WN, D>(sa, sb, K, KindEpi<EPI, 1>{epi}, bx, by, bz, smem);
+    else if (kd == 2) gemm_block_at<T, BM, BN, WM, WN, D>(sa, sb, K, KindEpi<EPI, 2>{epi}, bx, by, bz, smem);
+    else gemm_block_at<T, BM, BN, WM, WN, D>(sa, sb, K, KindEpi<EPI, 3>{epi}, bx, by, bz, smem);
+  } else {
   using WT = WaveTile<BM, BN, WM, WN>;
   constexpr bool RMS = requires_prepare<SA>::value;
   constexpr bool KM = SA::KMAJOR && SB::KMAJOR && D < 0;
@@ -677,8 +695,8 @@ DM_DEV void gemm_block_at(const SA& sa, const SB& sb, int K, const EPI& epi, int
 #pragma unroll
     for (int j = 0; j < WT::FN; ++j) acc[i][j] = zero4();
   // Row scales (row-scaled operands feed tile epilogues only): their inputs are
-  // loaded first and the scales are staged in LDS after the k-loop, so no wait on
-  // them, or on the epilogue's gathers issued after them, precedes the k-loop.
+  // loaded first, ahead of the operand stages, and the scales are staged in LDS after
+  // the k-loop.
   static_assert(!RMS || has_tile_epi<EPI>::value, "row-scaled operands need a tile epilogue");
   typename PrepOf<SA>::type pre_a{};
   if constexpr (has_tile_epi<EPI>::value) {
@@ -688,12 +706,10 @@ DM_DEV void gemm_block_at(const SA& sa, const SB& sb, int K, const EPI& epi, int
     static_assert(TR * LDT * 4 <= gemm_stage_bytes<T, BM, BN, D, KM>(), "output chunk fits the stages");
     typename EPI::TilePre pre;
     if constexpr (late_gathers_of<EPI>::value > 0 && D < 0 && !KM) {
-      // the gathers (and row-scale loads) are issued with the k-loop's last stage
-      constexpr int G = late_gathers_of<EPI>::value + prepare_loads_of<SA, BM>();
-      auto late = [&]() {
-        if constexpr (RMS) pre_a = sa.template prepare_load<BM>(m0, K);
-        pre = epi.tile_prefetch(m0, n0);
-      };
+      // the gathers are issued with the k-loop's last stage
+      constexpr int G = late_gathers_of<EPI>::value;
+      if constexpr (RMS) pre_a = sa.template prepare_load<BM>(m0, K);
+      auto late = [&]() { pre = epi.tile_prefetch(m0, n0); };
       gemm_mainloop_dma<T, BM, BN, WM, WN, -D, G>(sa, sb, K, m0, n0, smem, acc, bz * K, late);
     } else {
       if constexpr (RMS) pre_a = sa.template prepare_load<BM>(m0, K);
@@ -733,6 +749,7 @@ DM_DEV void gemm_block_at(const SA& sa, const SB& sb, int K, const EPI& epi, int
   } else {
     gemm_kloop<T, BM, BN, WM, WN, D>(sa, sb, K, m0, n0, smem, acc, bz * K);
     epi(acc, row0, col0, rs, bz);
+  }
   }
 }
 

@@ -300,23 +300,10 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
       if (seg <= 1) {
         const int r0 = DEVPOS ? dev_position(pos_dev, pos_cap) : rope_t0;
         const long rrow = (long)(r0 + t) * (DH / 2) + jj;
-        float c[4], s[4], o1[4], o2[4];
+        float c[4], s[4];
         unpackf4(ld_global<floatx4>(cos + rrow), c);
         unpackf4(ld_global<floatx4>(sin + rrow), s);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          o1[i] = a[i] * c[i] - b[i] * s[i];
-          o2[i] = b[i] * c[i] + a[i] * s[i];
-        }
-        if (seg == 0) {
-          st4<T>(qr + hrow, o1);
-          st4<T>(qr + hrow + DH / 2, o2);
-        } else {
-          st4<T>(kraw + hrow, a);
-          st4<T>(kraw + hrow + DH / 2, b);
-          st4<T>(kself + hrow, o1);
-          st4<T>(kself + hrow + DH / 2, o2);
-        }
+        rope_item(seg, hrow, a, b, c, s);
       } else if (vgain != nullptr) {
         float ya[4], yb[4];
 #pragma unroll
@@ -368,22 +355,28 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
         const float a[4] = {av.x, av.y, av.z, av.w}, b[4] = {bv.x, bv.y, bv.z, bv.w};
         const int bb = m / Tl, t = m - bb * Tl;
         const long hrow = (((long)bb * h + hh) * Tbuf + buf_t0 + t) * DH + jj;
-        float o1[4], o2[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          o1[i] = a[i] * cs[pass][i] - b[i] * sn[pass][i];
-          o2[i] = b[i] * cs[pass][i] + a[i] * sn[pass][i];
-        }
-        if (seg == 0) {
-          st4<T>(qr + hrow, o1);
-          st4<T>(qr + hrow + DH / 2, o2);
-        } else {
-          st4<T>(kraw + hrow, a);
-          st4<T>(kraw + hrow + DH / 2, b);
-          st4<T>(kself + hrow, o1);
-          st4<T>(kself + hrow + DH / 2, o2);
-        }
+        rope_item(seg, hrow, a, b, cs[pass], sn[pass]);
       }
+    }
+  }
+
+  // four RoPE pairs (a, b) of a q (rotated) or k (raw and rotated) row, at element hrow of the head buffers
+  DM_DEV void rope_item(int seg, long hrow, const float (&a)[4], const float (&b)[4], const float (&c)[4],
+                        const float (&s)[4]) const {
+    float o1[4], o2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o1[i] = a[i] * c[i] - b[i] * s[i];
+      o2[i] = b[i] * c[i] + a[i] * s[i];
+    }
+    if (seg == 0) {
+      st4<T>(qr + hrow, o1);
+      st4<T>(qr + hrow + DH / 2, o2);
+    } else {
+      st4<T>(kraw + hrow, a);
+      st4<T>(kraw + hrow + DH / 2, b);
+      st4<T>(kself + hrow, o1);
+      st4<T>(kself + hrow + DH / 2, o2);
     }
   }
 
@@ -424,19 +417,23 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
     for (int pass = 0; pass < TR / RP; ++pass) {
       const int r = threadIdx.x / L + pass * RP, m = m0 + r;
       if (m >= M) continue;
-      const floatx4 v = *reinterpret_cast<const floatx4*>(tl + r * LDT + e);
-      const int bb = m / Tl, t = m - bb * Tl;
-      const long xrow = (long)bb * Tbuf + buf_t0 + t;
-      float o[4] = {v.x + bs[0], v.y + bs[1], v.z + bs[2], v.w + bs[3]};
-      if (seg <= 4) {
-        st4<T>(glogx + xrow * 2 * d + (seg - 3) * d + col, o);
-      } else {
-        if (!fusion) {
+      gate_item(seg, m, col, *reinterpret_cast<const floatx4*>(tl + r * LDT + e), bs);
+    }
+  }
+
+  // four columns of a gate / v_gate row
+  DM_DEV void gate_item(int seg, int m, int col, const floatx4& v, const float (&bs)[4]) const {
+    const int bb = m / Tl, t = m - bb * Tl;
+    const long xrow = (long)bb * Tbuf + buf_t0 + t;
+    float o[4] = {v.x + bs[0], v.y + bs[1], v.z + bs[2], v.w + bs[3]};
+    if (seg <= 4) {
+      st4<T>(glogx + xrow * 2 * d + (seg - 3) * d + col, o);
+    } else {
+      if (!fusion) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = sigmoidf_(o[i]);
-        }
-        st4<T>(sig + xrow * d + col, o);
+        for (int i = 0; i < 4; ++i) o[i] = sigmoidf_(o[i]);
       }
+      st4<T>(sig + xrow * d + col, o);
     }
   }
 };
@@ -876,6 +873,149 @@ template <typename T, int DH, int NW> struct AttendBody {
 };
 
 // ---------------------------------------------------------------------------
+// The read of one chunk row q of every (b, h), for a cell run one row at a time (run_cell: the
+// exact scan): committed state (merged), the refined rows [0, q) of the chunk, the raw self pair.
+// One wave per (b, h); the 16 rows of its MFMA tile are all row q, and the products, the softmax
+// and the sums are those of attend_rows, so row q's result is the one a whole sweep gives. Keys come
+// as MFMA fragments straight from global memory; only V (transposed reads) and the probabilities go
+// through LDS. Bound by latency: one round of loads, then a chain of ~1500 cycles.
+// Writes o [B, d] and ssq [B, h] (one row per batch element), ocat / o_last rows of row q.
+// ---------------------------------------------------------------------------
+template <typename T, int DH>
+DM_DEV void attend_row(const AttendArgs<T>& a, int bh, int q, T* lds) {
+  static_assert(sizeof(T) == 2, "bf16 fragments");
+  using C = AttnCfg<T, DH>;
+  using MF = Mfma<T>;
+  T* Vs = lds;                      // [64][LDK]
+  T* Pr = Vs + C::KT * C::LDK;      // [64]
+  const CellGeom& g = a.g;
+  const int b = bh / g.h, hh = bh - b * g.h;
+  const int lane = threadIdx.x & 63, g4 = lane >> 4, col = lane & 15;
+  const long lrow = (long)bh * g.Tbuf + g.buf_t0 + q;   // layer-buffer row
+  const T* Kb = a.Kin + (long)bh * a.in_stride + (long)a.in_row0 * DH;
+  const T* Vb = a.Vin + (long)bh * a.in_stride + (long)a.in_row0 * DH;
+  const int nt = (q + 15) >> 4;     // key tiles with a kept key (uniform)
+  constexpr int VPR = DH / 8, NV = VPR;
+  constexpr int PER = DH / 16;
+
+  typename MF::frag qf[C::NKS], kf[4][C::NKS];
+#pragma unroll
+  for (int ks = 0; ks < C::NKS; ++ks) qf[ks] = MF::load(a.qr + lrow * DH + ks * MF::KSTEP + g4 * MF::KPL);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (t < nt) {
+#pragma unroll
+      for (int ks = 0; ks < C::NKS; ++ks)
+        kf[t][ks] = MF::load(Kb + (long)min(col + 16 * t, q - 1) * DH + ks * MF::KSTEP + g4 * MF::KPL);
+    }
+  uint4 vr[NV];   // rows [0, q) of V; passes of 64 / VPR rows
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int v = lane + 64 * i, k = v / VPR, c0 = (v % VPR) * 8;
+    if (64 / VPR * i < 32 * ((q + 31) >> 5)) vr[i] = *reinterpret_cast<const uint4*>(Vb + (long)min(k, max(q - 1, 0)) * DH + c0);
+  }
+  float m = NEG_INF, z = 0.f;
+  floatx4 O[C::NDT];
+#pragma unroll
+  for (int dt = 0; dt < C::NDT; ++dt) O[dt] = zero4();
+  if (a.merged_in) {
+    const long o = (long)bh * g.c + q;
+    m = a.Mx[o];
+    z = (col == 0) ? a.Z[o] : 0.f;
+#pragma unroll
+    for (int dt = 0; dt < C::NDT; ++dt) O[dt][0] = a.A[o * DH + col + 16 * dt];
+  }
+  float dot = 0.f, vself[C::NDT];
+  {
+    const T* qp = a.qr + lrow * DH + col * PER;
+    const T* kp = a.kself + lrow * DH + col * PER;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) dot += to_f(qp[e]) * to_f(kp[e]);
+    const T* vp = a.vraw + lrow * DH;
+#pragma unroll
+    for (int dt = 0; dt < C::NDT; ++dt) vself[dt] = to_f(vp[col + 16 * dt]);
+  }
+  if (q > 0) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int v = lane + 64 * i, k = v / VPR, c0 = (v % VPR) * 8;
+      if (64 / VPR * i < 32 * ((q + 31) >> 5)) *reinterpret_cast<uint4*>(Vs + k * C::LDK + c0) = keep_if(vr[i], k < q);
+    }
+    const KeyStrictLower keep{0, intra_wlim(g.window)};
+    float S[4], mx = NEG_INF;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      S[t] = NEG_INF;
+      if (t < nt) {
+        floatx4 s4 = zero4();
+#pragma unroll
+        for (int ks = 0; ks < C::NKS; ++ks) s4 = MF::mma(qf[ks], kf[t][ks], s4);
+        S[t] = keep(q, col + 16 * t) ? s4[0] * a.scale : NEG_INF;
+      }
+      mx = fmaxf(mx, S[t]);
+    }
+    mx = group16_max(mx);
+    const float mnew = fmaxf(m, mx);
+    const float alpha = (m == NEG_INF) ? 0.f : __expf(m - mnew);
+    m = mnew;
+    z *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < C::NDT; ++dt) O[dt][0] *= alpha;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float p = (S[t] == NEG_INF) ? 0.f : __expf(S[t] - mnew);
+      z += p;
+      if (g4 == 0) Pr[col + 16 * t] = from_f<T>(p);
+    }
+    __syncthreads();   // the block is this one wave
+#pragma unroll
+    for (int kb = 0; kb < C::NPS; ++kb)
+      if (MF::KSTEP * kb < q) {   // uniform: past q every probability is 0
+        const typename MF::frag pf = MF::load(Pr + kb * MF::KSTEP + g4 * MF::KPL);
+#pragma unroll
+        for (int dt = 0; dt < C::NDT; ++dt)
+          O[dt] = MF::mma(pf, MF::load_tr(Vs + kb * MF::KSTEP * C::LDK + 16 * dt, C::LDK), O[dt]);
+      }
+  }
+  {   // raw self column
+    const float ss = group16_sum(dot) * a.scale;
+    const float mnew = fmaxf(m, ss);
+    const float alpha = (m == NEG_INF) ? 0.f : __expf(m - mnew);
+    const float es = __expf(ss - mnew);
+#pragma unroll
+    for (int dt = 0; dt < C::NDT; ++dt) O[dt][0] = O[dt][0] * alpha + es * vself[dt];
+    z = z * alpha + (col == 0 ? es : 0.f);
+    m = mnew;
+  }
+  const float inv = 1.0f / group16_sum(z);
+  float sq = 0.f, ov[C::NDT];
+#pragma unroll
+  for (int dt = 0; dt < C::NDT; ++dt) {
+    ov[dt] = to_f(from_f<T>(O[dt][0] * inv));   // the stored (rounded) value
+    sq += ov[dt] * ov[dt];
+  }
+  sq = group16_sum(sq);
+  // the four 16-lane groups hold the same row: group g4 stores the column tiles g4, g4 + 4, ...
+#pragma unroll
+  for (int d4 = 0; d4 < C::NDT; d4 += 4) {
+    float v = ov[d4];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) v = g4 == i ? ov[d4 + i] : v;
+    const int cc = hh * DH + col + 16 * (d4 + g4);
+    a.o[(long)b * g.d + cc] = from_f<T>(v);
+    if (a.o_last != nullptr) a.o_last[((long)b * g.c + q) * g.d + cc] = v;
+    if (a.ocat != nullptr) a.ocat[((long)b * g.Tbuf + g.buf_t0 + q) * g.d + cc] = from_f<T>(v);
+  }
+  if (lane == 0) a.ssq[(long)b * g.h + hh] = sq;
+}
+
+template <typename T, int DH>
+static __global__ __launch_bounds__(64) void k_attend_row(AttendArgs<T> a, int q) {
+  __shared__ __attribute__((aligned(16))) T lds[AttnCfg<T, DH>::KT * AttnCfg<T, DH>::LDK + AttnCfg<T, DH>::KT];
+  attend_row<T, DH>(a, blockIdx.x, q, lds);
+}
+
+// ---------------------------------------------------------------------------
 // sweep GEMM 1: u . W_sweep^T (u = RMSNorm_ctx(o) on the A load)
 // (attention.py:314-387; fused_sweep.py:514-611, :1064-1089). W_sweep rows are
 // packed in 64-row groups so that one wave's 16 x 64 tile is self-contained:
@@ -907,247 +1047,269 @@ template <typename T, int DH, int NG = 1, bool DEVPOS = false, bool SPLIT = fals
   const float* __restrict__ kgain = nullptr;
   const float* __restrict__ vgain = nullptr;
 
-  // Block tile 64 x 64 NG: NG packed column groups of 64. Thread t owns row t / 4 and the
-  // column quad lc0 = 4 (t % 4) .. + 3 of each group's four 16-column sections, so its global
-  // inputs and outputs are runs of 4 consecutive elements. With up to two groups the inputs
-  // are gathered during the k-loop's last stage; with more, at the start of the epilogue.
-  // SPLIT: a 512-thread block of two groups (eight waves), each 256-thread half owning one
+  // ---- one row's items --------------------------------------------------------------------------
+  // Every 64-column group is of one kind (uniform over a block), which decides what an item gathers:
+  // K and the linear V take the same V columns of each of the group's four 16-column sections, v_map
+  // and g_v are plain columns, V of them in a row.
+  enum Kind { K_ROWS = 0, LIN_V = 1, V_MAP = 2, G_V = 3 };
+  DM_DEV int kind(int n0) const {
+    return n0 < 2 * g.d ? K_ROWS : (ctx_mod == 0 ? LIN_V : (n0 < 3 * g.d ? V_MAP : G_V));
+  }
+  template <int V> struct KPre {
+    typename RawV<T, V>::type x[2], h[2];   // gate x-halves, raw key: both RoPE halves
+    typename FloatV<V>::type f[2];          // cos, sin
+  };
+  template <int V> struct LPre { typename RawV<T, V>::type x[2], h[2]; };      // gate x-halves, raw value
+  template <int V> struct MPre { typename RawV<T, V>::type sg, ov, nw; };      // sig, o, norm weight
+  DM_DEV void row_of(int row, int& m, int& b, int& p, int& t) const {
+    m = min(row, M - 1);
+    b = m / g.c;
+    p = m - b * g.c;
+    t = g.buf_t0 + p;
+  }
+  // columns lc0 .. lc0 + V - 1 of the sections of group n0 (K)
+  template <int V> DM_DEV KPre<V> k_prefetch(int row, int n0, int lc0) const {
+    typedef typename RawV<T, V>::type R;
+    int m, b, p, t;
+    row_of(row, m, b, p, t);
+    const int pos = DEVPOS ? dev_position(g.pos_dev, g.pos_cap) + p : rope_row(g, p);
+    const int hd = n0 / (2 * DH), jj = 16 * ((n0 % (2 * DH)) / 64) + lc0;
+    const T* x = glogx + ((long)b * g.Tbuf + t) * 2 * g.d + hd * DH + jj;
+    const T* k = kraw + (((long)b * g.h + hd) * g.Tbuf + t) * DH + jj;
+    KPre<V> pr;
+    pr.x[0] = ld_global<R>(x);
+    pr.x[1] = ld_global<R>(x + DH / 2);
+    pr.f[0] = ld_global<typename FloatV<V>::type>(cos + (long)pos * (DH / 2) + jj);
+    pr.f[1] = ld_global<typename FloatV<V>::type>(sin + (long)pos * (DH / 2) + jj);
+    pr.h[0] = ld_global<R>(k);
+    pr.h[1] = ld_global<R>(k + DH / 2);
+    return pr;
+  }
+  template <int V, class SAVE>
+  DM_DEV void k_apply(const float (&a)[4][V], int m, int n0, int lc0, const KPre<V>& pr, const SAVE& save_raw) const {
+    float gxa[V], gxb[V], cs[V], sn[V], ka[V], kb[V];
+    unpackv<T, V>(pr.x[0], gxa); unpackv<T, V>(pr.x[1], gxb); unpackfv<V>(pr.f[0], cs); unpackfv<V>(pr.f[1], sn);
+    unpackv<T, V>(pr.h[0], ka); unpackv<T, V>(pr.h[1], kb);
+    settle(gxa); settle(gxb); settle(cs); settle(sn); settle(ka); settle(kb);   // all loads before any store
+    if (m >= M) return;
+    save_raw();
+    const int b = m / g.c, p = m - b * g.c;
+    const int orow0 = DEVPOS ? dev_position(g.pos_dev, g.pos_cap) : out_row0;
+    const int hd = n0 / (2 * DH), jj = 16 * ((n0 % (2 * DH)) / 64) + lc0;
+    float o1[V], o2[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const float ga = sigmoidf_(gxa[i] + a[2][i]);
+      const float gb = sigmoidf_(gxb[i] + a[3][i]);
+      const float k1 = ga * ka[i] + (1.f - ga) * a[0][i];
+      const float k2 = gb * kb[i] + (1.f - gb) * a[1][i];
+      o1[i] = k1 * cs[i] - k2 * sn[i];
+      o2[i] = k2 * cs[i] + k1 * sn[i];
+    }
+    T* crow = Kout + ((long)b * g.h + hd) * out_stride + (long)(orow0 + p) * DH + jj;
+    stv<T, V>(crow, o1);
+    stv<T, V>(crow + DH / 2, o2);
+  }
+  // columns lc0 .. lc0 + V - 1 of the sections of group n0 (linear V)
+  template <int V> DM_DEV LPre<V> l_prefetch(int row, int n0, int lc0) const {
+    typedef typename RawV<T, V>::type R;
+    int m, b, p, t;
+    row_of(row, m, b, p, t);
+    const int cl = n0 - 2 * g.d, hd = cl / (2 * DH), e = 32 * ((cl % (2 * DH)) / 64) + lc0;
+    const T* x = glogx + ((long)b * g.Tbuf + t) * 2 * g.d + g.d + hd * DH + e;
+    const T* v = vraw + (((long)b * g.h + hd) * g.Tbuf + t) * DH + e;
+    LPre<V> pr;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      pr.x[j] = ld_global<R>(x + 16 * j);
+      pr.h[j] = ld_global<R>(v + 16 * j);
+    }
+    return pr;
+  }
+  template <int V, class SAVE>
+  DM_DEV void l_apply(const float (&a)[4][V], int m, int n0, int lc0, const LPre<V>& pr, const SAVE& save_raw) const {
+    float gx[2][V], vr[2][V];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) { unpackv<T, V>(pr.x[j], gx[j]); unpackv<T, V>(pr.h[j], vr[j]); settle(gx[j]); settle(vr[j]); }
+    if (m >= M) return;
+    save_raw();
+    const int b = m / g.c, p = m - b * g.c;
+    const int orow0 = DEVPOS ? dev_position(g.pos_dev, g.pos_cap) : out_row0;
+    const int cl = n0 - 2 * g.d, hd = cl / (2 * DH), e = 32 * ((cl % (2 * DH)) / 64) + lc0;
+    T* crow = Vout + ((long)b * g.h + hd) * out_stride + (long)(orow0 + p) * DH + e;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float v[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        v[i] = value_blend(g, hd * DH + e + 16 * j + i, sigmoidf_(gx[j][i] + a[j + 2][i]), vr[j][i], a[j][i]);
+      stv<T, V>(crow + 16 * j, v);
+    }
+  }
+  // columns col .. col + V - 1 of v_map (col from 0)
+  template <int V> DM_DEV MPre<V> m_prefetch(int row, int col) const {
+    typedef typename RawV<T, V>::type R;
+    int m, b, p, t;
+    row_of(row, m, b, p, t);
+    return MPre<V>{ld_global<R>(sig + ((long)b * g.Tbuf + t) * g.d + col), ld_global<R>(o + (long)m * g.d + col),
+                   ld_global<R>(normw + col)};
+  }
+  template <int V> DM_DEV void m_settle(const MPre<V>& pr) const { settle_item(pr.sg); settle_item(pr.ov); settle_item(pr.nw); }
+  template <int V> DM_DEV void m_apply(const float (&a)[V], float sc, int m, int col, const MPre<V>& pr) const {
+    float sg[V], ov[V], nw[V], v[V];
+    unpackv<T, V>(pr.sg, sg); unpackv<T, V>(pr.ov, ov); unpackv<T, V>(pr.nw, nw);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      if (ctx_mod == 3) {   // fusion (attention.py:341-342): u + silu(v_pre x-half + u-half)
+        const float z = sg[i] + a[i];
+        v[i] = ov[i] * sc * nw[i] + z * sigmoidf_(z);
+      } else {
+        v[i] = sg[i] * tanhf_(a[i]);
+        if (ctx_mod == 1) v[i] += lam * (ov[i] * sc * nw[i]);
+      }
+    }
+    stv<T, V>(vin + (long)m * g.d + col, v);
+  }
+
+  // ---- block tiles ------------------------------------------------------------------------------
+  // Block tile 64 x 64 NG: NG packed column groups of 64. Thread t owns row t / 4; of a sectioned
+  // group (K, linear V) the column quad 4 (t % 4) .. + 3 of each section, of v_map and g_v 16
+  // consecutive columns. Inputs and outputs are runs of 4 or 8 consecutive elements. With up to two
+  // groups the inputs are gathered during the k-loop's last stage; with more, at the start of the
+  // epilogue. SPLIT: a 512-thread block of two groups (eight waves), each 256-thread half owning one
   // group (threads t and t + 256 the same row and quad); no per-head norms.
+  // A gather of 16 rows occupies the CU's vector-memory path for 16 to 32 clocks whatever its width,
+  // so a block issues what its kind reads and no more (6 loads per thread and group for K and v_map,
+  // 4 for the linear V, none for g_v; 14 + 16 of the row scales' before, most of them repeats).
   static_assert(!SPLIT || NG == 2, "split: two groups, one per 256-thread half");
   static constexpr int NGT = SPLIT ? 1 : NG;   // groups per thread
+  static constexpr int VM = 16 / (int)sizeof(T), NM = 16 / VM;   // v_map / g_v: items of VM columns per group
+  static constexpr bool LATE = NG <= 2;
   DM_DEV static int trow() { return (SPLIT ? (int)(threadIdx.x & 255) : (int)threadIdx.x) >> 2; }
   DM_DEV static int tquad() { return threadIdx.x & 3; }
   DM_DEV static int tgroup() { return SPLIT ? (int)(threadIdx.x >> 8) : 0; }
-  struct GroupPre {
-    typename Raw4<T>::type x[4];    // K: gx_a, gx_b; linear V: gx x2; v_map: sig x4 (storage dtype)
-    floatx4 f[2];                   // K: cos, sin
-    typename Raw4<T>::type h[8];    // K: kraw_a, kraw_b; linear V: v_raw x2; v_map: o x4, norm weight x4
-  };
-  static constexpr bool LATE = NG <= 2;
-  struct TilePre {
-    GroupPre p[LATE ? NGT : 1];
-  };
-  // tile_prefetch issues exactly 14 loads per group of the thread (one per x / f / h slot,
-  // unconditionally)
-  static constexpr int LATE_GATHERS = LATE ? 14 * NGT : 0;
-  DM_DEV TilePre tile_prefetch(int m0, int n0) const {
-    TilePre pr{};
+  // a block's epilogue, by the kind of its groups (gemm_block_at)
+  static constexpr int KINDS = 4;
+  struct GK { typedef std::integral_constant<int, K_ROWS> kd; KPre<4> v; };
+  struct GL { typedef std::integral_constant<int, LIN_V> kd; LPre<4> v; };
+  struct GM { typedef std::integral_constant<int, V_MAP> kd; MPre<VM> v[NM]; };
+  struct GG { typedef std::integral_constant<int, G_V> kd; };
+  template <int KD>
+  using GroupPre = std::conditional_t<KD == K_ROWS, GK, std::conditional_t<KD == LIN_V, GL, std::conditional_t<KD == V_MAP, GM, GG>>>;
+  template <int KD> struct TilePre { GroupPre<KD> p[LATE ? NGT : 1]; };
+  // exactly as many loads as group_prefetch issues (none can be merged: no two are adjacent, or each is 16 bytes)
+  template <int KD> static constexpr int late_gathers() {
+    return !LATE ? 0 : NGT * (KD == K_ROWS ? 6 : (KD == LIN_V ? 4 : (KD == V_MAP ? 3 * NM : 0)));
+  }
+  template <int KD> DM_DEV TilePre<KD> tile_prefetch(int m0, int n0) const {
+    TilePre<KD> pr{};
     if constexpr (LATE) {
 #pragma unroll
-      for (int gi = 0; gi < NGT; ++gi) pr.p[gi] = group_prefetch(m0, n0 + 64 * (gi + tgroup()));
+      for (int gi = 0; gi < NGT; ++gi) load_group(pr.p[gi], m0, n0 + 64 * (gi + tgroup()));
     }
-    return pr;
-  }
-  DM_DEV GroupPre group_prefetch(int m0, int n0) const {
-    const int r = trow(), lc0 = 4 * tquad();
-    const int d = g.d, h = g.h;
-    const int m = min(m0 + r, M - 1);
-    const int b = m / g.c, p = m - b * g.c;
-    const int t = g.buf_t0 + p, pos = DEVPOS ? dev_position(g.pos_dev, g.pos_cap) + p : rope_row(g, p);
-    const long xrow = (long)b * g.Tbuf + t;
-    // The (block-uniform) branches only pick addresses; the loads follow them
-    // unconditionally (unused slots re-read a valid address), so no loaded value
-    // has to be merged, and waited for, where the branches join.
-    const T* xp[4];
-    const float* fp[2];
-    const T* hp[8];
-    const T* x0 = glogx + xrow * 2 * d;
-    const T* h0 = kraw + ((long)b * h * g.Tbuf + t) * DH;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) xp[k] = x0;
-    fp[0] = cos + (long)pos * (DH / 2);
-    fp[1] = sin + (long)pos * (DH / 2);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) hp[k] = h0;
-    if (n0 < 2 * d) {
-      const int hd = n0 / (2 * DH), jj = 16 * ((n0 % (2 * DH)) / 64) + lc0;
-      const long lrow = (((long)b * h + hd) * g.Tbuf + t) * DH + jj;
-      xp[0] = x0 + hd * DH + jj;
-      xp[1] = xp[0] + DH / 2;
-      fp[0] += jj;
-      fp[1] += jj;
-      hp[0] = kraw + lrow;
-      hp[1] = hp[0] + DH / 2;
-    } else if (ctx_mod == 0) {
-      const int cl = n0 - 2 * d;
-      const int hd = cl / (2 * DH), e = 32 * ((cl % (2 * DH)) / 64) + lc0;
-      const long lrow = (((long)b * h + hd) * g.Tbuf + t) * DH + e;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        xp[j] = x0 + d + hd * DH + e + 16 * j;
-        hp[j] = vraw + lrow + 16 * j;
-      }
-    } else if (n0 < 3 * d) {
-      const int c0 = n0 - 2 * d + lc0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) xp[k] = sig + xrow * d + c0 + 16 * k;
-      if (ctx_mod == 1 || ctx_mod == 3) {   // mult_res, fusion: v_in has a u term
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          hp[k] = o + (long)m * d + c0 + 16 * k;
-          hp[4 + k] = normw + c0 + 16 * k;
-        }
-      }
-    }
-    GroupPre pr;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) pr.x[k] = ld_global<typename Raw4<T>::type>(xp[k]);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) pr.f[k] = ld_global<floatx4>(fp[k]);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) pr.h[k] = ld_global<typename Raw4<T>::type>(hp[k]);
     return pr;
   }
 
-  template <int BM, int BN, int LDT>
-  DM_DEV void tile_apply(const float* tile, int m0, int n0, const float* rs, const TilePre& pr, int) const {
+  template <int KD, int BM, int BN, int LDT>
+  DM_DEV void tile_apply(const float* tile, int m0, int n0, const float* rs, const TilePre<KD>& pr) const {
     static_assert(BM == 64 && BN == 64 * NG, "sweep GEMM 1 block tile is NG 64 x 64 column groups");
     const float sc = rs[trow()];
+    const float* srow = tile + trow() * LDT;
     if constexpr (NG == 1) {
-      group_apply<LDT>(tile, m0, n0, sc, pr.p[0], false, 0.f, 0.f);
+      thread_apply<KD>(srow, m0, n0, sc, pr.p[0], false, 0.f, 0.f);
     } else if constexpr (SPLIT) {
-      group_apply<LDT>(tile + 64 * tgroup(), m0, n0 + 64 * tgroup(), sc, pr.p[0], false, 0.f, 0.f);
+      thread_apply<KD>(srow + 64 * tgroup(), m0, n0 + 64 * tgroup(), sc, pr.p[0], false, 0.f, 0.f);
     } else {
-      GroupPre pg[NG];
+      GroupPre<KD> pg[NG];
 #pragma unroll
       for (int gi = 0; gi < NG; ++gi) {
         if constexpr (LATE) pg[gi] = pr.p[gi];
-        else pg[gi] = group_prefetch(m0, n0 + 64 * gi);
+        else load_group(pg[gi], m0, n0 + 64 * gi);
       }
       // The block's NG groups are one head's k_ctx / g_k(u) (or linear v_ctx / g_v(u)) columns:
       // the head's norm scale r * gain from sections 0 and 1 of every group (the k_ctx, v_ctx
       // columns), over the row's 4 threads.
-      const int r = trow(), lc0 = 4 * tquad();
-      const int d = g.d;
-      const float* gain = nullptr;
-      int hd = 0;
-      if (n0 < 2 * d) { gain = kgain; hd = n0 / (2 * DH); }
-      else if (ctx_mod == 0) { gain = vgain; hd = (n0 - 2 * d) / (2 * DH); }
+      const float* gain = KD == K_ROWS ? kgain : (KD == LIN_V ? vgain : nullptr);
       float nr = 0.f, ng = 0.f;
       if (gain != nullptr) {
+        const int lc0 = 4 * tquad();
         float ss = 0.f;
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi)
 #pragma unroll
           for (int k = 0; k < 2; ++k) {
-            const floatx4 v = *reinterpret_cast<const floatx4*>(tile + r * LDT + 64 * gi + 16 * k + lc0);
+            const floatx4 v = *reinterpret_cast<const floatx4*>(srow + 64 * gi + 16 * k + lc0);
             const float x0 = stored<T>(v.x * sc), x1 = stored<T>(v.y * sc);
             const float x2 = stored<T>(v.z * sc), x3 = stored<T>(v.w * sc);
             ss += x0 * x0 + x1 * x1 + x2 * x2 + x3 * x3;
           }
-        ss += __shfl_xor(ss, 1, 64);
-        ss += __shfl_xor(ss, 2, 64);
+        ss = lanes_sum<1, 2>(ss);
         nr = head_norm_r(ss, 1.0f / DH);
-        ng = gain[hd];
+        ng = gain[(KD == K_ROWS ? n0 : n0 - 2 * g.d) / (2 * DH)];
       }
 #pragma unroll
       for (int gi = 0; gi < NG; ++gi)
-        group_apply<LDT>(tile + 64 * gi, m0, n0 + 64 * gi, sc, pg[gi], gain != nullptr, nr, ng);
+        thread_apply<KD>(srow + 64 * gi, m0, n0 + 64 * gi, sc, pg[gi], gain != nullptr, nr, ng);
     }
   }
 
-  // One 64-column group of the tile (tile points at the group's first column). nrm: the group's
-  // k_ctx / v_ctx columns are normed, x -> (x nr) ng, from and to stored values.
-  template <int LDT>
-  DM_DEV void group_apply(const float* tile, int m0, int n0, float sc, const GroupPre& pr, bool nrm, float nr,
-                          float ng) const {
-    const int r = trow(), lc0 = 4 * tquad();
-    const int d = g.d, h = g.h;
-    const int m = m0 + r;
-    // the GEMM ran on o with norm_ctx.weight folded into W: u . W^T = rs * acc
-    float a[4][4];
+  DM_DEV void load_group(GK& p, int m0, int n0) const { p.v = k_prefetch<4>(m0 + trow(), n0, 4 * tquad()); }
+  DM_DEV void load_group(GL& p, int m0, int n0) const { p.v = l_prefetch<4>(m0 + trow(), n0, 4 * tquad()); }
+  DM_DEV void load_group(GM& p, int m0, int n0) const {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const floatx4 v = *reinterpret_cast<const floatx4*>(tile + r * LDT + 16 * k + lc0);
-      a[k][0] = v.x * sc; a[k][1] = v.y * sc; a[k][2] = v.z * sc; a[k][3] = v.w * sc;
-    }
-    // raw outputs for the tape: this thread's 16 consecutive columns of row r
+    for (int k = 0; k < NM; ++k) p.v[k] = m_prefetch<VM>(m0 + trow(), n0 - 2 * g.d + 16 * tquad() + VM * k);
+  }
+  DM_DEV void load_group(GG&, int, int) const {}
+
+  // The thread's part of the group n0 whose row is staged at srow. nrm: the group's k_ctx / v_ctx
+  // columns are normed, x -> (x nr) ng, from and to stored values.
+  template <int KD>
+  DM_DEV void thread_apply(const float* srow, int m0, int n0, float sc, const GroupPre<KD>& pr, bool nrm, float nr,
+                           float ng) const {
+    const int m = m0 + trow(), q = tquad();
+    // this thread's 16 consecutive columns: raw outputs for the tape, and v_map's / g_v's own
     float sv[16];
-    if (save != nullptr) {
-      const int cs0 = 16 * tquad();
+    if (KD >= V_MAP || save != nullptr) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const floatx4 v = *reinterpret_cast<const floatx4*>(tile + r * LDT + cs0 + 4 * k);
+        const floatx4 v = *reinterpret_cast<const floatx4*>(srow + 16 * q + 4 * k);
         sv[4 * k] = v.x * sc; sv[4 * k + 1] = v.y * sc; sv[4 * k + 2] = v.z * sc; sv[4 * k + 3] = v.w * sc;
       }
     }
-    if (NG > 1 && nrm) {   // normed k_ctx / v_ctx (sections 0 and 1)
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a[k][i] = stored<T>((stored<T>(a[k][i]) * nr) * ng);
-    }
-    if (m >= M) return;
-    const int b = m / g.c, p = m - b * g.c;
-    const int orow0 = DEVPOS ? dev_position(g.pos_dev, g.pos_cap) : out_row0;
-    if (n0 < 2 * d) {
-      float gxa[4], gxb[4], cs[4], sn[4], ka[4], kb[4];
-      unpack4<T>(pr.x[0], gxa); unpack4<T>(pr.x[1], gxb); unpackf4(pr.f[0], cs); unpackf4(pr.f[1], sn);
-      unpack4<T>(pr.h[0], ka); unpack4<T>(pr.h[1], kb);
-      settle(gxa); settle(gxb); settle(cs); settle(sn); settle(ka); settle(kb);   // all loads before any store
-      if (save != nullptr) store_vec_nt<T, 16>(save + (long)m * 4 * d + n0 + 16 * tquad(), sv);
-      const int hd = n0 / (2 * DH), jj = 16 * ((n0 % (2 * DH)) / 64) + lc0;
-      float o1[4], o2[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float ga = sigmoidf_(gxa[i] + a[2][i]);
-        const float gb = sigmoidf_(gxb[i] + a[3][i]);
-        const float k1 = ga * ka[i] + (1.f - ga) * a[0][i];
-        const float k2 = gb * kb[i] + (1.f - gb) * a[1][i];
-        o1[i] = k1 * cs[i] - k2 * sn[i];
-        o2[i] = k2 * cs[i] + k1 * sn[i];
-      }
-      T* crow = Kout + ((long)b * h + hd) * out_stride + (long)(orow0 + p) * DH + jj;
-      st4<T>(crow, o1);
-      st4<T>(crow + DH / 2, o2);
-    } else if (ctx_mod == 0) {
-      float gx[2][4], vr[2][4];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) { unpack4<T>(pr.x[j], gx[j]); unpack4<T>(pr.h[j], vr[j]); settle(gx[j]); settle(vr[j]); }
-      if (save != nullptr) store_vec_nt<T, 16>(save + (long)m * 4 * d + n0 + 16 * tquad(), sv);
-      const int cl = n0 - 2 * d;
-      const int hd = cl / (2 * DH), e = 32 * ((cl % (2 * DH)) / 64) + lc0;
-      T* crow = Vout + ((long)b * h + hd) * out_stride + (long)(orow0 + p) * DH + e;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          v[i] = value_blend(g, hd * DH + e + 16 * j + i, sigmoidf_(gx[j][i] + a[j + 2][i]), vr[j][i], a[j][i]);
-        st4<T>(crow + 16 * j, v);
-      }
-    } else if (n0 < 3 * d) {
-      float sg[4][4], ov[4][4], nw[4][4];
+    auto save_raw = [&]() {
+      if (save != nullptr) store_vec_nt<T, 16>(save + (long)m * 4 * g.d + n0 + 16 * q, sv);
+    };
+    if constexpr (KD <= LIN_V) {
+      // the GEMM ran on o with norm_ctx.weight folded into W: u . W^T = rs * acc
+      float a[4][4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        unpack4<T>(pr.x[k], sg[k]);
-        settle(sg[k]);
-        if (ctx_mod == 1 || ctx_mod == 3) {
-          unpack4<T>(pr.h[k], ov[k]); unpack4<T>(pr.h[4 + k], nw[k]); settle(ov[k]); settle(nw[k]);
-        }
+        const floatx4 v = *reinterpret_cast<const floatx4*>(srow + 16 * k + 4 * q);
+        a[k][0] = v.x * sc; a[k][1] = v.y * sc; a[k][2] = v.z * sc; a[k][3] = v.w * sc;
       }
-      if (save != nullptr) store_vec_nt<T, 16>(save + (long)m * 4 * d + n0 + 16 * tquad(), sv);
-      const int c0 = n0 - 2 * d + lc0;
+      if (NG > 1 && nrm) {   // normed k_ctx / v_ctx (sections 0 and 1)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        float v[4];
+        for (int k = 0; k < 2; ++k)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (ctx_mod == 3) {   // fusion (attention.py:341-342): u + silu(v_pre x-half + u-half)
-            const float z = sg[k][i] + a[k][i];
-            v[i] = ov[k][i] * sc * nw[k][i] + z * sigmoidf_(z);
-          } else {
-            v[i] = sg[k][i] * tanhf_(a[k][i]);
-            if (ctx_mod == 1) v[i] += lam * (ov[k][i] * sc * nw[k][i]);
-          }
-        }
-        st4<T>(vin + (long)m * d + c0 + 16 * k, v);
+          for (int i = 0; i < 4; ++i) a[k][i] = stored<T>((stored<T>(a[k][i]) * nr) * ng);
       }
+      if constexpr (KD == K_ROWS) k_apply<4>(a, m, n0, 4 * q, pr.v, save_raw);
+      else l_apply<4>(a, m, n0, 4 * q, pr.v, save_raw);
     } else {
-      if (save != nullptr) store_vec_nt<T, 16>(save + (long)m * 4 * d + n0 + 16 * tquad(), sv);
-      const int c0 = n0 - 3 * d + lc0;
+      if constexpr (KD == V_MAP) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) st4<T>(gvu + (long)m * d + c0 + 16 * k, a[k]);
+        for (int k = 0; k < NM; ++k) m_settle<VM>(pr.v[k]);   // all loads before any store
+      }
+      if (m >= M) return;
+      save_raw();
+#pragma unroll
+      for (int k = 0; k < NM; ++k) {
+        float a[VM];
+#pragma unroll
+        for (int i = 0; i < VM; ++i) a[i] = sv[VM * k + i];
+        if constexpr (KD == V_MAP) m_apply<VM>(a, sc, m, n0 - 2 * g.d + 16 * q + VM * k, pr.v[k]);
+        else stv<T, VM>(gvu + (long)m * g.d + n0 - 3 * g.d + 16 * q + VM * k, a);
+      }
     }
   }
 };
@@ -1172,6 +1334,38 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiSweep2 {
   // vector-memory load instructions tile_prefetch issues (Raw8 = one 16-byte load in bf16, two in
   // fp32: 16-byte loads, which the compiler cannot merge into fewer)
   static constexpr int LATE_GATHERS = 3 * (int)(sizeof(T) / 2);
+  // V consecutive columns of one row, from col
+  template <int V> struct ItemPre {
+    typename RawV<T, V>::type gx, gu, vr;
+  };
+  template <int V> DM_DEV ItemPre<V> item_prefetch(int row, int col) const {
+    typedef typename RawV<T, V>::type R;
+    const int m = min(row, M - 1);
+    const int b = m / g.c, t = g.buf_t0 + m - b * g.c;
+    const int hd = col / DH, e = col - hd * DH;
+    return ItemPre<V>{ld_global<R>(glogx + ((long)b * g.Tbuf + t) * 2 * g.d + g.d + col),
+                      ld_global<R>(gvu + (long)m * g.d + col),
+                      ld_global<R>(vraw + (((long)b * g.h + hd) * g.Tbuf + t) * DH + e)};
+  }
+  // v_ctx of the item at `at` (in the staged tile)
+  template <int V> DM_DEV void item_apply(const float* at, int m, int col, const ItemPre<V>& pr) const {
+    float a[V], gx[V], gu[V], vr[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) a[i] = at[i];
+    unpackv<T, V>(pr.gx, gx);
+    unpackv<T, V>(pr.gu, gu);
+    unpackv<T, V>(pr.vr, vr);
+    if (m >= M) return;
+    settle(gx); settle(gu); settle(vr);   // all loads before any store
+    const int b = m / g.c, p = m - b * g.c;
+    const int hd = col / DH, e = col - hd * DH;
+    float v[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) v[i] = value_blend(g, col + i, sigmoidf_(gx[i] + gu[i]), vr[i], a[i]);
+    const int orow0 = DEVPOS ? dev_position(g.pos_dev, g.pos_cap) : out_row0;
+    stv<T, V>(Vout + ((long)b * g.h + hd) * out_stride + (long)(orow0 + p) * DH + e, v);
+    if (save2 != nullptr) stv_nt<T, V>(save2 + (long)m * g.d + col, a);
+  }
   DM_DEV TilePre tile_prefetch(int m0, int n0) const {
     const int r = threadIdx.x >> 2, col = n0 + 8 * (threadIdx.x & 3);
     const int m = min(m0 + r, M - 1);
@@ -1289,8 +1483,7 @@ template <typename T, int DH> struct EpiSweep2Head {
         vc[i] = stored<T>(a[i]);
         sn += vc[i] * vc[i];
       }
-      sn += __shfl_xor(sn, 1, 64);
-      sn += __shfl_xor(sn, 2, 64);
+      sn = lanes_sum<1, 2>(sn);
       const float nr = head_norm_r(sn, 1.0f / DH), ng = vgain[n0 / DH];
 #pragma unroll
       for (int i = 0; i < CW; ++i) vc[i] = stored<T>((vc[i] * nr) * ng);
@@ -1302,8 +1495,7 @@ template <typename T, int DH> struct EpiSweep2Head {
       ss += v[i] * v[i];
     }
     if (g.v_clamp_tau > 0.f) {   // norm clamp of the stored row (as k_clamp_v): the row's 4 threads
-      ss += __shfl_xor(ss, 1, 64);
-      ss += __shfl_xor(ss, 2, 64);
+      ss = lanes_sum<1, 2>(ss);
       const float n = sqrtf(ss);
       if (n > g.v_clamp_tau) {
         const float sc = g.v_clamp_tau / fmaxf(n, 1e-20f);

@@ -60,7 +60,11 @@ def dm_layer(x, cell, params, cos, sin, schedule, normalize=True, residual=True,
     sublayer y = x + W_O DM(attn_norm(x)) (default) or DualModAttention.forward's
     W_O DM(xhat). save_tape keeps every cell's sweep states from the forward
     (``cell.tape_bytes(schedule)`` of device memory) so the backward does not
-    recompute them; False trades that memory for an exact recompute."""
+    recompute them; False trades that memory for an exact recompute. Without a gradient to
+    compute (grad mode off, or no input that requires one) no state is kept: the tape's writes
+    are over half of a sweep's output, and exact cells then run row by row (K = c)."""
+    save_tape = save_tape and torch.is_grad_enabled() and (
+        x.requires_grad or any(p.requires_grad for p in params.values()))
     names = [n for n in params if normalize or n != "attn_norm.weight"]
     return DMLayerFn.apply(x, cos, sin, cell, schedule, normalize, residual, save_tape, names,
                            *[params[n] for n in names])

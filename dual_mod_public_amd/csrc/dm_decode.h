@@ -43,23 +43,18 @@ DM_DEV void dec_geometry(const DecodeArgs<T>& a, int& pos, int& lo, int& nsplit)
   nsplit = pos > lo ? (pos - lo + a.split_len - 1) / a.split_len : 0;
 }
 
+// The unnormalised state of one split's keys [k_begin, k_end) by 256 threads (tid 0 .. 255): A[DH], Z, m
+// into out[0 .. DH + 2). red is the group's LDS; block-wide barriers, so every group of a block calls it.
 template <typename T, int DH, int L>
-__global__ __launch_bounds__(256) void k_decode_partial(DecodeArgs<T> a) {
+DM_DEV void decode_split(const DecodeArgs<T>& a, int bh, int k_begin, int k_end, int tid, float (*red)[DH + 2],
+                         float* out) {
   constexpr int VEC = 16 / (int)sizeof(T);
   constexpr int LPK = DH / VEC;          // lanes per key row
   constexpr int KPP = 256 / LPK;         // keys per pass
   constexpr int NP = L / KPP;            // passes
   static_assert(L % KPP == 0, "split length");
-  const uint64_t t0 = prof_begin(a.prof_ts);
-  __shared__ float red[4][DH + 2];
-  const int s = blockIdx.x, bh = blockIdx.y;
-  int pos, lo, nsplit;
-  dec_geometry(a, pos, lo, nsplit);
-  if (s >= nsplit) return;   // whole block: past the position (device-position grids only)
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = tid >> 6;
   const int kslot = tid / LPK, part = tid - kslot * LPK;
-  const int k_begin = lo + s * a.split_len;
-  const int k_end = min(k_begin + a.split_len, pos);
 
   float qv[VEC];
   unpack16<T>(*reinterpret_cast<const uint4*>(a.q + (long)bh * DH + part * VEC), qv);
@@ -81,8 +76,7 @@ __global__ __launch_bounds__(256) void k_decode_partial(DecodeArgs<T> a) {
     float dot = 0.f;
 #pragma unroll
     for (int j = 0; j < VEC; ++j) dot += qv[j] * kv[j];
-#pragma unroll
-    for (int o = 1; o < LPK; o <<= 1) dot += __shfl_xor(dot, o, 64);
+    dot = lanes_sum<1, LPK / 2>(dot);
     const int key = k_begin + i * KPP + kslot;
     sc[i] = (key < k_end) ? dot * a.scale : NEG_INF;
     mx = fmaxf(mx, sc[i]);
@@ -92,9 +86,8 @@ __global__ __launch_bounds__(256) void k_decode_partial(DecodeArgs<T> a) {
     const int key = k_begin + i * KPP + kslot;
     raw[i] = keep_if(ld_nt(Vb + (long)(key < k_end ? key : k_begin) * DH), key < k_end);
   }
-  // block max
-#pragma unroll
-  for (int o = LPK; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  // group max
+  mx = lanes_max<LPK, 32>(mx);
   if (lane == 0) red[wave][0] = mx;
   __syncthreads();
   const float M = fmaxf(fmaxf(red[0][0], red[1][0]), fmaxf(red[2][0], red[3][0]));
@@ -114,10 +107,7 @@ __global__ __launch_bounds__(256) void k_decode_partial(DecodeArgs<T> a) {
   }
   // reduce over key slots: lanes with equal `part` inside the wave, then waves
 #pragma unroll
-  for (int o = LPK; o < 64; o <<= 1) {
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) acc[j] += __shfl_xor(acc[j], o, 64);
-  }
+  for (int j = 0; j < VEC; ++j) acc[j] = lanes_sum<LPK, 32>(acc[j]);
   // z counted once per key (all LPK lanes of a key hold the same p): use part 0
   float zz = (part == 0) ? z : 0.f;
   zz = wave_sum(zz);
@@ -127,34 +117,57 @@ __global__ __launch_bounds__(256) void k_decode_partial(DecodeArgs<T> a) {
   }
   if (lane == 0) red[wave][DH] = zz;
   __syncthreads();
-  float* out = a.part + ((long)s * (a.B * a.h) + bh) * (DH + 2);
   for (int i = tid; i < DH + 1; i += 256) out[i] = red[0][i] + red[1][i] + red[2][i] + red[3][i];
   if (tid == 0) out[DH + 1] = M;
+}
+
+template <typename T, int DH, int L>
+__global__ __launch_bounds__(256) void k_decode_partial(DecodeArgs<T> a) {
+  const uint64_t t0 = prof_begin(a.prof_ts);
+  __shared__ float red[4][DH + 2];
+  const int s = blockIdx.x, bh = blockIdx.y;
+  int pos, lo, nsplit;
+  dec_geometry(a, pos, lo, nsplit);
+  if (s >= nsplit) return;   // whole block: past the position (device-position grids only)
+  const int k_begin = lo + s * a.split_len;
+  decode_split<T, DH, L>(a, bh, k_begin, min(k_begin + a.split_len, pos), threadIdx.x, red,
+                         a.part + ((long)s * (a.B * a.h) + bh) * (DH + 2));
   prof_end(a.prof_ts, t0);
 }
 
-// merge split partials + raw self column -> o, ssq, o_cat (one wave per (b, h))
-template <typename T, int DH>
-__global__ __launch_bounds__(64) void k_decode_merge(DecodeArgs<T> a) {
+// The step's own inputs of one (b, h) for the merge, per lane of one wave
+template <int DH> struct DecodeSelf {
+  float qk, v[DH / 64];
+};
+template <typename T, int DH> DM_DEV DecodeSelf<DH> decode_self(const DecodeArgs<T>& a, int bh, int lane) {
   constexpr int PER = DH / 64;
-  const int bh = blockIdx.x, lane = threadIdx.x;
-  const int b = bh / a.h, hh = bh - b * a.h;
-  int pos, lo, nsplit;
-  dec_geometry(a, pos, lo, nsplit);
-  float qk = 0.f;
+  DecodeSelf<DH> sf;
+  sf.qk = 0.f;
 #pragma unroll
-  for (int e = 0; e < PER; ++e)
-    qk += to_f(a.q[(long)bh * DH + lane * PER + e]) * to_f(a.kself[(long)bh * DH + lane * PER + e]);
-  const float ss = wave_sum(qk) * a.scale;
+  for (int e = 0; e < PER; ++e) {
+    sf.qk += to_f(a.q[(long)bh * DH + lane * PER + e]) * to_f(a.kself[(long)bh * DH + lane * PER + e]);
+    sf.v[e] = to_f(a.vself[(long)bh * DH + lane * PER + e]);
+  }
+  return sf;
+}
+
+// merge of nsplit split states (split s at part + s pstride) and the raw self column -> o, ssq, o_cat,
+// by the 64 lanes of one wave
+template <typename T, int DH>
+DM_DEV void decode_merge(const DecodeArgs<T>& a, const DecodeSelf<DH>& sf, const float* part, long pstride, int nsplit,
+                         int bh, int lane) {
+  constexpr int PER = DH / 64;
+  const int b = bh / a.h, hh = bh - b * a.h;
+  const float ss = wave_sum(sf.qk) * a.scale;
   float M = ss;
-  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, a.part[((long)s * (a.B * a.h) + bh) * (DH + 2) + DH + 1]);
+  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, part[s * pstride + DH + 1]);
   const float es = __expf(ss - M);
   float z = es;
   float acc[PER];
 #pragma unroll
-  for (int e = 0; e < PER; ++e) acc[e] = es * to_f(a.vself[(long)bh * DH + lane * PER + e]);
+  for (int e = 0; e < PER; ++e) acc[e] = es * sf.v[e];
   for (int s = 0; s < nsplit; ++s) {
-    const float* pp = a.part + ((long)s * (a.B * a.h) + bh) * (DH + 2);
+    const float* pp = part + s * pstride;
     const float w = (pp[DH + 1] == NEG_INF) ? 0.f : __expf(pp[DH + 1] - M);
     z += w * pp[DH];
 #pragma unroll
@@ -171,6 +184,38 @@ __global__ __launch_bounds__(64) void k_decode_merge(DecodeArgs<T> a) {
   }
   sq = wave_sum(sq);
   if (lane == 0) a.ssq[(long)b * a.h + hh] = sq;
+}
+
+// merge split partials + raw self column -> o, ssq, o_cat (one wave per (b, h))
+template <typename T, int DH>
+__global__ __launch_bounds__(64) void k_decode_merge(DecodeArgs<T> a) {
+  const int bh = blockIdx.x, lane = threadIdx.x;
+  int pos, lo, nsplit;
+  dec_geometry(a, pos, lo, nsplit);
+  const DecodeSelf<DH> sf = decode_self<T, DH>(a, bh, lane);
+  decode_merge<T, DH>(a, sf, a.part + (long)bh * (DH + 2), (long)(a.B * a.h) * (DH + 2), nsplit, bh, lane);
+}
+
+// The whole read of a short tape in one launch: block = one (b, h), NS groups of 256 threads each one
+// split of L keys (the split kernel's arithmetic), their states in LDS, merged by the first wave (the
+// merge kernel's arithmetic: the same results as the two launches). A launch and a round trip of the
+// partials less; the grid is B*h blocks whatever the tape's length, so it pays while NS groups cover
+// the read and B*h blocks of them are resident together (decode_reads_direct).
+template <typename T, int DH, int L, int NS>
+__global__ __launch_bounds__(256 * NS) void k_decode_direct(DecodeArgs<T> a) {
+  __shared__ float red[NS][4][DH + 2];
+  __shared__ float part[NS][DH + 2];
+  const int bh = blockIdx.x, grp = threadIdx.x >> 8, tid = threadIdx.x & 255;
+  int pos, lo, nsplit;
+  dec_geometry(a, pos, lo, nsplit);
+  DecodeSelf<DH> sf{};
+  if (threadIdx.x < 64) sf = decode_self<T, DH>(a, bh, threadIdx.x);
+  // a group past the position reads no key (k_end = k_begin, clamped into the tape) and its state is not merged
+  const int kb = min(lo + grp * L, max(pos - 1, 0));
+  const int ke = grp < nsplit ? min(lo + (grp + 1) * L, pos) : kb;
+  decode_split<T, DH, L>(a, bh, kb, ke, tid, red[grp], part[grp]);
+  __syncthreads();
+  if (threadIdx.x < 64) decode_merge<T, DH>(a, sf, &part[0][0], DH + 2, min(nsplit, NS), bh, threadIdx.x);
 }
 
 // device position: the RoPE rows of position *pos_dev -> rope[0, half) cos, rope[half, 2 half) sin

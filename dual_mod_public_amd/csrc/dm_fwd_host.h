@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "dm_host.h"
+#include "dm_rows.h"
 
 namespace dm {
 
@@ -114,6 +115,66 @@ inline const float* v_gain(const dm_config* c, const dm_packed* w) {
   return (c->norms & DM_NORM_V) ? w->gains + 2 * c->h : nullptr;
 }
 
+// ---- wave-tile products (dm_rows.h) -----------------------------------------------------------
+// Where they are taken: bf16, M <= WT_MAX_M rows, 16-byte aligned operands, the launch issued directly
+// (not recorded for a grouped launch). Per-head norms need a whole head per block and stay on the
+// tiled GEMMs.
+template <typename T> bool wt_ok(int M, const void* A, const void* W) {
+  return sizeof(T) == 2 && M <= WT_MAX_M && launch_log() == nullptr && aligned16(A) && aligned16(W);
+}
+// f(WTile) with the tile of least expected time for M x N outputs (N a multiple of 64): a wave's
+// own time goes with its operand rows (8 NA + 16 CT; 57 ns each per 1024 of k), a CU's with the sum
+// over its waves (35 ns per row); fitted to 30 measured (M, N, tile) times, K = 512 .. 2048, M = 1 ..
+// 256, all within 15% of the best tile. max_ct: the epilogue's widest tile.
+template <class F> void with_wt(int M, int N, int max_ct, const F& f) {
+  struct C { int na, ct; };
+  constexpr C cand[] = {{1, 1}, {2, 1}, {2, 2}, {4, 1}, {4, 2}, {4, 4}};
+  int best = 0;
+  long bt = -1;
+  for (int i = 0; i < 6; ++i) {
+    if (cand[i].ct > max_ct || (i > 0 && M <= 8 * cand[i - 1].na && cand[i].na > cand[i - 1].na)) continue;
+    const long rows = 8 * cand[i].na + 16 * cand[i].ct, waves = (long)cdiv(M, 8 * cand[i].na) * (N / (16 * cand[i].ct));
+    const long t = std::max<long>(57 * rows, 35 * rows * cdiv(waves, 256));
+    if (bt < 0 || t < bt) {
+      bt = t;
+      best = i;
+    }
+  }
+  switch (best) {
+    case 0: f(WTile<1, 1>{}); break;
+    case 1: f(WTile<2, 1>{}); break;
+    case 2: f(WTile<2, 2>{}); break;
+    case 3: f(WTile<4, 1>{}); break;
+    case 4: f(WTile<4, 2>{}); break;
+    default: f(WTile<4, 4>{}); break;
+  }
+}
+// N output columns, halved for an epilogue that takes two weight rows per column (pair = 2)
+template <typename T, class E>
+void launch_wt(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls = PROF_NONE, int max_ct = 4) {
+  with_wt(op.M, N, max_ct, [&](auto wt) {
+    using WT = decltype(wt);
+    op.nx = N / WT::COLS;
+    launch_k(prof_cls, k_wt<T, WT, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64), 0, s, op, e);
+  });
+}
+template <typename T, class E1, class E2>
+void launch_wt2(WtOp<T> op1, int N1, const E1& e1, WtOp<T> op2, int N2, const E2& e2, hipStream_t s,
+                int prof_cls = PROF_NONE) {
+  with_wt(op1.M, N1 + N2, 4, [&](auto wt) {
+    using WT = decltype(wt);
+    op1.nx = N1 / WT::COLS;
+    op2.nx = N2 / WT::COLS;
+    launch_k(prof_cls, k_wt2<T, WT, E1, E2>, dim3(op1.nx + op2.nx, cdiv(op1.M, WT::ROWS)), dim3(64), 0, s, op1, e1, op2,
+             e2);
+  });
+}
+// a decode step's W_O product riding in its refine's first launch (both read o_cat)
+template <typename T> struct WtWo {
+  const T* W;
+  T* y;
+};
+
 // vpre: v_raw before the v_norm (nullptr: not kept); sa: the M input rows (x-hat);
 // small_tiles: 128 x 128 blocks even where 256 x 256 ones fit (more blocks for a short M; the
 // k-order of every output element, and so the result, is the same)
@@ -124,6 +185,25 @@ void run_proj_src(const dm_config* c, const dm_packed* w, const SA& sa, int M, i
                   int pos_cap = 0) {
   const int nseg = (c->ctx_mod == DM_CTX_LINEAR) ? 5 : 6;
   SrcRows<T> sb{(const T*)w->w_proj, c->d, nseg * c->d};
+  if constexpr (std::is_same<SA, SrcRows<bf16>>::value) {
+    if (wt_ok<T>(M, sa.p, w->w_proj) && v_gain(c, w) == nullptr) {
+      const WtOp<T> op{sa.p, sa.ld, M, c->d};
+      if (pos_dev != nullptr)
+        launch_wt(op, nseg * c->d, WtProj<T, DH, true>{(const T*)w->w_proj,
+                                              EpiProj<T, DH, true>{M, c->d, c->h, Tl, Tbuf, buf_t0, 0, cos, sin, w->b_proj,
+                                                                   qr, kraw, kself, vraw, glogx, sig,
+                                                                   c->ctx_mod == DM_CTX_FUSION, nullptr, nullptr, pos_dev,
+                                                                   pos_cap}},
+                    s, PROF_PROJ);
+      else
+        launch_wt(op, nseg * c->d, WtProj<T, DH, false>{(const T*)w->w_proj,
+                                               EpiProj<T, DH>{M, c->d, c->h, Tl, Tbuf, buf_t0, rope_t0, cos, sin,
+                                                              w->b_proj, qr, kraw, kself, vraw, glogx, sig,
+                                                              c->ctx_mod == DM_CTX_FUSION}},
+                    s, PROF_PROJ);
+      return;
+    }
+  }
   if (pos_dev != nullptr) {
     // a decode step at a device position (M <= 64 rows): the RoPE row read from device memory
     EpiProj<T, DH, true> epi{M, c->d, c->h, Tl, Tbuf, buf_t0, 0, cos, sin, w->b_proj, qr, kraw, kself, vraw,
@@ -186,12 +266,68 @@ template <typename T> struct AheadComm {
 
 // One sweep's refine: sweep GEMM 1 (+ GEMM 2 for the mult family) with the blend
 // epilogues, writing the refined rows to (Kout, Vout).
+template <typename T, int DH, bool DEVPOS>
+void launch_gemm2_wt(const dm_config* c, const dm_packed* w, const CellGeom& g, int N, const T* vraw, const T* glogx,
+                     T* Vout, long out_stride, int out_row0, const T* vin, const T* gvu, T* save2, hipStream_t s) {
+  launch_wt(WtOp<T>{vin, c->d, N, c->d}, c->d,
+            WtSweep2<T, DH, DEVPOS>{(const T*)w->w_vctx, EpiSweep2<T, DH, DEVPOS>{g, N, vraw, glogx, gvu, Vout,
+                                                                                 out_stride, out_row0, save2}},
+            s, PROF_SWEEP2);
+}
+
+template <typename T, int DH, bool DEVPOS>
+void run_refine_wt(const dm_config* c, const dm_packed* w, const CellGeom& g, int N, const T* o, const float* ssq,
+                     const T* kraw, const T* vraw, const T* glogx, const T* sig, const float* cos, const float* sin,
+                     T* Kout, T* Vout, long out_stride, int out_row0, T* vin, T* gvu, T* save1, T* save2,
+                   hipStream_t s, const WtWo<T>* wo) {
+  const int d = c->d;
+  const WtSweep1<T, DH, DEVPOS> e1{
+      (const T*)w->w_sweep,
+      EpiSweep1<T, DH, 1, DEVPOS>{g, N, c->ctx_mod, c->mult_res_lambda, kraw, vraw, glogx, sig, cos, sin, o,
+                                  (const T*)w->norm_ctx_w, Kout, Vout, out_stride, out_row0, vin, gvu, save1},
+      ssq, c->h, 1.0f / (float)d, c->rms_eps};
+  const WtOp<T> op1{o, d, N, d};
+  if (wo != nullptr)
+    launch_wt2(op1, 4 * d, e1, op1, d, WtStore<T>{wo->W, d, wo->y, N, d}, s, PROF_SWEEP1);
+  else
+    launch_wt(op1, 4 * d, e1, s, PROF_SWEEP1);
+  if (c->ctx_mod != DM_CTX_LINEAR)
+    launch_gemm2_wt<T, DH, DEVPOS>(c, w, g, N, vraw, glogx, Vout, out_stride, out_row0, vin, gvu, save2, s);
+}
+
+// The wave-tile forms apply: no per-head norm.
+template <typename T> bool refine_wt_ok(const dm_config* c, const dm_packed* w, int N, const T* o, const T* vin) {
+  return wt_ok<T>(N, o, w->w_sweep) && kctx_gain(c, w) == nullptr && vctx_gain(c, w) == nullptr &&
+         (c->ctx_mod == DM_CTX_LINEAR || (aligned16(vin) && aligned16(w->w_vctx)));
+}
+// Both GEMMs in wave tiles: up to 64 rows (one row of 64 x 64 blocks would use 4d / 64 CUs). With more
+// rows sweep GEMM 1's 64-wide block tiles are the faster ones: their epilogue touches each row of its
+// inputs in longer runs (M = 128 equal; 192: 16.8 against 11.0 us; 256: 15.8 against 13.1).
+template <typename T> bool refine_few_rows(const dm_config* c, const dm_packed* w, int N, const T* o, const T* vin) {
+  return N <= ROWS_MAX && refine_wt_ok<T>(c, w, N, o, vin);
+}
+
 template <typename T, int DH>
 void run_refine(const dm_config* c, const dm_packed* w, const CellGeom& g, int N, const T* o, const float* ssq,
                 const T* kraw, const T* vraw, const T* glogx, const T* sig, const float* cos,
                 const float* sin, T* Kout, T* Vout, long out_stride, int out_row0, T* vin, T* gvu,
                 T* save1, T* save2, hipStream_t s, const AttendArgs<T>* next_attend = nullptr,
-                bool wide = false, const AheadComm<T>* ahead = nullptr) {
+                bool wide = false, const AheadComm<T>* ahead = nullptr, const WtWo<T>* wo = nullptr) {
+  if constexpr (sizeof(T) == 2) {
+    // wo: only given where refine_few_rows holds
+    if (next_attend == nullptr && !wide && refine_few_rows<T>(c, w, N, o, vin)) {
+      if (g.pos_dev != nullptr)
+        run_refine_wt<T, DH, true>(c, w, g, N, o, ssq, kraw, vraw, glogx, sig, cos, sin, Kout, Vout, out_stride,
+                                     out_row0, vin, gvu, save1, save2, s, wo);
+      else
+        run_refine_wt<T, DH, false>(c, w, g, N, o, ssq, kraw, vraw, glogx, sig, cos, sin, Kout, Vout, out_stride,
+                                      out_row0, vin, gvu, save1, save2, s, wo);
+      if (g.v_clamp_tau > 0.f)
+        hipLaunchKernelGGL((k_clamp_v<T, DH>), dim3(cdiv((long)N * c->h, 4)), dim3(256), 0, s, g, Vout, out_stride,
+                           out_row0, N, g.v_clamp_tau);
+      return;
+    }
+  }
   const T* normw = (const T*)w->norm_ctx_w;
   SrcRowsRs<T> sa{o, c->d, N, ssq, c->h, 1.0f / (float)c->d, c->rms_eps};
   SrcRows<T> sb{(const T*)w->w_sweep, c->d, 4 * c->d};
@@ -218,9 +354,11 @@ void run_refine(const dm_config* c, const dm_packed* w, const CellGeom& g, int N
     EpiSweep1<T, DH, 1, true> e1{g, N, c->ctx_mod, c->mult_res_lambda, kraw, vraw, glogx, sig, cos, sin, o, normw,
                                  Kout, Vout, out_stride, out_row0, vin, gvu, save1};
     launch_gemm_auto<T, 64, 64, 2, 2, SW1_STAGES, 4>(sa, sb, N, 4 * c->d, c->d, e1, s, PROF_SWEEP1);
-  } else if (sizeof(T) == 2 && DM_SW1_EIGHT_WAVES && launch_log() == nullptr) {
+  } else if (sizeof(T) == 2 && DM_SW1_EIGHT_WAVES && launch_log() == nullptr &&
+             cdiv(N, 64) * (4 * c->d / 128) >= 256) {
     // bf16: 64 x 128 blocks of eight waves (each 256-thread half one 64-column group; d is a
-    // multiple of 128, so the direct-to-LDS k-loop always applies): the two column groups share
+    // multiple of 128, so the direct-to-LDS k-loop always applies) where they give every CU one (fewer:
+    // 64 x 64 blocks, 12.2 against 13.1 us at 256 rows, d = 1024): the two column groups share
     // the block's o rows, so a k-step moves 24 KB into a CU's LDS instead of the 32 KB of two
     // 64 x 64 blocks, still with eight waves per CU; the same per-element k order
     if constexpr (sizeof(T) == 2) {
@@ -265,7 +403,20 @@ void run_refine(const dm_config* c, const dm_packed* w, const CellGeom& g, int N
     launch_gemm_auto<T, 64, DH, 4, 1, S2, 4>(av, bv, N, c->d, c->d, e2, s, PROF_SWEEP2);
     return;
   }
-  if (!linear) {
+  // GEMM 2 in wave tiles where 64 x 32 blocks would not give every CU one: measured (with the sweep
+  // around it) at d = 1024 and 256 / 192 / 128 rows 6.4 / 6.0 / 4.7 us against 6.8 / 6.6 / 6.5, at d = 2048
+  // and 256 rows (256 blocks) 10.9 us in 64 x 32 blocks, 1.8 us more in wave tiles
+  bool gemm2_done = false;
+  if constexpr (sizeof(T) == 2) {
+    if (!linear && cdiv(N, 64) * (c->d / 32) < 256 && refine_wt_ok<T>(c, w, N, o, vin)) {
+      if (g.pos_dev != nullptr)
+        launch_gemm2_wt<T, DH, true>(c, w, g, N, vraw, glogx, Vout, out_stride, out_row0, vin, gvu, save2, s);
+      else
+        launch_gemm2_wt<T, DH, false>(c, w, g, N, vraw, glogx, Vout, out_stride, out_row0, vin, gvu, save2, s);
+      gemm2_done = true;
+    }
+  }
+  if (!linear && !gemm2_done) {
     SrcRows<T> av{vin, c->d, N};
     SrcRows<T> bv{(const T*)w->w_vctx, c->d, c->d};
     if (g.pos_dev != nullptr) {   // device position (see GEMM 1)
@@ -328,6 +479,18 @@ template <typename T> struct CellRows {
   int rope_t0 = -1;                 // RoPE table row of chunk row 0 (-1: pos0)
 };
 
+// k_attend over a cell's rows: 16-row waves; the (b, h) blocks split by query rows until there are
+// >= 256 blocks
+template <typename T, int DH> void launch_attend(const AttendArgs<T>& aa, int BH, hipStream_t s) {
+  if (launch_log() != nullptr) {
+    if (BH >= 256) record_launch<AttendBody<T, DH, 4>>(dim3(BH, 1), dim3(256), aa);
+    else if (BH >= 128) record_launch<AttendBody<T, DH, 2>>(dim3(BH, 2), dim3(128), aa);
+    else record_launch<AttendBody<T, DH, 1>>(dim3(BH, 4), dim3(64), aa);
+  } else if (BH >= 256) launch_k(PROF_ATTEND, k_attend<T, DH, 4>, dim3(BH, 1), dim3(256), 0, s, aa);
+  else if (BH >= 128) launch_k(PROF_ATTEND, k_attend<T, DH, 2>, dim3(BH, 2), dim3(128), 0, s, aa);
+  else launch_k(PROF_ATTEND, k_attend<T, DH, 1>, dim3(BH, 4), dim3(64), 0, s, aa);
+}
+
 // One chunk cell [pos0, pos0+cc) of the layer: n_sweeps Jacobi sweeps against the
 // committed rows [0, pos0) of the cache. Without `sv` the sweeps refine the
 // chunk's rows in place (the cache rows, or `rows`) and the last sweep leaves the final rows
@@ -366,6 +529,39 @@ int run_cell(const dm_config* c, const dm_packed* w, const dm_layer_bufs* L, con
   const bool committed = pos0 > comm_kstart(pos0, g.window);
   const long cache_stride = (long)cache_T * DH, ws_stride = (long)CMAX * DH;
   const size_t slot = (size_t)BH * CMAX * DH;
+
+  // Exact cells (K >= c) whose sweeps nobody reads back: row q is final after sweep q and a sweep's
+  // rows do not depend on each other, so step q computes row q alone, from the refined rows before
+  // it: c steps of B rows instead of c sweeps of B c, every row's arithmetic the same (the same
+  // results, bit for bit). A step is three few-row launches: measured on MI355X at B = 2, d = 512,
+  // T = 300 (DualModAttention.forward) 13 us against 21 us for a sweep of 128 rows.
+  if constexpr (sizeof(T) == 2) {
+    if (sv == nullptr && n_sweeps >= cc && cc > 1 && refine_few_rows<T>(c, w, c->B, (const T*)ws.o, (const T*)ws.vin)) {
+      AttendArgs<T> aa{g, qr, kself, vraw, Kr, Vr, rows_stride, rows_row0, 0, ws.Ap, ws.Zp, ws.Mp, ws.A, ws.Z, ws.M,
+                       scale, (T*)ws.o, ws.ssq, nullptr, nullptr, nullptr, nullptr, 0, Kc, Vc, pos0};
+      if (committed) {   // the first sweep's attention merges the committed state of every row
+        AttendArgs<T> am = aa;
+        am.Kin = kself; am.Vin = vraw; am.in_stride = (long)Tbuf * DH; am.in_row0 = buf_t0;
+        am.nsplit = nsplit;
+        am.prev_lo = prev_lo;
+        launch_attend<T, DH>(am, BH, s);
+        aa.merged_in = 1;
+      }
+      aa.ocat = ocat;
+      aa.o_last = o_last;
+      for (int q = 0; q < cc; ++q) {
+        launch_k(PROF_ATTEND, k_attend_row<T, DH>, dim3(BH), dim3(64), 0, s, aa, q);
+        CellGeom gq = g;
+        gq.c = 1;
+        gq.pos0 = pos0 + q;
+        gq.buf_t0 = buf_t0 + q;
+        if (g.rope_t0 >= 0) gq.rope_t0 = g.rope_t0 + q;
+        run_refine<T, DH>(c, w, gq, c->B, (const T*)ws.o, ws.ssq, kraw, vraw, (const T*)L->glogx, (const T*)L->sig, cos,
+                          sin, Kr, Vr, rows_stride, rows_row0 + q, (T*)ws.vin, (T*)ws.gvu, nullptr, nullptr, s);
+      }
+      return -1;
+    }
+  }
 
   // sweep s + 1's attention runs inside sweep s's GEMM 2 launch (mult family, whole 64-row
   // chunks) when B*h gives that kernel enough blocks, or when forced by the flags
@@ -435,14 +631,7 @@ int run_cell(const dm_config* c, const dm_packed* w, const dm_layer_bufs* L, con
     float* ssq = sv ? sv->ssq + sw * NS * c->h : ws.ssq;
     if (sw == 0 || !fuse) {   // else the previous sweep's GEMM 2 launch ran it
       const AttendArgs<T> aa = attend_args(sw);
-      // 16-row waves; the (b, h) blocks split by query rows until there are >= 256 blocks
-      if (launch_log() != nullptr) {
-        if (BH >= 256) record_launch<AttendBody<T, DH, 4>>(dim3(BH, 1), dim3(256), aa);
-        else if (BH >= 128) record_launch<AttendBody<T, DH, 2>>(dim3(BH, 2), dim3(128), aa);
-        else record_launch<AttendBody<T, DH, 1>>(dim3(BH, 4), dim3(64), aa);
-      } else if (BH >= 256) launch_k(PROF_ATTEND, k_attend<T, DH, 4>, dim3(BH, 1), dim3(256), 0, s, aa);
-      else if (BH >= 128) launch_k(PROF_ATTEND, k_attend<T, DH, 2>, dim3(BH, 2), dim3(128), 0, s, aa);
-      else launch_k(PROF_ATTEND, k_attend<T, DH, 1>, dim3(BH, 4), dim3(64), 0, s, aa);
+      launch_attend<T, DH>(aa, BH, s);
     }
     T* vin = sv ? sv->vin + sw * NS * d : (T*)ws.vin;
     const AttendArgs<T> next = attend_args(last ? sw : sw + 1);

@@ -5,7 +5,6 @@
 // and launch sequencing. Never allocates device memory, never synchronizes.
 #include "dm_decode.h"
 #include "dm_fwd_host.h"
-#include "dm_mlp.h"
 
 #include <mutex>
 #include <vector>
@@ -344,6 +343,28 @@ DecWs carve_dec(const dm_config* c, int tape_T, void* base) {
   return w;
 }
 
+// The tape read: one launch where NS groups of a block cover it (decode_reads_direct), else split
+// partials and their merge; the same results.
+template <typename T, int DH>
+void run_decode_read(DecodeArgs<T>& da, hipStream_t s) {
+  const int BH = da.B * da.h;
+  // One launch while a (b, h)'s splits fit one block and the chip still holds the grid: with more
+  // than one split per (b, h) each block keeps 256 threads per split resident until the slowest is
+  // done, so from 512 (b, h) up the split grid balances better.
+  if (da.nsplit >= 1 && (da.nsplit == 1 || (da.nsplit <= 4 && BH <= 512))) {
+    if (da.nsplit == 1) launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 1>, dim3(BH), dim3(256), 0, s, da);
+    else if (da.nsplit == 2) launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 2>, dim3(BH), dim3(512), 0, s, da);
+    else launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 4>, dim3(BH), dim3(1024), 0, s, da);
+    return;
+  }
+  if (da.nsplit > 0) {
+    const int idx = prof_launch_begin(PROF_DEC_READ, true, da.prof_ts);
+    launch_timed(idx, k_decode_partial<T, DH, DEC_SPLIT>, dim3(da.nsplit, BH), dim3(256), 0, s, da);
+    da.prof_ts = nullptr;
+  }
+  launch_k(PROF_DEC_MERGE, k_decode_merge<T, DH>, dim3(BH), dim3(64), 0, s, da);
+}
+
 template <typename T, int DH>
 int run_decode(const dm_config* c, const dm_packed* w, const float* cos, const float* sin,
                const dm_decode_args* a, const DecWs& ws, hipStream_t s) {
@@ -376,12 +397,7 @@ int run_decode(const dm_config* c, const dm_packed* w, const float* cos, const f
                    (const T*)ws.q, (const T*)ws.kself, (const T*)ws.vraw, (const T*)a->K_tape,
                    (const T*)a->V_tape, ws.part, ws.o, ws.ssq, (T*)a->o_cat, nullptr,
                    (const int*)a->pos_dev, window_of(c)};
-  if (nsplit > 0) {
-    const int idx = prof_launch_begin(PROF_DEC_READ, true, da.prof_ts);
-    launch_timed(idx, k_decode_partial<T, DH, DEC_SPLIT>, dim3(nsplit, B * h), dim3(256), 0, s, da);
-    da.prof_ts = nullptr;
-  }
-  launch_k(PROF_DEC_MERGE, k_decode_merge<T, DH>, dim3(B * h), dim3(64), 0, s, da);
+  run_decode_read<T, DH>(da, s);
 
   // refine_kv for the B rows (c = 1, position pos), write slot pos of the tape (device
   // position: a staging row, copied into the slot by k_decode_commit)
@@ -390,33 +406,37 @@ int run_decode(const dm_config* c, const dm_packed* w, const float* cos, const f
   g.kmod_mode = c->kmod_mode;
   g.v_clamp_tau = c->v_clamp_tau;
   ProfScope pr(PROF_DEC_REFINE, s);
+  // W_O rides in the refine's first launch where both are few-row products
+  WtWo<T> wo{(const T*)w->wo, (T*)a->y};
+  const bool wo_rides = a->y != nullptr && aligned16(w->wo) &&
+                        refine_few_rows<T>(c, w, B, (const T*)a->o_cat, (const T*)ws.vin);
+  const WtWo<T>* wop = wo_rides ? &wo : nullptr;
   if (dev_direct) {
     g.pos_dev = (const int*)a->pos_dev;
     g.pos_cap = a->tape_T;
     g.cache_T = a->tape_T;
     run_refine<T, DH>(c, w, g, B, (const T*)a->o_cat, ws.ssq, (const T*)ws.kraw, (const T*)ws.vraw,
                       (const T*)ws.glogx, (const T*)ws.sig, cos, sin, (T*)a->K_tape, (T*)a->V_tape,
-                      (long)a->tape_T * DH, 0, (T*)ws.vin, (T*)ws.gvu, nullptr, nullptr, s);
+                      (long)a->tape_T * DH, 0, (T*)ws.vin, (T*)ws.gvu, nullptr, nullptr, s, nullptr, false, nullptr, wop);
   } else if (dev_pos) {
     run_refine<T, DH>(c, w, g, B, (const T*)a->o_cat, ws.ssq, (const T*)ws.kraw, (const T*)ws.vraw,
                       (const T*)ws.glogx, (const T*)ws.sig, rc, rs, (T*)ws.kst, (T*)ws.vst, (long)DH, 0, (T*)ws.vin,
-                      (T*)ws.gvu, nullptr, nullptr, s);
+                      (T*)ws.gvu, nullptr, nullptr, s, nullptr, false, nullptr, wop);
     hipLaunchKernelGGL((k_decode_commit<T, DH>), dim3(B * h), dim3(DH), 0, s, (const int*)a->pos_dev, a->tape_T,
                        (const T*)ws.kst, (const T*)ws.vst, (T*)a->K_tape, (T*)a->V_tape);
   } else {
     run_refine<T, DH>(c, w, g, B, (const T*)a->o_cat, ws.ssq, (const T*)ws.kraw, (const T*)ws.vraw,
                       (const T*)ws.glogx, (const T*)ws.sig, cos, sin, (T*)a->K_tape, (T*)a->V_tape,
-                      (long)a->tape_T * DH, pos, (T*)ws.vin, (T*)ws.gvu, nullptr, nullptr, s);
+                      (long)a->tape_T * DH, pos, (T*)ws.vin, (T*)ws.gvu, nullptr, nullptr, s, nullptr, false, nullptr, wop);
   }
-  if (a->y != nullptr) {
+  if (a->y != nullptr && !wo_rides) {
     SrcRows<T> ao{(const T*)a->o_cat, d, B};
     SrcRows<T> bo{(const T*)w->wo, d, d};
     EpiResidual<T> ep{B, d, nullptr, (T*)a->y};
     bool done = false;
     if constexpr (sizeof(T) == 2) {
-      if (B <= MLP_ROWS && d % 32 == 0 && aligned16(a->o_cat) && aligned16(w->wo)) {
-        // bf16, one token per row: the weight-streaming product
-        launch_rows_wt<T>((const T*)a->o_cat, (const T*)w->wo, (T*)a->y, B, d, d, s);
+      if (wt_ok<T>(B, a->o_cat, w->wo)) {
+        launch_wt(WtOp<T>{(const T*)a->o_cat, d, B, d}, d, WtStore<T>{(const T*)w->wo, d, (T*)a->y, B, d}, s);
         done = true;
       }
     }
@@ -515,9 +535,7 @@ void run_attend_one(const dm_config* c, const void* q, const void* ks, const voi
   const int nsplit = P > lo ? cdiv(P - lo, DEC_SPLIT) : 0;
   DecodeArgs<T> da{B, h, d, past_T, P, lo, DEC_SPLIT, nsplit, 1.0f / sqrtf((float)DH), (const T*)q, (const T*)ks,
                    (const T*)vs, (const T*)Kp, (const T*)Vp, ws.part, ws.o, ws.ssq, (T*)o, nullptr};
-  if (nsplit > 0)
-    hipLaunchKernelGGL((k_decode_partial<T, DH, DEC_SPLIT>), dim3(nsplit, B * h), dim3(256), 0, s, da);
-  hipLaunchKernelGGL((k_decode_merge<T, DH>), dim3(B * h), dim3(64), 0, s, da);
+  run_decode_read<T, DH>(da, s);
 }
 
 template <typename T, int DH>
@@ -674,23 +692,15 @@ int dm_swiglu_rows(int32_t dtype, const void* x, const void* w1, const void* w3,
                    void* out, int32_t M, int32_t d, int32_t H, void* stream) {
   DM_REQUIRE(x && w1 && w3 && w2 && act && out, DM_ERR_INVALID, "null operand");
   DM_REQUIRE(dtype == DM_BF16, DM_ERR_UNSUPPORTED, "dm_swiglu_rows: bf16 only (dtype %d)", dtype);
-  DM_REQUIRE(M >= 1 && M <= MLP_ROWS, DM_ERR_INVALID, "M=%d (1..%d rows)", M, MLP_ROWS);
+  DM_REQUIRE(M >= 1 && M <= ROWS_MAX, DM_ERR_INVALID, "M=%d (1..%d rows)", M, ROWS_MAX);
   DM_REQUIRE(d > 0 && H > 0 && d % 128 == 0 && H % 32 == 0, DM_ERR_INVALID,
              "d=%d H=%d (d a multiple of 128, H of 32)", d, H);
   DM_REQUIRE(aligned16(x) && aligned16(w1) && aligned16(w3) && aligned16(w2) && aligned16(act), DM_ERR_INVALID,
              "operands must be 16-byte aligned");
   hipStream_t s = S(stream);
-  auto up = [&](auto rt) {
-    constexpr int RT = decltype(rt)::value;
-    hipLaunchKernelGGL((k_swiglu_up<bf16, RT>), dim3(H / 16), dim3(256), 0, s, (const bf16*)x, (const bf16*)w1,
-                       (const bf16*)w3, (bf16*)act, M, d, H);
-  };
-  const int rts = (M + 15) / 16;
-  if (rts == 1) up(std::integral_constant<int, 1>{});
-  else if (rts == 2) up(std::integral_constant<int, 2>{});
-  else if (rts == 3) up(std::integral_constant<int, 3>{});
-  else up(std::integral_constant<int, 4>{});
-  launch_rows_wt<bf16>((const bf16*)act, (const bf16*)w2, (bf16*)out, M, d, H, s);
+  launch_wt(WtOp<bf16>{(const bf16*)x, d, M, d}, 2 * H,
+            WtSwiGLU<bf16>{(const bf16*)w1, (const bf16*)w3, d, (bf16*)act, M, H}, s);
+  launch_wt(WtOp<bf16>{(const bf16*)act, H, M, H}, d, WtStore<bf16>{(const bf16*)w2, H, (bf16*)out, M, d}, s);
   DM_HIP(hipGetLastError());
   return DM_OK;
 }

@@ -1,0 +1,127 @@
+"""The few-row forms against the forms they replace, bit for bit: a row's result does not depend on how
+many rows a launch holds (every output sums its k in the same order), so the wave-tile products of few
+rows must equal the same rows inside a larger call, exact cells run row by row must equal whole
+Jacobi sweeps at K = c (which the tape keeps), and a short tape read in one launch must equal the split
+read."""
+
+import pytest
+import torch
+
+from dual_mod_public_amd import _lib as L
+from dual_mod_public_amd.attention import DualModAttention
+from dual_mod_public_amd.engine import HipSweepCell, uniform_chunks
+from dual_mod_public_amd.rope import build_rope_cache
+from dual_mod_public_amd.synthetic import make_state_dict
+from tests.hip_helpers import DEV, cfg_of, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    L.load()
+
+
+def _rand(*shape, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randn(*shape, generator=g, device=DEV).bfloat16()
+
+
+def _sd(cfg):
+    return {k: v.to(DEV, torch.bfloat16) for k, v in make_state_dict(cfg, seed=5).items()}
+
+
+def _same(a, b, what):
+    torch.cuda.synchronize()
+    assert torch.equal(a, b), f"{what}: {(a.float() - b.float()).abs().max().item():.3g} apart"
+
+
+# B rows per step: one and several row tiles; T: whole chunks and a ragged last one
+@pytest.mark.parametrize("B,T", [(1, 64), (2, 70), (9, 65), (17, 96), (33, 20)])
+@pytest.mark.parametrize("mod,d,h,kw", [("mult_res", 256, 4, {}), ("linear", 256, 4, dict(local_window=9)),
+                                        ("fusion", 512, 4, {}), ("mult", 256, 2, dict(v_clamp_tau=0.5))])
+def test_exact_rows_equal_sweeps(B, T, mod, d, h, kw):
+    say(f"exact rows B={B} T={T} {mod} d={d} h={h} {kw}")
+    cfg = cfg_of(d, h, mod, T, **kw)
+    cell = HipSweepCell(cfg, B, T, device=DEV, dtype=torch.bfloat16).pack(_sd(cfg))
+    x = _rand(B, T, d, seed=B + T)
+    cos, sin = (t.to(DEV) for t in build_rope_cache(T, cfg.head_dim, cfg.rope_theta))
+    sched = uniform_chunks(T, 64)
+    out = []
+    for tape in (None, cell.new_tape(sched)):
+        K = torch.full((B, h, T, cfg.head_dim), float("nan"), device=DEV, dtype=torch.bfloat16)
+        V, ocat, y = K.clone(), torch.empty_like(x), torch.empty_like(x)
+        cell.layer_forward(x, y, cos, sin, sched, K, V, ocat, cell.new_bufs(T), tape=tape)
+        out.append((y, K, V, ocat))
+    for a, b, what in zip(*out, ("y", "K", "V", "ocat")):
+        _same(a, b, what)
+
+
+# rows of the small call: edges of the 8-, 16- and 32-row tiles and of the wave-tile range
+@pytest.mark.parametrize("n", [1, 8, 9, 16, 17, 32, 33, 63, 64, 65, 130, 256])
+@pytest.mark.parametrize("mod,d,h", [("mult_res", 256, 4), ("linear", 1024, 16), ("fusion", 512, 4), ("mult", 1024, 8)])
+def test_refine_rows_equal_larger_call(n, mod, d, h):
+    say(f"refine rows n={n} {mod} d={d} h={h}")
+    N = 320
+    cfg = cfg_of(d, h, mod, N)
+    m = DualModAttention(cfg)
+    m.load_state_dict({k: v for k, v in _sd(cfg).items() if k != "attn_norm.weight"})
+    m = m.to(DEV, torch.bfloat16)
+    x, o, k, v = (_rand(1, N, d, seed=s) for s in (1, 2, 3, 4))
+    with torch.no_grad():
+        Ka, Va = m.refine_kv(x, o, k, v)
+        Kb, Vb = m.refine_kv(*(t[:, :n].contiguous() for t in (x, o, k, v)))
+    _same(Ka[:, :n], Kb, "K")
+    _same(Va[:, :n], Vb, "V")
+
+
+@pytest.mark.parametrize("T", [1, 8, 13, 16, 32, 40, 64, 100, 256])
+@pytest.mark.parametrize("d,h", [(256, 4), (1024, 8), (1024, 16)])
+def test_projection_rows_equal_larger_call(T, d, h):
+    say(f"projection rows T={T} d={d} h={h}")
+    N = 512
+    cfg = cfg_of(d, h, "mult_res", N)
+    cell = HipSweepCell(cfg, 1, N, device=DEV, dtype=torch.bfloat16).pack(_sd(cfg))
+    cos, sin = (t.to(DEV) for t in build_rope_cache(N, cfg.head_dim, cfg.rope_theta))
+    x = _rand(1, N, d, seed=7)
+    a = cell.layer_proj(x, cell.new_bufs(N), cos, sin)
+    b = cell.layer_proj(x[:, :T].contiguous(), cell.new_bufs(T), cos, sin)
+    for n in ("xhat", "qr", "kraw", "kself", "vraw", "glogx", "sig"):
+        ta, tb = getattr(a, n), getattr(b, n)
+        _same(ta[:, :, :T] if ta.dim() == 4 else ta[:, :T], tb, n)
+
+
+# splits of 512 keys: one, two and up to four in one launch; 40 batch rows (B*h > 512) take the split grid
+@pytest.mark.parametrize("P", [1, 511, 512, 513, 1024, 1025, 1600, 2048])
+@pytest.mark.parametrize("W", [0, 600])
+@pytest.mark.parametrize("d,h", [(1024, 16), (2048, 16)])
+def test_short_read_equals_split_read(P, W, d, h):
+    say(f"short read P={P} W={W} d={d} h={h}")
+    B, few, dh = 40, 3, d // h
+    m = DualModAttention(cfg_of(d, h, "mult_res", 2048, local_window=W)).to(DEV, torch.bfloat16)
+    q, ks, vs = (_rand(B, h, 1, dh, seed=s) for s in (1, 2, 3))
+    K, V = _rand(B, h, P, dh, seed=4), _rand(B, h, P, dh, seed=5)
+    with torch.no_grad():
+        a = m.attend_one(q, ks, vs, K, V)[0]
+        b = m.attend_one(q[:few], ks[:few], vs[:few], K[:few], V[:few])[0]
+    _same(a[:few], b, "o")
+
+
+# mlp widths whose last k step is a half one (H = 32 mod 64), rows at the tiles' edges
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 33, 64])
+@pytest.mark.parametrize("d,H", [(128, 32), (512, 1376), (1024, 2752)])
+def test_swiglu_rows_half_step(M, d, H):
+    say(f"swiglu rows M={M} d={d} H={H}")
+    x, w1, w3, w2 = (_rand(*s, seed=i) for i, s in enumerate([(M, d), (H, d), (H, d), (d, H)]))
+    w1, w3, w2 = w1 * 0.05, w3 * 0.05, w2 * 0.05
+    out = L.swiglu_rows(x, w1, w3, w2)
+    torch.cuda.synchronize()
+    g, u = x.float() @ w1.float().t(), x.float() @ w3.float().t()
+    act = (torch.nn.functional.silu(g) * u).bfloat16().float()
+    ref = act @ w2.float().t()
+    # act and the output rounded to bf16 (2^-9 each, relative); act may round the other way where the
+    # fp32 sums differ in the last bits: 4 * 2^-9
+    err = ((out.float() - ref).norm() / ref.norm()).item()
+    assert err < 4 * 2 ** -9, err

@@ -4,6 +4,8 @@ rows must equal the same rows inside a larger call, exact cells run row by row m
 Jacobi sweeps at K = c (which the tape keeps), and a short tape read in one launch must equal the split
 read."""
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -12,6 +14,7 @@ from dual_mod_public_amd.attention import DualModAttention
 from dual_mod_public_amd.engine import HipSweepCell, uniform_chunks
 from dual_mod_public_amd.rope import build_rope_cache
 from dual_mod_public_amd.synthetic import make_state_dict
+from dual_mod_public_amd.trunk import MlpBufs, MlpWeights
 from tests.hip_helpers import DEV, cfg_of, say
 
 pytestmark = pytest.mark.gpu
@@ -125,3 +128,40 @@ def test_swiglu_rows_half_step(M, d, H):
     # fp32 sums differ in the last bits: 4 * 2^-9
     err = ((out.float() - ref).norm() / ref.norm()).item()
     assert err < 4 * 2 ** -9, err
+
+
+# weight gradients whose row count is no multiple of the k-tile: whole k-tiles and the last rows by two launches
+@pytest.mark.parametrize("M", [64, 65, 127, 130, 2049])
+def test_weight_grad_last_rows(M):
+    import ctypes
+    say(f"weight gradients over M={M} rows")
+    d, H, dt = 256, 384, torch.bfloat16
+    blk = SimpleNamespace(mlp=SimpleNamespace(**{
+        n: SimpleNamespace(weight=_rand(*s, seed=i) * 0.05)
+        for i, (n, s) in enumerate([("w1", (H, d)), ("w3", (H, d)), ("w2", (d, H))])}),
+        mlp_norm=SimpleNamespace(weight=_rand(d, seed=3)))
+    mw = MlpWeights(d, H, DEV, dt)
+    mw.pack(blk)
+    mb = MlpBufs(1, M, d, H, DEV, dt)
+    y, dz = _rand(M, d, seed=4), _rand(M, d, seed=5)
+    z, dy = torch.empty_like(y), torch.empty_like(y)
+    g = {k: torch.zeros(*s, device=DEV) for k, s in dict(w1=(H, d), w3=(H, d), w2=(d, H), norm_w=(d,)).items()}
+    gs = L.dm_mlp_grads()
+    for k in g:
+        setattr(gs, k, L.ptr(g[k]))
+    code = L.dtype_code(dt)
+    L.check(L.lib().dm_mlp_fwd(code, ctypes.byref(mw.s), L.ptr(y), L.ptr(z), ctypes.byref(mb.s), M, d, H, 1e-5,
+                               L.stream_ptr()))
+    nb = L.lib().dm_mlp_workspace_bytes(code, M, d, H)
+    ws = torch.empty(nb, device=DEV, dtype=torch.uint8)
+    L.check(L.lib().dm_mlp_bwd(code, ctypes.byref(mw.s), L.ptr(y), L.ptr(dz), L.ptr(dy), ctypes.byref(mb.s),
+                               ctypes.byref(gs), M, d, H, 1e-5, L.ptr(ws), nb, L.stream_ptr()))
+    torch.cuda.synchronize()
+    rows = lambda t: t.double().cpu().reshape(M, -1)
+    dab, h = rows(mb.dab), rows(mb.h)
+    w13 = (dab.t() @ h).reshape(-1, 2, 32, d)   # packed: 32 rows of w1, 32 of w3, ...
+    for k, ref in (("w2", rows(dz).t() @ rows(mb.mid)), ("w1", w13[:, 0].reshape(H, d)),
+                   ("w3", w13[:, 1].reshape(H, d))):
+        err = ((g[k].double().cpu() - ref).norm() / ref.norm()).item()
+        # fp32 sums of M exact products: at most M 2^-24 of sum |a b|, which is about sqrt(M) |sum a b|
+        assert err < M ** 1.5 * 2 ** -24, (k, err)

@@ -147,6 +147,8 @@ SIGNATURES = {
     "dm_decode_workspace_bytes": (ctypes.c_size_t, [P(dm_config), c_i32]),
     "dm_decode_step": (ctypes.c_int, [P(dm_config), P(dm_packed), c_fp, c_fp,
                                       P(dm_decode_args), c_vp]),
+    "dm_decode_step_norm": (ctypes.c_int, [P(dm_config), P(dm_packed), c_fp, c_fp, P(dm_decode_args), c_fp, c_fp,
+                                           ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p]),
     "dm_decode_step_noalloc": (ctypes.c_int, [P(dm_config), P(dm_packed), c_fp, c_fp,
                                               P(dm_decode_args), c_vp]),
     "dm_attend_one": (ctypes.c_int, [P(dm_config), c_vp, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_vp, c_vp,

@@ -43,14 +43,25 @@ DM_DEV void dec_geometry(const DecodeArgs<T>& a, int& pos, int& lo, int& nsplit)
   nsplit = pos > lo ? (pos - lo + a.split_len - 1) / a.split_len : 0;
 }
 
-// The unnormalised state of one split's keys [k_begin, k_end) by 256 threads (tid 0 .. 255): A[DH], Z, m
+// Threads per split: 16 passes of whole key rows over a split of 512 keys in bf16. Bound by the read of
+// the tape; at head_dim 128 256 threads held 32 passes = 128 registers of loads, three blocks per CU,
+// and 512 threads read faster (a step of B = 16, h = 16, 3001 keys: 121 us against 99).
+template <typename T, int DH> constexpr int dec_threads() { return sizeof(T) == 2 ? 4 * DH : 256; }
+
+// The unnormalised state of one split's keys [k_begin, k_end) by NT threads (tid 0 .. NT - 1): A[DH], Z, m
 // into out[0 .. DH + 2). red is the group's LDS; block-wide barriers, so every group of a block calls it.
-template <typename T, int DH, int L>
+// EARLY: the V rows are loaded with the K rows (short reads, whose time is their round trips) instead of
+// in K's registers after the scores (long ones, where more blocks per CU hide them). L: the keys whose
+// passes are made, at least the split's (a pass past its keys adds probabilities 0: the same results).
+// No pass is made conditional: with branches between the loads each use would wait for all of them
+// (measured at B*h = 1024, P = 32769: 1360 us against 1302).
+template <typename T, int DH, int L, bool EARLY>
 DM_DEV void decode_split(const DecodeArgs<T>& a, int bh, int k_begin, int k_end, int tid, float (*red)[DH + 2],
                          float* out) {
+  constexpr int NT = dec_threads<T, DH>(), NW = NT / 64;
   constexpr int VEC = 16 / (int)sizeof(T);
   constexpr int LPK = DH / VEC;          // lanes per key row
-  constexpr int KPP = 256 / LPK;         // keys per pass
+  constexpr int KPP = NT / LPK;          // keys per pass
   constexpr int NP = L / KPP;            // passes
   static_assert(L % KPP == 0, "split length");
   const int lane = tid & 63, wave = tid >> 6;
@@ -61,36 +72,42 @@ DM_DEV void decode_split(const DecodeArgs<T>& a, int bh, int k_begin, int k_end,
   const T* Kb = a.Kt + (long)bh * a.tape_T * DH + part * VEC;
   const T* Vb = a.Vt + (long)bh * a.tape_T * DH + part * VEC;
 
-  uint4 raw[NP];
-#pragma unroll
-  for (int i = 0; i < NP; ++i) {
+  uint4 raw[NP], rv[EARLY ? NP : 1];
+  auto load = [&](const T* base, int i) {
     const int key = k_begin + i * KPP + kslot;
-    raw[i] = keep_if(ld_nt(Kb + (long)(key < k_end ? key : k_begin) * DH), key < k_end);
+    return keep_if(ld_nt(base + (long)(key < k_end ? key : k_begin) * DH), key < k_end);
+  };
+#pragma unroll
+  for (int i = 0; i < NP; ++i) raw[i] = load(Kb, i);
+  if constexpr (EARLY) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) rv[i] = load(Vb, i);
   }
   float sc[NP];
   float mx = NEG_INF;
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
+    const bool ok = k_begin + i * KPP + kslot < k_end;
     float kv[VEC];
     unpack16<T>(raw[i], kv);
     float dot = 0.f;
 #pragma unroll
     for (int j = 0; j < VEC; ++j) dot += qv[j] * kv[j];
     dot = lanes_sum<1, LPK / 2>(dot);
-    const int key = k_begin + i * KPP + kslot;
-    sc[i] = (key < k_end) ? dot * a.scale : NEG_INF;
+    sc[i] = ok ? dot * a.scale : NEG_INF;
     mx = fmaxf(mx, sc[i]);
   }
+  if constexpr (!EARLY) {
 #pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int key = k_begin + i * KPP + kslot;
-    raw[i] = keep_if(ld_nt(Vb + (long)(key < k_end ? key : k_begin) * DH), key < k_end);
+    for (int i = 0; i < NP; ++i) raw[i] = load(Vb, i);
   }
   // group max
   mx = lanes_max<LPK, 32>(mx);
   if (lane == 0) red[wave][0] = mx;
   __syncthreads();
-  const float M = fmaxf(fmaxf(red[0][0], red[1][0]), fmaxf(red[2][0], red[3][0]));
+  float M = red[0][0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) M = fmaxf(M, red[w][0]);
   __syncthreads();
   float acc[VEC];
 #pragma unroll
@@ -101,7 +118,7 @@ DM_DEV void decode_split(const DecodeArgs<T>& a, int bh, int k_begin, int k_end,
     const float p = (sc[i] == NEG_INF) ? 0.f : __expf(sc[i] - M);
     z += p;
     float vv[VEC];
-    unpack16<T>(raw[i], vv);
+    unpack16<T>(EARLY ? rv[EARLY ? i : 0] : raw[i], vv);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) acc[j] += p * vv[j];
   }
@@ -117,20 +134,25 @@ DM_DEV void decode_split(const DecodeArgs<T>& a, int bh, int k_begin, int k_end,
   }
   if (lane == 0) red[wave][DH] = zz;
   __syncthreads();
-  for (int i = tid; i < DH + 1; i += 256) out[i] = red[0][i] + red[1][i] + red[2][i] + red[3][i];
+  for (int i = tid; i < DH + 1; i += NT) {
+    float v = red[0][i];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += red[w][i];
+    out[i] = v;
+  }
   if (tid == 0) out[DH + 1] = M;
 }
 
 template <typename T, int DH, int L>
-__global__ __launch_bounds__(256) void k_decode_partial(DecodeArgs<T> a) {
+__global__ __launch_bounds__((dec_threads<T, DH>())) void k_decode_partial(DecodeArgs<T> a) {
   const uint64_t t0 = prof_begin(a.prof_ts);
-  __shared__ float red[4][DH + 2];
+  __shared__ float red[dec_threads<T, DH>() / 64][DH + 2];
   const int s = blockIdx.x, bh = blockIdx.y;
   int pos, lo, nsplit;
   dec_geometry(a, pos, lo, nsplit);
   if (s >= nsplit) return;   // whole block: past the position (device-position grids only)
   const int k_begin = lo + s * a.split_len;
-  decode_split<T, DH, L>(a, bh, k_begin, min(k_begin + a.split_len, pos), threadIdx.x, red,
+  decode_split<T, DH, L, false>(a, bh, k_begin, min(k_begin + a.split_len, pos), threadIdx.x, red,
                          a.part + ((long)s * (a.B * a.h) + bh) * (DH + 2));
   prof_end(a.prof_ts, t0);
 }
@@ -196,16 +218,17 @@ __global__ __launch_bounds__(64) void k_decode_merge(DecodeArgs<T> a) {
   decode_merge<T, DH>(a, sf, a.part + (long)bh * (DH + 2), (long)(a.B * a.h) * (DH + 2), nsplit, bh, lane);
 }
 
-// The whole read of a short tape in one launch: block = one (b, h), NS groups of 256 threads each one
+// The whole read of a short tape in one launch: block = one (b, h), NS groups of threads each one
 // split of L keys (the split kernel's arithmetic), their states in LDS, merged by the first wave (the
 // merge kernel's arithmetic: the same results as the two launches). A launch and a round trip of the
 // partials less; the grid is B*h blocks whatever the tape's length, so it pays while NS groups cover
 // the read and B*h blocks of them are resident together (decode_reads_direct).
 template <typename T, int DH, int L, int NS>
-__global__ __launch_bounds__(256 * NS) void k_decode_direct(DecodeArgs<T> a) {
-  __shared__ float red[NS][4][DH + 2];
+__global__ __launch_bounds__((dec_threads<T, DH>() * NS)) void k_decode_direct(DecodeArgs<T> a) {
+  constexpr int NT = dec_threads<T, DH>();
+  __shared__ float red[NS][NT / 64][DH + 2];
   __shared__ float part[NS][DH + 2];
-  const int bh = blockIdx.x, grp = threadIdx.x >> 8, tid = threadIdx.x & 255;
+  const int bh = blockIdx.x, grp = threadIdx.x / NT, tid = threadIdx.x % NT;
   int pos, lo, nsplit;
   dec_geometry(a, pos, lo, nsplit);
   DecodeSelf<DH> sf{};
@@ -213,13 +236,18 @@ __global__ __launch_bounds__(256 * NS) void k_decode_direct(DecodeArgs<T> a) {
   // a group past the position reads no key (k_end = k_begin, clamped into the tape) and its state is not merged
   const int kb = min(lo + grp * L, max(pos - 1, 0));
   const int ke = grp < nsplit ? min(lo + (grp + 1) * L, pos) : kb;
-  decode_split<T, DH, L>(a, bh, kb, ke, tid, red[grp], part[grp]);
+  // EARLY in blocks of 256 threads only: with 512 (two splits, 777 keys) a step took 24.0 us against 23.4.
+  // The first split's keys bound every group's passes (uniform over the block): up to a quarter of a
+  // split makes a quarter of the passes.
+  constexpr bool EARLY = NT * NS <= 256;
+  if (pos - lo <= L / 4) decode_split<T, DH, L / 4, EARLY>(a, bh, kb, ke, tid, red[grp], part[grp]);
+  else decode_split<T, DH, L, EARLY>(a, bh, kb, ke, tid, red[grp], part[grp]);
   __syncthreads();
   if (threadIdx.x < 64) decode_merge<T, DH>(a, sf, &part[0][0], DH + 2, min(nsplit, NS), bh, threadIdx.x);
 }
 
 // device position: the RoPE rows of position *pos_dev -> rope[0, half) cos, rope[half, 2 half) sin
-__global__ __launch_bounds__(64) void k_decode_pos_rope(const int* pos_dev, int tape_T, const float* cos,
+static __global__ __launch_bounds__(64) void k_decode_pos_rope(const int* pos_dev, int tape_T, const float* cos,
                                                         const float* sin, int half, float* rope) {
   const int pos = clamp_pos(*pos_dev, tape_T);
   for (int i = threadIdx.x; i < half; i += 64) {
@@ -307,24 +335,24 @@ __global__ __launch_bounds__(256) void k_argmax_rows(const T* x, long ld, int co
 
 // k_residual_rmsnorm with the row held in registers (d <= 256 NPT): every load (x, delta, w) is
 // issued before the reduction and nothing is re-read; the same per-element arithmetic and the same
-// order of the sums, so the same results.
+// order of the sums, so the same results. Row `row` by a 256-thread block.
 template <typename T, int NPT>
-__global__ __launch_bounds__(256) void k_residual_rmsnorm_reg(float* x, const T* delta, const float* w, T* y, int d,
-                                                             float eps) {
-  __shared__ float red[4];
-  float* xr = x + (long)blockIdx.x * d;
+DM_DEV void residual_rmsnorm_row(int row, float* x, const T* delta, const float* w, T* y, int d, float eps, float* red) {
+  float* xr = x + (long)row * d;
   float v[NPT], wv[NPT];
 #pragma unroll
   for (int i = 0; i < NPT; ++i) {
+    if (256 * i >= d) break;   // uniform
     const int j = threadIdx.x + 256 * i;
     const int jc = j < d ? j : 0;
     v[i] = xr[jc];
-    if (delta != nullptr) v[i] += to_f(delta[(long)blockIdx.x * d + jc]);
+    if (delta != nullptr) v[i] += to_f(delta[(long)row * d + jc]);
     wv[i] = w != nullptr ? w[jc] : 0.f;
   }
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < NPT; ++i) {
+    if (256 * i >= d) break;
     const int j = threadIdx.x + 256 * i;
     if (j < d) {
       if (delta != nullptr) xr[j] = v[i];
@@ -336,12 +364,19 @@ __global__ __launch_bounds__(256) void k_residual_rmsnorm_reg(float* x, const T*
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   const float rs = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)d + eps);
-  T* yr = y + (long)blockIdx.x * d;
+  T* yr = y + (long)row * d;
 #pragma unroll
   for (int i = 0; i < NPT; ++i) {
+    if (256 * i >= d) break;
     const int j = threadIdx.x + 256 * i;
     if (j < d) yr[j] = from_f<T>(v[i] * rs * wv[i]);
   }
+}
+template <typename T, int NPT>
+__global__ __launch_bounds__(256) void k_residual_rmsnorm_reg(float* x, const T* delta, const float* w, T* y, int d,
+                                                             float eps) {
+  __shared__ float red[4];
+  residual_rmsnorm_row<T, NPT>(blockIdx.x, x, delta, w, y, d, eps, red);
 }
 
 // k_argmax_rows for 16-byte aligned rows (ld a multiple of the vector width): 1024 threads per row,

@@ -6,6 +6,7 @@
 
 #include <vector>
 
+#include "dm_decode.h"
 #include "dm_host.h"
 #include "dm_rows.h"
 
@@ -158,6 +159,23 @@ void launch_wt(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls = PROF
     launch_k(prof_cls, k_wt<T, WT, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64), 0, s, op, e);
   });
 }
+// a product with a long K whose tiles would leave half of the CUs idle: K over four waves per tile
+template <typename T, class E>
+void launch_wt_long(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls = PROF_NONE) {
+  constexpr int KW = 4;
+  if (op.K < 1536 || (long)cdiv(op.M, 32) * (N / 16) > 128) {
+    launch_wt(op, N, e, s, prof_cls);
+    return;
+  }
+  auto run = [&](auto wt) {
+    using WT = decltype(wt);
+    op.nx = N / WT::COLS;
+    launch_k(prof_cls, k_wt_ksplit<T, WT, KW, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64 * KW), 0, s, op, e);
+  };
+  if (op.M <= 8) run(WTile<1, 1>{});
+  else if (op.M <= 16) run(WTile<2, 1>{});
+  else run(WTile<4, 1, 6>{});
+}
 template <typename T, class E1, class E2>
 void launch_wt2(WtOp<T> op1, int N1, const E1& e1, WtOp<T> op2, int N2, const E2& e2, hipStream_t s,
                 int prof_cls = PROF_NONE) {
@@ -169,11 +187,28 @@ void launch_wt2(WtOp<T> op1, int N1, const E1& e1, WtOp<T> op2, int N2, const E2
              e2);
   });
 }
-// a decode step's W_O product riding in its refine's first launch (both read o_cat)
+// What rides in a decode step's refine: the W_O product in its first launch (both read o_cat), and the
+// residual add and norm after it (x += y, h = rmsnorm(x) norm_w) in its second, which they do not depend on
 template <typename T> struct WtWo {
   const T* W;
   T* y;
+  float* x = nullptr;
+  const float* norm_w = nullptr;
+  T* h = nullptr;
+  float eps = 0.f;
 };
+// blocks [0, M): one row of the residual norm each; then four column tiles of GEMM 2 per block
+template <typename T, class WT, class E>
+static __global__ __launch_bounds__(256) void k_norm_wt(WtWo<T> n, int M, int d, WtOp<T> op, E e) {
+  __shared__ __attribute__((aligned(1024))) char smem[4 * WT::LDS];
+  const int b = blockIdx.x;
+  if (b < M) {
+    residual_rmsnorm_row<T, 16>(b, n.x, n.y, n.norm_w, n.h, d, n.eps, reinterpret_cast<float*>(smem));
+    return;
+  }
+  const int t = 4 * (b - M) + (threadIdx.x >> 6);   // the grid holds whole fours of tiles
+  wt_tile<T, WT>(e, op, t % op.nx, t / op.nx, smem + (threadIdx.x >> 6) * WT::LDS);
+}
 
 // vpre: v_raw before the v_norm (nullptr: not kept); sa: the M input rows (x-hat);
 // small_tiles: 128 x 128 blocks even where 256 x 256 ones fit (more blocks for a short M; the
@@ -291,8 +326,22 @@ void run_refine_wt(const dm_config* c, const dm_packed* w, const CellGeom& g, in
     launch_wt2(op1, 4 * d, e1, op1, d, WtStore<T>{wo->W, d, wo->y, N, d}, s, PROF_SWEEP1);
   else
     launch_wt(op1, 4 * d, e1, s, PROF_SWEEP1);
-  if (c->ctx_mod != DM_CTX_LINEAR)
+  if (c->ctx_mod == DM_CTX_LINEAR) return;
+  if (wo == nullptr || wo->x == nullptr) {
     launch_gemm2_wt<T, DH, DEVPOS>(c, w, g, N, vraw, glogx, Vout, out_stride, out_row0, vin, gvu, save2, s);
+    return;
+  }
+  const WtSweep2<T, DH, DEVPOS> e2{(const T*)w->w_vctx, EpiSweep2<T, DH, DEVPOS>{g, N, vraw, glogx, gvu, Vout, out_stride,
+                                                                                out_row0, save2}};
+  auto run = [&](auto wt) {
+    using WT = decltype(wt);
+    const WtOp<T> op2{vin, d, N, d, d / WT::COLS};   // d a multiple of 128: whole fours of tiles per row tile
+    launch_k(PROF_SWEEP2, k_norm_wt<T, WT, WtSweep2<T, DH, DEVPOS>>, dim3(N + op2.nx * cdiv(N, WT::ROWS) / 4), dim3(256),
+             0, s, *wo, N, d, op2, e2);
+  };
+  if (N <= 8) run(WTile<1, 1>{});
+  else if (N <= 16) run(WTile<2, 1>{});
+  else run(WTile<4, 1, 6>{});
 }
 
 // The wave-tile forms apply: no per-head norm.

@@ -351,23 +351,35 @@ void run_decode_read(DecodeArgs<T>& da, hipStream_t s) {
   // One launch while a (b, h)'s splits fit one block and the chip still holds the grid: with more
   // than one split per (b, h) each block keeps 256 threads per split resident until the slowest is
   // done, so from 512 (b, h) up the split grid balances better.
-  if (da.nsplit >= 1 && (da.nsplit == 1 || (da.nsplit <= 4 && BH <= 512))) {
-    if (da.nsplit == 1) launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 1>, dim3(BH), dim3(256), 0, s, da);
-    else if (da.nsplit == 2) launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 2>, dim3(BH), dim3(512), 0, s, da);
-    else launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 4>, dim3(BH), dim3(1024), 0, s, da);
+  constexpr int NT = dec_threads<T, DH>(), NSMAX = 1024 / NT;
+  if (da.nsplit >= 1 && (da.nsplit == 1 || (da.nsplit <= NSMAX && BH <= 512))) {
+    if (da.nsplit == 1)
+      launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 1>, dim3(BH), dim3(NT), 0, s, da);
+    else if (da.nsplit == 2)
+      launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 2>, dim3(BH), dim3(2 * NT), 0, s, da);
+    else
+      launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, NSMAX>, dim3(BH), dim3(NSMAX * NT), 0, s, da);
     return;
   }
   if (da.nsplit > 0) {
     const int idx = prof_launch_begin(PROF_DEC_READ, true, da.prof_ts);
-    launch_timed(idx, k_decode_partial<T, DH, DEC_SPLIT>, dim3(da.nsplit, BH), dim3(256), 0, s, da);
+    launch_timed(idx, k_decode_partial<T, DH, DEC_SPLIT>, dim3(da.nsplit, BH), dim3(NT), 0, s, da);
     da.prof_ts = nullptr;
   }
   launch_k(PROF_DEC_MERGE, k_decode_merge<T, DH>, dim3(BH), dim3(64), 0, s, da);
 }
 
+// the residual norm after a step (dm_decode_step_norm); x nullptr: none
+struct StepNorm {
+  float* x = nullptr;
+  const float* w = nullptr;
+  void* h = nullptr;
+  float eps = 0.f;
+};
+
 template <typename T, int DH>
 int run_decode(const dm_config* c, const dm_packed* w, const float* cos, const float* sin,
-               const dm_decode_args* a, const DecWs& ws, hipStream_t s) {
+               const dm_decode_args* a, const DecWs& ws, hipStream_t s, const StepNorm& nrm) {
   const int B = c->B, d = c->d, h = c->h;
   // device position (a->pos_dev): one launch shape for every position — the RoPE rows are
   // gathered first, the split grid covers the whole tape, the refined pair is staged and
@@ -411,6 +423,14 @@ int run_decode(const dm_config* c, const dm_packed* w, const float* cos, const f
   const bool wo_rides = a->y != nullptr && aligned16(w->wo) &&
                         refine_few_rows<T>(c, w, B, (const T*)a->o_cat, (const T*)ws.vin);
   const WtWo<T>* wop = wo_rides ? &wo : nullptr;
+  // the norm rides where the refine has a second launch that nothing of this step reads
+  const bool norm_rides = nrm.x != nullptr && wo_rides && c->ctx_mod != DM_CTX_LINEAR && d <= 4096;
+  if (norm_rides) {
+    wo.x = nrm.x;
+    wo.norm_w = nrm.w;
+    wo.h = (T*)nrm.h;
+    wo.eps = nrm.eps;
+  }
   if (dev_direct) {
     g.pos_dev = (const int*)a->pos_dev;
     g.pos_cap = a->tape_T;
@@ -446,6 +466,8 @@ int run_decode(const dm_config* c, const dm_packed* w, const float* cos, const f
       else launch_gemm_auto<T, 64, 128, 2, 2, 3, 4>(ao, bo, B, d, d, ep, s);
     }
   }
+  if (nrm.x != nullptr && !norm_rides)
+    return dm_residual_rmsnorm(c->dtype, nrm.x, a->y, nrm.w, nrm.h, B, d, nrm.eps, s);
   return DM_OK;
 }
 
@@ -460,8 +482,8 @@ size_t dm_decode_workspace_bytes(const dm_config* c, int32_t tape_T) {
   return carve_dec(c, tape_T, nullptr).bytes;
 }
 
-int dm_decode_step(const dm_config* c, const dm_packed* w, const float* cos, const float* sin,
-                   const dm_decode_args* a, void* stream) {
+static int decode_step(const dm_config* c, const dm_packed* w, const float* cos, const float* sin,
+                       const dm_decode_args* a, void* stream, const StepNorm& nrm) {
   int rc = check_cfg(c);
   if (rc) return rc;
   if ((rc = check_packed(c, w))) return rc;
@@ -480,12 +502,23 @@ int dm_decode_step(const dm_config* c, const dm_packed* w, const float* cos, con
   hipStream_t s = S(stream);
   ProfScope whole(PROF_LAYER, s);
   if (c->dtype == DM_BF16)
-    rc = c->dh == 64 ? run_decode<bf16, 64>(c, w, cos, sin, a, ws, s) : run_decode<bf16, 128>(c, w, cos, sin, a, ws, s);
+    rc = c->dh == 64 ? run_decode<bf16, 64>(c, w, cos, sin, a, ws, s, nrm) : run_decode<bf16, 128>(c, w, cos, sin, a, ws, s, nrm);
   else
-    rc = c->dh == 64 ? run_decode<float, 64>(c, w, cos, sin, a, ws, s) : run_decode<float, 128>(c, w, cos, sin, a, ws, s);
+    rc = c->dh == 64 ? run_decode<float, 64>(c, w, cos, sin, a, ws, s, nrm) : run_decode<float, 128>(c, w, cos, sin, a, ws, s, nrm);
   if (rc) return rc;
   DM_HIP(hipGetLastError());
   return DM_OK;
+}
+
+int dm_decode_step(const dm_config* c, const dm_packed* w, const float* cos, const float* sin,
+                   const dm_decode_args* a, void* stream) {
+  return decode_step(c, w, cos, sin, a, stream, StepNorm{});
+}
+
+int dm_decode_step_norm(const dm_config* c, const dm_packed* w, const float* cos, const float* sin,
+                        const dm_decode_args* a, float* x, const float* norm_w, void* h, float eps, void* stream) {
+  DM_REQUIRE(a != nullptr && a->y && x && norm_w && h, DM_ERR_INVALID, "null operand");
+  return decode_step(c, w, cos, sin, a, stream, StepNorm{x, norm_w, h, eps});
 }
 
 }  // extern "C"
@@ -700,7 +733,7 @@ int dm_swiglu_rows(int32_t dtype, const void* x, const void* w1, const void* w3,
   hipStream_t s = S(stream);
   launch_wt(WtOp<bf16>{(const bf16*)x, d, M, d}, 2 * H,
             WtSwiGLU<bf16>{(const bf16*)w1, (const bf16*)w3, d, (bf16*)act, M, H}, s);
-  launch_wt(WtOp<bf16>{(const bf16*)act, H, M, H}, d, WtStore<bf16>{(const bf16*)w2, H, (bf16*)out, M, d}, s);
+  launch_wt_long(WtOp<bf16>{(const bf16*)act, H, M, H}, d, WtStore<bf16>{(const bf16*)w2, H, (bf16*)out, M, d}, s);
   DM_HIP(hipGetLastError());
   return DM_OK;
 }

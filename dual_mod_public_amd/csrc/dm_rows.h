@@ -31,12 +31,12 @@ namespace dm {
 constexpr int WT_MAX_M = 256;
 constexpr int ROWS_MAX = 64;   // rows of a decode-style call (dm_swiglu_rows)
 
-template <int NA_, int CT_> struct WTile {
+template <int NA_, int CT_, int S_ = 0> struct WTile {
   static constexpr int NA = NA_, CT = CT_;              // 8-row groups of A, 16-column tiles of W
   static constexpr int RT = (NA + 1) / 2;               // 16-row MFMA tiles
   static constexpr int ROWS = 8 * NA, COLS = 16 * CT;
   static constexpr int L = 2 * CT + NA;                 // load instructions per stage
-  static constexpr int S = L <= 4 ? 8 : (L <= 6 ? 10 : (L <= 8 ? 7 : 5));   // stages (measured)
+  static constexpr int S = S_ > 0 ? S_ : (L <= 4 ? 8 : (L <= 6 ? 10 : (L <= 8 ? 7 : 5)));   // stages (measured)
   static constexpr int STAGE = (16 * CT + 8 * NA) * 128;
   static constexpr int LDT = COLS + 4;                  // floats per row of the staged output tile
   static constexpr int LDS = S * STAGE;
@@ -54,9 +54,11 @@ template <typename T> struct WtOp {   // the A operand: row m at A + m lda; K a 
   int M, K, nx;   // nx column tiles
 };
 
-// One tile (column tile bx, row tile by) by one wave.
+// The accumulators of one tile (column tile bx, row tile by) by one wave, over its 64-wide k steps
+// [kt0, kt0 + nk); leaves the stages free.
 template <typename T, class WT, class E>
-DM_DEV void wt_tile(const E& e, const WtOp<T>& op, int bx, int by, char* smem) {
+DM_DEV void wt_kloop(const E& e, const WtOp<T>& op, int bx, int by, int kt0, int nk, char* smem,
+                     floatx4 (&acc)[WT::RT][WT::CT]) {
   using MF = Mfma<T>;
   constexpr int NA = WT::NA, CT = WT::CT, RT = WT::RT, S = WT::S, L = WT::L;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -68,12 +70,9 @@ DM_DEV void wt_tile(const E& e, const WtOp<T>& op, int bx, int by, char* smem) {
   for (int i = 0; i < 2 * CT; ++i) pw[i] = e.wrow(bx, WT{}, 8 * i + lr);
 #pragma unroll
   for (int i = 0; i < NA; ++i) pa[i] = op.A + (long)min(m0 + 8 * i + lr, op.M - 1) * op.lda;   // past M: row M - 1 again
-  typename E::template Pre<WT> pre;
-  e.prefetch(bx, m0, pre);
-  const int nk = (K + 63) / 64;
   auto issue = [&](int kt, int st) {
     char* b = smem + st * WT::STAGE;
-    const int k = min(64 * kt + 8 * lc, K - 8);   // a half last step: chunks past K read K's last, unused
+    const int k = min(64 * (kt0 + kt) + 8 * lc, K - 8);   // a half last step: chunks past K read K's last, unused
 #pragma unroll
     for (int i = 0; i < 2 * CT; ++i)
       __builtin_amdgcn_global_load_lds((const void*)(pw[i] + k), (lds_void_t*)(b + i * 1024), 16, 0, 0);
@@ -81,7 +80,6 @@ DM_DEV void wt_tile(const E& e, const WtOp<T>& op, int bx, int by, char* smem) {
     for (int i = 0; i < NA; ++i)
       __builtin_amdgcn_global_load_lds((const void*)(pa[i] + k), (lds_void_t*)(b + (2 * CT + i) * 1024), 16, 0, 0);
   };
-  floatx4 acc[RT][CT];
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
@@ -90,7 +88,7 @@ DM_DEV void wt_tile(const E& e, const WtOp<T>& op, int bx, int by, char* smem) {
     const char* b = smem + st * WT::STAGE;
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
-      if (64 * kt + 32 * hf >= K) break;   // uniform
+      if (64 * (kt0 + kt) + 32 * hf >= K) break;   // uniform
       const int sw = ((4 * hf + g) ^ (r & 7)) << 4;
       typename MF::frag w[CT];
 #pragma unroll
@@ -123,15 +121,30 @@ DM_DEV void wt_tile(const E& e, const WtOp<T>& op, int bx, int by, char* smem) {
     }
   });
   // every load has landed and one wave's LDS operations complete in order: the stages are free
-  float* tile = reinterpret_cast<float*>(smem);
+}
+
+// the accumulators staged as the output tile
+template <class WT> DM_DEV void wt_stage(const floatx4 (&acc)[WT::RT][WT::CT], float* tile) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
+  for (int t = 0; t < WT::RT; ++t)
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int c = 0; c < WT::CT; ++c)
 #pragma unroll
       for (int q = 0; q < 4; ++q) tile[(16 * t + 4 * g + q) * WT::LDT + 16 * c + r] = acc[t][c][q];
-  __syncthreads();   // the block is this one wave
-  e.apply(bx, m0, tile, pre);
+}
+
+// one tile by one wave: a block's waves each call it with LDS of their own
+template <typename T, class WT, class E>
+DM_DEV void wt_tile(const E& e, const WtOp<T>& op, int bx, int by, char* smem) {
+  typename E::template Pre<WT> pre;
+  e.prefetch(bx, by * WT::ROWS, pre);
+  floatx4 acc[WT::RT][WT::CT];
+  wt_kloop<T, WT>(e, op, bx, by, 0, (op.K + 63) / 64, smem, acc);
+  float* tile = reinterpret_cast<float*>(smem);
+  wt_stage<WT>(acc, tile);
+  __syncthreads();
+  e.apply(bx, by * WT::ROWS, tile, pre);
 }
 
 template <typename T, class WT, class E>
@@ -146,6 +159,34 @@ static __global__ __launch_bounds__(64) void k_wt2(WtOp<T> op1, E1 e1, WtOp<T> o
   const int b = blockIdx.x;
   if (b < op1.nx) wt_tile<T, WT>(e1, op1, b, blockIdx.y, smem);
   else wt_tile<T, WT>(e2, op2, b - op1.nx, blockIdx.y, smem);
+}
+
+// A long K in few tiles (an MLP's down product): KW waves per tile, each a quarter of the k steps with its
+// own ring, their partial tiles added in wave order. One wave alone keeps 24 KB in flight; 64 tiles
+// on 64 CUs then read K = 2752 at 34 KB/us each.
+template <typename T, class WT, int KW, class E>
+static __global__ __launch_bounds__(64 * KW) void k_wt_ksplit(WtOp<T> op, E e) {
+  __shared__ __attribute__((aligned(1024))) char smem[KW * WT::LDS];
+  const int wave = threadIdx.x >> 6, nk = (op.K + 63) / 64;
+  const int k0 = wave * nk / KW, k1 = (wave + 1) * nk / KW;
+  typename E::template Pre<WT> pre;
+  e.prefetch(blockIdx.x, blockIdx.y * WT::ROWS, pre);
+  floatx4 acc[WT::RT][WT::CT];
+  char* mine = smem + wave * WT::LDS;
+  wt_kloop<T, WT>(e, op, blockIdx.x, blockIdx.y, k0, k1 - k0, mine, acc);
+  wt_stage<WT>(acc, reinterpret_cast<float*>(mine));
+  __syncthreads();
+  if (wave > 0) return;
+  float* tile = reinterpret_cast<float*>(smem);
+  constexpr int NE = WT::ROWS * WT::LDT;
+  for (int i = threadIdx.x; i < NE; i += 64) {
+    float v = tile[i];
+#pragma unroll
+    for (int w = 1; w < KW; ++w) v += reinterpret_cast<const float*>(smem + w * WT::LDS)[i];
+    tile[i] = v;
+  }
+  __builtin_amdgcn_wave_barrier();   // one wave's LDS operations complete in order
+  e.apply(blockIdx.x, blockIdx.y * WT::ROWS, tile, pre);
 }
 
 // ---- epilogues ----------------------------------------------------------------------------------

@@ -60,6 +60,21 @@ class StaticTape:
         pos: the absolute position (int), or a one-element int32 tensor on the device that
         the kernels read at run time (lm/eval/graph_decode.py:24: one captured graph serves
         every position); the caller keeps it inside [0, P_max)."""
+        self._run(xhat, pos, cos, sin, with_wo, None)
+        return self.o_cat, (self.y if with_wo else None)
+
+    def step_norm(self, xhat, pos, cos, sin, x, norm_w, h, eps):
+        """``step`` with W_O, then the residual add and the RMSNorm after it (L.residual_rmsnorm) in the
+        same call: x [B, d] fp32 += y, h = rmsnorm(x) * norm_w (fp32 [d]) in the storage dtype; the
+        results of the two calls."""
+        assert not self.noalloc
+        assert x.dtype == torch.float32 and x.is_contiguous() and x.numel() == self.B * self.cfg.d_model
+        assert norm_w.dtype == torch.float32 and norm_w.is_contiguous() and norm_w.numel() == self.cfg.d_model
+        assert h.dtype == self.dtype and h.is_contiguous() and h.numel() == x.numel()
+        self._run(xhat, pos, cos, sin, True, (x, norm_w, h, eps))
+        return h
+
+    def _run(self, xhat, pos, cos, sin, with_wo, norm):
         self._refresh()
         xhat = xhat.contiguous()
         assert xhat.dtype == self.dtype and xhat.shape == (self.B, self.cfg.d_model)
@@ -86,6 +101,10 @@ class StaticTape:
                                                    L.ptr(sin), ctypes.byref(a), L.stream_ptr()))
         else:
             a.workspace, a.workspace_bytes = L.ptr(self.workspace), self.workspace.numel()
-            L.check(L.lib().dm_decode_step(ctypes.byref(self.conf), ctypes.byref(ws), L.ptr(cos),
-                                           L.ptr(sin), ctypes.byref(a), L.stream_ptr()))
-        return self.o_cat, (self.y if with_wo else None)
+            args = (ctypes.byref(self.conf), ctypes.byref(ws), L.ptr(cos), L.ptr(sin), ctypes.byref(a))
+            if norm is None:
+                L.check(L.lib().dm_decode_step(*args, L.stream_ptr()))
+            else:
+                x, norm_w, h, eps = norm
+                L.check(L.lib().dm_decode_step_norm(*args, L.ptr(x), L.ptr(norm_w), L.ptr(h), float(eps),
+                                                    L.stream_ptr()))

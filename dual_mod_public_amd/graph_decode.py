@@ -76,8 +76,9 @@ class GraphDecoder:
         blocks = list(m.blocks)
         h = L.residual_rmsnorm(x, None, blocks[0].attn_norm.weight, dt, eps=blocks[0].attn_norm.eps)
         for l, (blk, tape, (w1, w3, w2)) in enumerate(zip(blocks, self.tapes, self._mlp)):
-            _, y = tape.step(h.view(B, d), self.pos, self.cos, self.sin, with_wo=True)
-            h = L.residual_rmsnorm(x, y, blk.mlp_norm.weight, dt, eps=blk.mlp_norm.eps)
+            # the attention step, its residual add and the mlp_norm
+            h = tape.step_norm(h.view(B, d), self.pos, self.cos, self.sin, x, blk.mlp_norm.weight,
+                               torch.empty(B, 1, d, device=self.dev, dtype=dt), blk.mlp_norm.eps)
             mo = blk.mlp.decode(h, (w1, w3, w2), act=self._act, out=self._mo)
             # the MLP's residual add fused with the next norm (the next block's attn_norm, or norm_f)
             nrm = blocks[l + 1].attn_norm if l + 1 < len(blocks) else m.norm_f

@@ -424,6 +424,13 @@ size_t dm_decode_workspace_bytes(const dm_config* cfg, int32_t tape_T);
 int dm_decode_step(const dm_config* cfg, const dm_packed* w, const float* cos, const float* sin,
                    const dm_decode_args* a, void* stream);
 
+/* dm_decode_step (a->y given) followed by dm_residual_rmsnorm(x += y, h = rmsnorm(x) * norm_w): the same
+ * results as the two calls. Where the step's last product (the value half of the refine, which only
+ * the next token reads) and the norm are small, they run side by side in one launch. x [B, d] fp32 in
+ * place, norm_w [d] fp32, h [B, d] in the storage dtype. */
+int dm_decode_step_norm(const dm_config* cfg, const dm_packed* w, const float* cos, const float* sin,
+                        const dm_decode_args* a, float* x, const float* norm_w, void* h, float eps, void* stream);
+
 /* ---- decode step that allocates nothing ------------------------------------------
  * No counterpart in the reference. For callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid it):

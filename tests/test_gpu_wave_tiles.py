@@ -11,6 +11,7 @@ import torch
 
 from dual_mod_public_amd import _lib as L
 from dual_mod_public_amd.attention import DualModAttention
+from dual_mod_public_amd.decode import StaticTape
 from dual_mod_public_amd.engine import HipSweepCell, uniform_chunks
 from dual_mod_public_amd.rope import build_rope_cache
 from dual_mod_public_amd.synthetic import make_state_dict
@@ -128,6 +129,36 @@ def test_swiglu_rows_half_step(M, d, H):
     # fp32 sums differ in the last bits: 4 * 2^-9
     err = ((out.float() - ref).norm() / ref.norm()).item()
     assert err < 4 * 2 ** -9, err
+
+
+# dm_decode_step_norm against dm_decode_step and dm_residual_rmsnorm: the norm in GEMM 2's launch (bf16,
+# B <= 64, no per-head norm), and where it follows the step (linear: one refine GEMM; B = 65; v_norm; fp32)
+@pytest.mark.parametrize("dt,B,d,h,P0,kw", [
+    (torch.bfloat16, 1, 256, 4, 0, {}), (torch.bfloat16, 9, 1024, 16, 700, dict(ctx_mod="mult")),
+    (torch.bfloat16, 64, 512, 4, 520, dict(ctx_mod="fusion")), (torch.bfloat16, 3, 256, 4, 30, dict(ctx_mod="linear")),
+    (torch.bfloat16, 65, 256, 4, 30, {}), (torch.bfloat16, 3, 256, 4, 30, dict(v_norm="rms")),
+    (torch.float32, 5, 256, 4, 30, {})])
+def test_step_norm_equals_two_calls(dt, B, d, h, P0, kw):
+    say(f"decode step + norm in one call, {dt} B={B} d={d} P0={P0} {kw}")
+    cfg = cfg_of(d=d, h=h, T=P0 + 4, **kw)
+    dh = cfg.head_dim
+    sd = {k: v.to(DEV, dt) for k, v in make_state_dict(cfg, seed=5).items()}
+    cos, sin = (t.to(DEV) for t in build_rope_cache(P0 + 4, dh, 10000.0))
+    tapes = [StaticTape(cfg, B, P0 + 4, DEV, dt, sd=sd) for _ in range(2)]
+    for t in tapes:
+        t.K.copy_(_rand(B, h, P0 + 4, dh, seed=1))
+        t.V.copy_(_rand(B, h, P0 + 4, dh, seed=2))
+    w = _rand(d, seed=3).float()
+    xs = [_rand(B, d, seed=4).float() for _ in range(2)]
+    for p in range(P0, P0 + 3):
+        xh = _rand(B, d, seed=10 + p).to(dt)
+        _, y = tapes[0].step(xh, p, cos, sin, with_wo=True)
+        h0 = L.residual_rmsnorm(xs[0], y, w, dt)
+        h1 = tapes[1].step_norm(xh, p, cos, sin, xs[1], w, torch.empty(B, d, device=DEV, dtype=dt), 1e-5)
+        _same(h1, h0, "h")
+        _same(xs[1], xs[0], "x")
+    _same(tapes[1].K, tapes[0].K, "K tape")
+    _same(tapes[1].V, tapes[0].V, "V tape")
 
 
 # weight gradients whose row count is no multiple of the k-tile: whole k-tiles and the last rows by two launches

@@ -37,7 +37,7 @@ template <typename T> struct EpiSwiGLU {
     static_assert(BN % 64 == 0, "whole 64-column groups");
     constexpr int IPR = BN / 16;   // items of 8 hidden units per row
 #pragma unroll 1
-    for (int it = threadIdx.x; it < TR * IPR; it += 256) {
+    for (int it = tid256(); it < TR * IPR; it += 256) {
       const int r = it / IPR, q = it % IPR, gg = q >> 2, u0 = 8 * (q & 3);
       const int m = m0 + r;
       if (m >= M) continue;
@@ -85,7 +85,7 @@ template <typename T> struct EpiSwiGLUBwd {
     ChunkPre cp;
 #pragma unroll
     for (int i = 0; i < S::NI; ++i) {
-      const int it = threadIdx.x + 256 * i, r = it / S::IPR, u = n0 + 8 * (it % S::IPR);
+      const int it = tid256() + 256 * i, r = it / S::IPR, u = n0 + 8 * (it % S::IPR);
       const T* p = ab + map(min(m0 + r, M - 1)) * 2 * H + item_col(u);
       cp.a[i] = ld8_global(p);
       cp.b[i] = ld8_global(p + MLP_GROUP);
@@ -98,7 +98,7 @@ template <typename T> struct EpiSwiGLUBwd {
     using S = Shape<TR, BN>;
 #pragma unroll
     for (int i = 0; i < S::NI; ++i) {
-      const int it = threadIdx.x + 256 * i, r = it / S::IPR, u = n0 + 8 * (it % S::IPR);
+      const int it = tid256() + 256 * i, r = it / S::IPR, u = n0 + 8 * (it % S::IPR);
       const int m = m0 + r;
       if (m >= M) continue;
       const long row = map(m);

@@ -255,7 +255,7 @@ void run_proj_src(const dm_config* c, const dm_packed* w, const SA& sa, int M, i
   // two direct-to-LDS stages); otherwise 128 x 128 with wave tiles spanning whole heads
   if constexpr (sizeof(T) == 2) {
     if (!small_tiles && M % 256 == 0 && (nseg * c->d) % 256 == 0 && c->d % 64 == 0) {
-      launch_gemm<T, 256, 256, 2, 2, -2>(sa, sb, M, nseg * c->d, c->d, epi, s, PROF_PROJ);
+      launch_gemm<T, 256, 256, 4, 2, -2>(sa, sb, M, nseg * c->d, c->d, epi, s, PROF_PROJ);
       return;
     }
   }

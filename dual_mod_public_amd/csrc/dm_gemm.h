@@ -166,6 +166,11 @@ template <class E, int KD> struct KindEpi {
     e.template tile_apply<KD, BM, BN, LDT>(tile, m0, n0, rs, pre);
   }
 };
+// A block of 512 threads runs a tile epilogue written for 256 on the two halves of each chunk's rows
+// (its threads index with tid256()); KindEpi's epilogues take 512 threads themselves.
+DM_DEV int tid256() { return threadIdx.x & 255; }
+template <class E> struct own_rows { static constexpr bool value = false; };
+template <class E, int KD> struct own_rows<KindEpi<E, KD>> { static constexpr bool value = true; };
 template <class E, class = void> struct tile_rows_of { static constexpr int value = 1 << 30; };
 // An EPI with a static LATE_GATHERS = the exact number of vector-memory load instructions its
 // tile_prefetch issues gets them issued late in the direct-to-LDS k-loop (gemm_mainloop_dma).
@@ -529,33 +534,46 @@ DM_DEV void gemm_mainloop_dma_kk(const SA& sa, const SB& sb, int K, int m0, int 
                 "stages / tile columns");
   using MF = Mfma<T>;
   using WT = WaveTile<BM, BN, WM, WN>;
-  static_assert(WM * WN == 4, "K-major k-loop: 4 waves");
+  constexpr int NWV = WM * WN;
   constexpr int FM = WT::FM, FN = WT::FN, TM = WT::TM, TN = WT::TN;
   constexpr int KS = kk_stage_k<BM, BN, S>();             // k-rows per stage
   constexpr int ROWA = BM * 2, ROWB = BN * 2;              // bytes per k-row
   constexpr int STAGE = KS * (ROWA + ROWB);
   constexpr int RPA = 1024 / ROWA, RPB = 1024 / ROWB;      // k-rows per wave load instruction
-  static_assert(KS % (4 * RPA) == 0 && KS % (4 * RPB) == 0, "whole wave loads per stage");
-  constexpr int LA = KS / RPA / 4, LB = KS / RPB / 4, L = LA + LB;
+  static_assert(KS % (NWV * RPA) == 0 && KS % (NWV * RPB) == 0, "whole wave loads per stage");
+  constexpr int LA = KS / RPA / NWV, LB = KS / RPB / NWV, L = LA + LB;
   constexpr int CPA = ROWA / 16, CPB = ROWB / 16;          // 16-byte chunks per k-row
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
 
+  // Load i of the block covers k-rows [r0, r0 + RP): its address is a uniform base (scalar registers) plus
+  // the lane's 32-bit offset, of which there are at most four for A and four for B (the swizzle's
+  // dependence on the k-row: bits 0, 1 and 3), held over the loop. With whole 64-bit addresses per lane
+  // the loop made 16 of them per k-tile in quarter-rate multiplies, and they and the fragments of four
+  // 128 x 128 wave tiles overflowed the registers (240 copies per k-tile). M x N x K = 4096 x 1024 x 65536:
+  // 673 us (817 TFLOP/s) then, 500 us (1100) with the offsets and eight 64 x 128 wave tiles; four wave
+  // tiles with the offsets were 5% slower than without, eight 128 x 64 ones 6% slower than 64 x 128.
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  auto off_of = [&](int r0, auto row, long ld) {
+    constexpr int ROW = decltype(row)::value, CP = ROW / 16;
+    const int dr = lane / CP;
+    return (unsigned)(dr * (int)ld + 8 * ((lane % CP) ^ kk_swz<ROW>(r0 + dr))) * 2u;
+  };
   auto issue = [&](int kt, int st) {
     char* base = smem + st * STAGE;
-    const int k = kbase + kt * KS;
+    const long k = kbase + (long)kt * KS;
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
-      const int r0 = (wave * LA + i) * RPA, r = r0 + lane / CPA;
-      const int c = (lane % CPA) ^ kk_swz<ROWA>(r);
-      __builtin_amdgcn_global_load_lds((const void*)sa.ptr_k(k + r, m0 + 8 * c), (lds_void_t*)(base + r0 * ROWA),
-                                       16, 0, 0);
+      const int r0 = (uwave * LA + i) * RPA;
+      const char* ub = reinterpret_cast<const char*>(sa.p + (k + r0) * sa.ld + m0);
+      __builtin_amdgcn_global_load_lds((const void*)(ub + off_of(r0, std::integral_constant<int, ROWA>{}, sa.ld)),
+                                       (lds_void_t*)(base + r0 * ROWA), 16, 0, 0);
     }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
-      const int r0 = (wave * LB + i) * RPB, r = r0 + lane / CPB;
-      const int c = (lane % CPB) ^ kk_swz<ROWB>(r);
-      __builtin_amdgcn_global_load_lds((const void*)sb.ptr_k(k + r, n0 + 8 * c),
+      const int r0 = (uwave * LB + i) * RPB;
+      const char* ub = reinterpret_cast<const char*>(sb.p + (k + r0) * sb.ld + n0);
+      __builtin_amdgcn_global_load_lds((const void*)(ub + off_of(r0, std::integral_constant<int, ROWB>{}, sb.ld)),
                                        (lds_void_t*)(base + KS * ROWA + r0 * ROWB), 16, 0, 0);
     }
   };
@@ -720,9 +738,12 @@ DM_DEV void gemm_block_at(const SA& sa, const SB& sb, int K, const EPI& epi, int
     float* tile = reinterpret_cast<float*>(smem);
     const float* rs_lds = reinterpret_cast<const float*>(smem + gemm_stage_bytes<T, BM, BN, D, KM>());
     const int lane = threadIdx.x & 63;
+    constexpr bool HALVES = WM * WN == 8 && !own_rows<EPI>::value;
+    constexpr int TRE = HALVES ? TR / 2 : TR;
+    const int hr = HALVES ? (int)(threadIdx.x >> 8) * TRE : 0;
     constexpr int NCP = has_chunk_pre<EPI>::value ? 2 : 0;
     typename EPI_ChunkPre<EPI>::type cp[2];
-    if constexpr (NCP > 0) cp[0] = epi.template chunk_prefetch<TR, BN>(m0, n0);
+    if constexpr (NCP > 0) cp[0] = epi.template chunk_prefetch<TRE, BN>(m0 + hr, n0);
 #pragma unroll
     for (int c = 0; c < BM / TR; ++c) {
       if (c > 0) __syncthreads();   // the previous chunk has been read
@@ -740,10 +761,11 @@ DM_DEV void gemm_block_at(const SA& sa, const SB& sb, int K, const EPI& epi, int
         if (c == 0) sa.template prepare_store<BM>(pre_a, const_cast<float*>(rs_lds), nullptr, K);
       __syncthreads();
       if constexpr (NCP > 0) {
-        if (c + 1 < BM / TR) cp[(c + 1) & 1] = epi.template chunk_prefetch<TR, BN>(m0 + (c + 1) * TR, n0);
-        epi.template tile_apply<TR, BN, LDT>(tile, m0 + c * TR, n0, rs_lds + c * TR, pre, bz, cp[c & 1]);
+        if (c + 1 < BM / TR) cp[(c + 1) & 1] = epi.template chunk_prefetch<TRE, BN>(m0 + (c + 1) * TR + hr, n0);
+        epi.template tile_apply<TRE, BN, LDT>(tile + hr * LDT, m0 + c * TR + hr, n0, rs_lds + c * TR + hr, pre, bz,
+                                              cp[c & 1]);
       } else {
-        epi.template tile_apply<TR, BN, LDT>(tile, m0 + c * TR, n0, rs_lds + c * TR, pre, bz);
+        epi.template tile_apply<TRE, BN, LDT>(tile + hr * LDT, m0 + c * TR + hr, n0, rs_lds + c * TR + hr, pre, bz);
       }
     }
   } else {
@@ -784,7 +806,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm(SA sa, SB sb, int K, EPI 
 // a split-K k_gemm as a grouped-launch body: slice z of S in grid rows [z * mt, (z + 1) * mt)
 template <typename T, int BM, int BN, int WM, int WN, int D, class SA, class SB, class EPI>
 struct SplitGemmBody {
-  static constexpr int THREADS = 256;
+  static constexpr int THREADS = 64 * WM * WN;
   struct Args {
     SA sa;
     SB sb;
@@ -800,7 +822,7 @@ struct SplitGemmBody {
 // k_gemm as a grouped-launch body (one split-K slice)
 template <typename T, int BM, int BN, int WM, int WN, int D, class SA, class SB, class EPI>
 struct GemmBody {
-  static constexpr int THREADS = 256;
+  static constexpr int THREADS = 64 * WM * WN;
   struct Args {
     SA sa;
     SB sb;
@@ -825,8 +847,13 @@ struct GemmPart {
   EPI epi;
   int gx, gy, nz, skip_z;
   DM_DEV int blocks() const { return gx * gy * nz; }
+  // Blocks go round-robin over the 8 XCDs: each gets a contiguous range of tiles, rows fastest, then
+  // columns, then slices, so that an XCD's L2 takes one slice's columns of A and a few column tiles of B
+  // in place of every slice of A (M = 512, K = 4 x 1024: 2 to 3 MB in place of 6.3; 13.8 -> 13.4 us).
   DM_DEV void run(int L, char* smem) const {
-    const int bx = L % gx, by = (L / gx) % gy, zi = L / (gx * gy);
+    const int nb = gx * gy * nz;
+    const int t = nb % 8 == 0 ? (L % 8) * (nb / 8) + L / 8 : L;
+    const int by = t % gy, bx = (t / gy) % gx, zi = t / (gx * gy);
     const int bz = (skip_z >= 0 && zi >= skip_z) ? zi + 1 : zi;
     gemm_block_at<T, BM_, BN_, WM, WN, D, SA, SB, EPI>(sa, sb, K, epi, bx, by, bz, smem);
   }

@@ -275,11 +275,11 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
     constexpr int L = DH / 8;     // lanes per row
     constexpr int RP = 256 / L;   // rows per pass
     static_assert(TR % RP == 0, "whole passes");
-    const int jj = 4 * (threadIdx.x % L);
+    const int jj = 4 * (tid256() % L);
     const float gn = (seg == 2 && vgain != nullptr) ? vgain[hh] : 0.f;
 #pragma unroll
     for (int pass = 0; pass < TR / RP; ++pass) {
-      const int r = threadIdx.x / L + pass * RP, m = m0 + r;
+      const int r = tid256() / L + pass * RP, m = m0 + r;
       const floatx4 av = *reinterpret_cast<const floatx4*>(tl + r * LDT + jj);
       const floatx4 bv = *reinterpret_cast<const floatx4*>(tl + r * LDT + jj + DH / 2);
       float a[4] = {av.x, av.y, av.z, av.w}, b[4] = {bv.x, bv.y, bv.z, bv.w};
@@ -331,12 +331,12 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
   DM_DEV void rope_block(const float* tl, int m0, int n0, int seg) const {
     constexpr int L = DH / 8, RP = 256 / L, NP = TR / RP;
     static_assert(TR % RP == 0, "whole passes");
-    const int jj = 4 * (threadIdx.x % L);
+    const int jj = 4 * (tid256() % L);
     const int r0 = DEVPOS ? dev_position(pos_dev, pos_cap) : rope_t0;
     float cs[NP][4], sn[NP][4];
 #pragma unroll
     for (int pass = 0; pass < NP; ++pass) {
-      const int m = min(m0 + (int)threadIdx.x / L + pass * RP, M - 1);
+      const int m = min(m0 + tid256() / L + pass * RP, M - 1);
       const int t = m - (m / Tl) * Tl;
       const long rrow = (long)(r0 + t) * (DH / 2) + jj;
       unpackf4(ld_global<floatx4>(cos + rrow), cs[pass]);
@@ -348,7 +348,7 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
       const float* tu = tl + hu * DH;
 #pragma unroll
       for (int pass = 0; pass < NP; ++pass) {
-        const int r = threadIdx.x / L + pass * RP, m = m0 + r;
+        const int r = tid256() / L + pass * RP, m = m0 + r;
         if (m >= M) continue;
         const floatx4 av = *reinterpret_cast<const floatx4*>(tu + r * LDT + jj);
         const floatx4 bv = *reinterpret_cast<const floatx4*>(tu + r * LDT + jj + DH / 2);
@@ -385,7 +385,7 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
   template <int TR, int BN, int LDT>
   DM_DEV void row_block(const float* tl, int m0, int n0, int seg) const {
     constexpr int NU = BN / DH, L = DH / 4;
-    const int e = 4 * (threadIdx.x % L);
+    const int e = 4 * (tid256() % L);
     float bs[NU][4];
 #pragma unroll
     for (int hu = 0; hu < NU; ++hu) {
@@ -402,7 +402,7 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
   template <int TR, int LDT>
   DM_DEV void row_unit(const float* tl, int m0, int seg, int c0) const {
     constexpr int L = DH / 4;
-    const int e = 4 * (threadIdx.x % L), col = c0 + e;
+    const int e = 4 * (tid256() % L), col = c0 + e;
     float bs[4] = {0.f, 0.f, 0.f, 0.f};
     if (!(seg == 5 && fusion)) unpackf4(ld_global<floatx4>(bias + (seg - 3) * d + col), bs);
     row_rows<TR, LDT>(tl, m0, seg, c0, bs);
@@ -412,10 +412,10 @@ template <typename T, int DH, bool DEVPOS = false> struct EpiProj {
     constexpr int L = DH / 4;
     constexpr int RP = 256 / L;
     static_assert(TR % RP == 0, "whole passes");
-    const int e = 4 * (threadIdx.x % L), col = c0 + e;
+    const int e = 4 * (tid256() % L), col = c0 + e;
 #pragma unroll
     for (int pass = 0; pass < TR / RP; ++pass) {
-      const int r = threadIdx.x / L + pass * RP, m = m0 + r;
+      const int r = tid256() / L + pass * RP, m = m0 + r;
       if (m >= M) continue;
       gate_item(seg, m, col, *reinterpret_cast<const floatx4*>(tl + r * LDT + e), bs);
     }
@@ -1633,7 +1633,7 @@ template <typename T> struct EpiResidual {
     using S = Shape<TR, BN>;
     ChunkPre cp;
     if (x == nullptr) return cp;   // uniform
-    const int cg = threadIdx.x % S::TPR, r0 = threadIdx.x / S::TPR;
+    const int cg = tid256() % S::TPR, r0 = tid256() / S::TPR;
 #pragma unroll
     for (int p = 0; p < S::NP; ++p)
       cp.v[p] = ld8_global(x + map(min(m0 + r0 + p * S::RPP, M - 1)) * N + n0 + cg * VEC);
@@ -1643,7 +1643,7 @@ template <typename T> struct EpiResidual {
   DM_DEV void tile_apply(const float* tile, int m0, int n0, const float*, const TilePre&, int,
                          const ChunkPre& cp) const {
     using S = Shape<TR, BN>;
-    const int cg = threadIdx.x % S::TPR, r0 = threadIdx.x / S::TPR;
+    const int cg = tid256() % S::TPR, r0 = tid256() / S::TPR;
 #pragma unroll
     for (int p = 0; p < S::NP; ++p) {
       const int r = r0 + p * S::RPP, m = m0 + r;
@@ -1677,7 +1677,7 @@ struct EpiStoreTileF32 {
     float* __restrict__ C = this->C + (long)z * zstride;
 #pragma unroll
     for (int it = 0; it < NV / 256; ++it) {
-      const int idx = it * 256 + threadIdx.x, r = idx / C4, c = 4 * (idx % C4);
+      const int idx = it * 256 + tid256(), r = idx / C4, c = 4 * (idx % C4);
       const floatx4 v = *reinterpret_cast<const floatx4*>(tile + r * LDT + c);
       if (m0 + r < M) *reinterpret_cast<floatx4*>(C + map(m0 + r) * N + n0 + c) = v;
     }

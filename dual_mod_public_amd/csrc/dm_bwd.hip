@@ -202,6 +202,7 @@ void gemm_tn(const T* A, long lda, const T* Bm, long ldb, float* C, int M, int N
   EpiStoreTileF32 ep{M, N, part, (long)M * N};
   if constexpr (sizeof(T) == 2) {
     if (big) launch_gemm_splitk<T, 256, 256, 4, 2, -KK_STAGES>(sa, sb, M, N, K, S, ep, s);
+    else if (dma && two_stages_128(blocks * S)) launch_gemm_splitk<T, 128, 128, 2, 2, -2>(sa, sb, M, N, K, S, ep, s);
     else if (dma) launch_gemm_splitk<T, 128, 128, 2, 2, -3>(sa, sb, M, N, K, S, ep, s);
     else launch_gemm_splitk<T, 128, 128, 2, 2, 4>(sa, sb, M, N, K, S, ep, s);
   } else {
@@ -451,7 +452,7 @@ void bwd_cell(const dm_config* c, const dm_packed* w, const float* cos, const fl
           // (half the LDS traffic per product; every element's k order is the same, so the results
           // are too)
           grouped = true;
-          using PDu = GemmPart<T, 128, 128, 2, 2, -3, SrcRows<T>, SrcRows<T>, EpiStoreTileF32>;
+          using PDu = GemmPart<T, 128, 128, 2, 2, -2, SrcRows<T>, SrcRows<T>, EpiStoreTileF32>;
           using PVin = GemmPart<T, 64, 32, 4, 1, -SW2_STAGES, SrcRows<T>, SrcRows<T>, EpiVinBwd<T, 32>>;
           const EpiVinBwd<T, 32> ev{g, N, c->ctx_mod, c->mult_res_lambda, sv.save1 + sw * NS * 4 * d,
                                     (const T*)L->sig, dctx + sw * NS * 4 * d, ws.dsig, ws.lamdv};
@@ -476,7 +477,7 @@ void bwd_cell(const dm_config* c, const dm_packed* w, const float* cos, const fl
       }
     } else {
       if (sizeof(T) == 2 && launch_log() != nullptr)
-        launch_gemm_splitk<T, 128, 128, 2, 2, sizeof(T) == 2 ? -3 : 4>(da, db, N, d, 4 * d, DU_SPLIT, ep, s);
+        launch_gemm_splitk<T, 128, 128, 2, 2, sizeof(T) == 2 ? -2 : 4>(da, db, N, d, 4 * d, DU_SPLIT, ep, s);
       else
         launch_gemm_splitk<T, 64, 64, 2, 2, sizeof(T) == 2 ? -DU_STAGES : 4>(da, db, N, d, 4 * d, DU_SPLIT, ep, s);
       const dim3 egrid(cdiv(N, 16), d / DU_EPI_TN);

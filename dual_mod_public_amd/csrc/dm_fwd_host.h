@@ -251,7 +251,7 @@ void run_proj_src(const dm_config* c, const dm_packed* w, const SA& sa, int M, i
   }
   EpiProj<T, DH> epi{M, c->d, c->h, Tl, Tbuf, buf_t0, rope_t0, cos, sin, w->b_proj,
                      qr, kraw, kself, vraw, glogx, sig, c->ctx_mod == DM_CTX_FUSION, v_gain(c, w), vpre};
-  // bf16, whole 256-row / 256-column tiles: 256 x 256 blocks (four 128 x 128 wave tiles,
+  // bf16, whole 256-row / 256-column tiles: 256 x 256 blocks (eight 64 x 128 wave tiles,
   // two direct-to-LDS stages); otherwise 128 x 128 with wave tiles spanning whole heads
   if constexpr (sizeof(T) == 2) {
     if (!small_tiles && M % 256 == 0 && (nseg * c->d) % 256 == 0 && c->d % 64 == 0) {
@@ -268,9 +268,9 @@ void run_proj_src(const dm_config* c, const dm_packed* w, const SA& sa, int M, i
     return;
   }
   if constexpr (DH == 64)
-    launch_gemm_auto<T, 128, 128, 2, 2, 3, 4>(sa, sb, M, nseg * c->d, c->d, epi, s, PROF_PROJ);
+    launch_gemm_128<T, 2, 2>(sa, sb, M, nseg * c->d, c->d, epi, s, PROF_PROJ);
   else
-    launch_gemm_auto<T, 128, 128, 4, 1, 3, 4>(sa, sb, M, nseg * c->d, c->d, epi, s, PROF_PROJ);
+    launch_gemm_128<T, 4, 1>(sa, sb, M, nseg * c->d, c->d, epi, s, PROF_PROJ);
 }
 
 template <typename T, int DH>

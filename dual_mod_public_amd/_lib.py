@@ -157,6 +157,8 @@ SIGNATURES = {
     "dm_refine_kv": (ctypes.c_int, [P(dm_config), P(dm_packed), P(dm_layer_bufs), c_vp, c_fp, c_fp, c_vp, c_vp,
                                     c_vp, ctypes.c_size_t, c_vp]),
     "dm_linear": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_vp]),
+    "dm_embed_bwd": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_vp]),
+    "dm_ce_rows": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_vp]),
     "dm_argmax_rows": (ctypes.c_int, [c_i32, c_vp, c_i32, c_i32, ctypes.c_int64, c_vp, c_vp]),
     "dm_stack_fwd_plan_bytes": (ctypes.c_size_t, [P(dm_config), c_i32, P(dm_stack_layer), P(c_i32), c_i32, c_i32]),
     "dm_stack_fwd": (ctypes.c_int, [P(dm_config), c_i32, P(dm_stack_layer), c_fp, c_fp, P(c_i32), c_i32, c_i32,
@@ -308,6 +310,27 @@ def residual_rmsnorm(x, delta=None, w=None, dtype=torch.bfloat16, y=None, eps=1e
                                     ptr(w) if w is not None else None, ptr(y) if w is not None else None, M, d,
                                     float(eps), stream_ptr()))
     return y if w is not None else None
+
+
+def embed_bwd(dx, idx, g):
+    """dm_embed_bwd on contiguous device tensors: g[idx[m]] += dx[m] (g fp32 [n, d], idx int64 [M], dx [M, d])."""
+    M, d = dx.shape
+    assert dx.is_contiguous() and idx.is_contiguous() and g.is_contiguous()
+    assert idx.dtype == torch.int64 and idx.numel() == M and g.dtype == torch.float32 and g.shape[1] == d
+    check(lib().dm_embed_bwd(dtype_code(dx.dtype), ptr(dx), ptr(idx), ptr(g), M, d, g.shape[0], stream_ptr()))
+
+
+def ce_rows(logits, target, nvalid):
+    """dm_ce_rows on contiguous device tensors: the rows' cross entropies (fp32 [M], 0 for targets < 0);
+    logits [M, V] becomes the gradient of their sum / nvalid (a one-element fp32 tensor)."""
+    M, V = logits.shape
+    assert logits.is_contiguous() and target.is_contiguous()
+    assert target.dtype == torch.int64 and target.numel() == M
+    assert nvalid.dtype == torch.float32 and nvalid.numel() == 1
+    loss = torch.empty(M, device=logits.device, dtype=torch.float32)
+    check(lib().dm_ce_rows(dtype_code(logits.dtype), ptr(logits), ptr(target), ptr(nvalid), ptr(loss), M, V,
+                           stream_ptr()))
+    return loss
 
 
 MLP_ROWS = 64   # rows dm_swiglu_rows takes per call

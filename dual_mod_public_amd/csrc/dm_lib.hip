@@ -760,6 +760,38 @@ int dm_residual_rmsnorm(int32_t dtype, float* x, const void* delta, const float*
   return DM_OK;
 }
 
+int dm_embed_bwd(int32_t dtype, const void* dx, const int64_t* idx, float* g, int32_t M, int32_t d, int32_t n,
+                 void* stream) {
+  DM_REQUIRE(dx && idx && g, DM_ERR_INVALID, "null operand");
+  DM_REQUIRE(M > 0 && d > 0 && n > 0, DM_ERR_INVALID, "M=%d d=%d n=%d", M, d, n);
+  DM_REQUIRE(dtype == DM_BF16 || dtype == DM_F32, DM_ERR_INVALID, "dtype %d", dtype);
+  hipStream_t s = S(stream);
+  if (dtype == DM_BF16) hipLaunchKernelGGL(k_embed_bwd<bf16>, dim3(M), dim3(256), 0, s, (const bf16*)dx, idx, g, M, d, n);
+  else hipLaunchKernelGGL(k_embed_bwd<float>, dim3(M), dim3(256), 0, s, (const float*)dx, idx, g, M, d, n);
+  DM_HIP(hipGetLastError());
+  return DM_OK;
+}
+
+int dm_ce_rows(int32_t dtype, void* logits, const int64_t* target, const float* nvalid, float* loss, int32_t rows,
+               int32_t cols, void* stream) {
+  DM_REQUIRE(logits && target && nvalid && loss, DM_ERR_INVALID, "null operand");
+  DM_REQUIRE(rows > 0 && cols > 0, DM_ERR_INVALID, "rows=%d cols=%d", rows, cols);
+  DM_REQUIRE(dtype == DM_BF16 || dtype == DM_F32, DM_ERR_INVALID, "dtype %d", dtype);
+  hipStream_t s = S(stream);
+  auto run = [&](auto tag) {
+    using T = decltype(tag);
+    constexpr int V = 16 / (int)sizeof(T);
+    if (aligned16(logits) && cols % V == 0)
+      hipLaunchKernelGGL((k_ce_rows<T, V>), dim3(rows), dim3(256), 0, s, (T*)logits, target, nvalid, loss, cols);
+    else
+      hipLaunchKernelGGL((k_ce_rows<T, 1>), dim3(rows), dim3(256), 0, s, (T*)logits, target, nvalid, loss, cols);
+  };
+  if (dtype == DM_BF16) run(bf16{});
+  else run(float{});
+  DM_HIP(hipGetLastError());
+  return DM_OK;
+}
+
 int dm_argmax_rows(int32_t dtype, const void* x, int32_t rows, int32_t cols, int64_t ld, int64_t* out,
                    void* stream) {
   DM_REQUIRE(x && out, DM_ERR_INVALID, "null operand");

@@ -330,14 +330,8 @@ class HipTrunk:
             r1 = min(r0 + self.loss_chunk, M)
             xc, t = x[r0:r1], tg[r0:r1]
             hf, r = _rms(xc, m.norm_f.weight, m.norm_f.eps)
-            lg = (hf @ self.w_emb.t()).float()
-            lse = torch.logsumexp(lg, -1)
-            valid = t >= 0
-            tc = t.clamp_min(0)
-            loss = loss + ((lse - lg.gather(1, tc[:, None])[:, 0]) * valid).sum()
-            p = torch.exp(lg - lse[:, None])
-            p.scatter_add_(1, tc[:, None], -valid[:, None].float())
-            dl = (p * (valid[:, None].float() / nvalid)).to(self.dt)
+            dl = hf @ self.w_emb.t()
+            loss = loss + L.ce_rows(dl, t, nvalid).sum()   # dl: the logits, then their gradient
             gw.add_(_mm32(dl.t(), hf))
             dhf = dl @ self.w_emb
             dxl[r0:r1].copy_(_rms_vjp(dhf, xc, r, m.norm_f.weight, gnf))
@@ -345,9 +339,7 @@ class HipTrunk:
 
     def _embed_bwd(self):
         M, d = self.B * self.T, self.cfg.d_model
-        g = torch.ops.aten.embedding_dense_backward(self.dxs[0].view(M, d).float(), self.idx.view(M),
-                                                    self.cfg.vocab_size, -1, False)
-        self.grad["tok_emb.weight"].add_(g)
+        L.embed_bwd(self.dxs[0].view(M, d), self.idx.view(M), self.grad["tok_emb.weight"])
 
     def _run(self):
         with torch.no_grad():

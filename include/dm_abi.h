@@ -495,6 +495,20 @@ int dm_residual_rmsnorm(int32_t dtype, float* x, const void* delta, const float*
 int dm_swiglu_rows(int32_t dtype, const void* x, const void* w1, const void* w3, const void* w2, void* act,
                    void* out, int32_t M, int32_t d, int32_t H, void* stream);
 
+/* ---- embedding backward ----------------------------------------------------------------
+ * g [n, d] fp32: g[idx[m]] += dx[m] for the M rows of dx [M, d] (storage dtype bf16 or fp32), the rows of
+ * an id summed in ascending order in fp32 (graphs.py:503). No library sort, nothing to clear. */
+int dm_embed_bwd(int32_t dtype, const void* dx, const int64_t* idx, float* g, int32_t M, int32_t d, int32_t n,
+                 void* stream);
+
+/* ---- cross entropy of logit rows, with its gradient -----------------------------------
+ * logits [rows, cols] (contiguous, storage dtype bf16 or fp32), target [rows] int64 (< 0: ignored),
+ * nvalid: one fp32 on the device. loss[r] = logsumexp(logits[r]) - logits[r, target[r]] (0 where
+ * ignored; NaN for a target >= cols), and the logits are replaced by the gradient of sum(loss) / nvalid
+ * (models/dualmod/model.py:279-281, graphs.py:322-341). Statistics in fp32, one block per row. */
+int dm_ce_rows(int32_t dtype, void* logits, const int64_t* target, const float* nvalid, float* loss, int32_t rows,
+               int32_t cols, void* stream);
+
 /* ---- row argmax ------------------------------------------------------------------
  * out[r] = the first index of the maximum of x[r, 0:cols) (row stride ld elements),
  * storage dtype bf16 or fp32: the greedy pick of lm/eval/graph_decode.py:62

@@ -196,3 +196,45 @@ def test_weight_grad_last_rows(M):
         err = ((g[k].double().cpu() - ref).norm() / ref.norm()).item()
         # fp32 sums of M exact products: at most M 2^-24 of sum |a b|, which is about sqrt(M) |sum a b|
         assert err < M ** 1.5 * 2 ** -24, (k, err)
+
+
+# cross entropy rows and their gradient: vector rows, rows of no whole vectors, fewer columns than threads,
+# ignored targets; against fp64
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,V", [(1, 3), (5, 1000), (7, 2049), (33, 32000)])
+def test_ce_rows(dt, M, V):
+    say(f"cross entropy rows {dt} M={M} V={V}")
+    x = (4 * _rand(M, V, seed=1).float()).to(dt)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    t = torch.randint(0, V, (M,), generator=g, device=DEV)
+    t[M // 2::3] = -1
+    nv = (t >= 0).sum().clamp_min(1).float()
+    leaf = x.double().cpu().requires_grad_(True)
+    ref = torch.nn.functional.cross_entropy(leaf, t.cpu(), ignore_index=-1, reduction="none")
+    (ref.sum() / nv.double().cpu()).backward()
+    loss = L.ce_rows(x, t, nv)
+    torch.cuda.synchronize()
+    # fp32 sums of V exponentials (1 ulp each): 256 partial sums of V / 256 terms, then a tree
+    tol = (V / 256 + 16) * 2 ** -23
+    assert ((loss.double().cpu() - ref.detach()).abs() <= tol * (1 + ref.detach().abs())).all()
+    d = (x.double().cpu() - leaf.grad).abs()
+    rnd = 2 ** -8 if dt == torch.bfloat16 else 0.0   # the stored gradient's rounding
+    # exp(x - lse): |x - lse| <= 64 rounded to 2^-19 absolute, then the sum's error
+    assert (d <= leaf.grad.abs() * (rnd + tol + 2 ** -18) + 2 ** -22 / nv.item()).all(), d.max()
+
+
+# embedding backward: repeated ids across the block's 256-token passes, one id for all, d beyond one pass
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,d,n", [(1, 64, 5), (300, 128, 7), (700, 2176, 400), (513, 64, 1)])
+def test_embed_bwd(dt, M, d, n):
+    say(f"embedding backward {dt} M={M} d={d} n={n}")
+    dx = _rand(M, d, seed=1).to(dt)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    idx = torch.randint(0, n, (M,), generator=g, device=DEV)
+    out = _rand(n, d, seed=3).float()
+    ref = out.double().cpu().index_add_(0, idx.cpu(), dx.double().cpu())
+    mag = out.abs().double().cpu().index_add_(0, idx.cpu(), dx.abs().double().cpu())
+    L.embed_bwd(dx, idx, out)
+    torch.cuda.synchronize()
+    # fp32 sums of at most M + 1 terms
+    assert ((out.double().cpu() - ref).abs() <= (M + 1) * 2 ** -24 * mag).all()

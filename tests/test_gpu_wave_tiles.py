@@ -238,3 +238,22 @@ def test_embed_bwd(dt, M, d, n):
     torch.cuda.synchronize()
     # fp32 sums of at most M + 1 terms
     assert ((out.double().cpu() - ref).abs() <= (M + 1) * 2 ** -24 * mag).all()
+
+
+def test_captured_trunk_new_tokens():
+    """A captured trunk step of 4096 tokens replayed with new ids each time, against eager steps between the
+    replays (the ids are not sorted by a library call in the step), bit for bit."""
+    from dual_mod_public_amd.trunk import HipTrunk
+    from tests.test_gpu_trunk import _batch, _cfg, _model, _same as same_bits, _snapshot
+    say("captured trunk, 4096 tokens, new ids per replay")
+    cfg = _cfg(n_layers=1, max_seq_len=1024)
+    B, T = 4, 1024
+    m, _ = _model(cfg, torch.bfloat16)
+    a, b = HipTrunk(m, B, T), HipTrunk(m, B, T)
+    b.capture()
+    for seed in (21, 22, 23, 24):
+        idx, tg = (t.to(DEV) for t in _batch(cfg, B, T, seed=seed))
+        a.train_step(idx, tg)
+        b.train_step(idx, tg)
+        torch.cuda.synchronize()
+        assert same_bits(_snapshot(a), _snapshot(b)), seed

@@ -222,7 +222,7 @@ __global__ __launch_bounds__(64) void k_decode_merge(DecodeArgs<T> a) {
 // split of L keys (the split kernel's arithmetic), their states in LDS, merged by the first wave (the
 // merge kernel's arithmetic: the same results as the two launches). A launch and a round trip of the
 // partials less; the grid is B*h blocks whatever the tape's length, so it pays while NS groups cover
-// the read and B*h blocks of them are resident together (decode_reads_direct).
+// the read and B*h blocks of them are resident together (run_decode_read).
 template <typename T, int DH, int L, int NS>
 __global__ __launch_bounds__((dec_threads<T, DH>() * NS)) void k_decode_direct(DecodeArgs<T> a) {
   constexpr int NT = dec_threads<T, DH>();

@@ -343,13 +343,13 @@ DecWs carve_dec(const dm_config* c, int tape_T, void* base) {
   return w;
 }
 
-// The tape read: one launch where NS groups of a block cover it (decode_reads_direct), else split
+// The tape read: one launch where NS groups of a block cover it, else split
 // partials and their merge; the same results.
 template <typename T, int DH>
 void run_decode_read(DecodeArgs<T>& da, hipStream_t s) {
   const int BH = da.B * da.h;
   // One launch while a (b, h)'s splits fit one block and the chip still holds the grid: with more
-  // than one split per (b, h) each block keeps 256 threads per split resident until the slowest is
+  // than one split per (b, h) each block keeps its threads (256 or 512 per split) resident until the slowest is
   // done, so from 512 (b, h) up the split grid balances better.
   constexpr int NT = dec_threads<T, DH>(), NSMAX = 1024 / NT;
   if (da.nsplit >= 1 && (da.nsplit == 1 || (da.nsplit <= NSMAX && BH <= 512))) {

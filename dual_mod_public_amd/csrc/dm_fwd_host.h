@@ -126,17 +126,19 @@ template <typename T> bool wt_ok(int M, const void* A, const void* W) {
 // f(WTile) with the tile of least expected time for M x N outputs (N a multiple of 64): a wave's
 // own time goes with its operand rows (8 NA + 16 CT; 57 ns each per 1024 of k), a CU's with the sum
 // over its waves (35 ns per row); fitted to 30 measured (M, N, tile) times, K = 512 .. 2048, M = 1 ..
-// 256, all within 15% of the best tile. max_ct: the epilogue's widest tile.
-template <class F> void with_wt(int M, int N, int max_ct, const F& f) {
+// 256, all within 15% of the best tile. tall: also 64 rows x 32 columns, which read the weights once
+// where shorter tiles read them twice (a tie goes to it: M = 33, N = 11008, K = 2048 17.0 us against
+// 18.5 and 21.8; N = 21888, K = 4096 55.4 against 63.9).
+template <class F> void with_wt(int M, int N, const F& f, bool tall = false) {
   struct C { int na, ct; };
-  constexpr C cand[] = {{1, 1}, {2, 1}, {2, 2}, {4, 1}, {4, 2}, {4, 4}};
+  constexpr C cand[] = {{1, 1}, {2, 1}, {2, 2}, {4, 1}, {4, 2}, {4, 4}, {8, 2}};
   int best = 0;
   long bt = -1;
-  for (int i = 0; i < 6; ++i) {
-    if (cand[i].ct > max_ct || (i > 0 && M <= 8 * cand[i - 1].na && cand[i].na > cand[i - 1].na)) continue;
+  for (int i = 0; i < (tall ? 7 : 6); ++i) {
+    if (i > 0 && M <= 8 * cand[i - 1].na && cand[i].na > cand[i - 1].na) continue;
     const long rows = 8 * cand[i].na + 16 * cand[i].ct, waves = (long)cdiv(M, 8 * cand[i].na) * (N / (16 * cand[i].ct));
     const long t = std::max<long>(57 * rows, 35 * rows * cdiv(waves, 256));
-    if (bt < 0 || t < bt) {
+    if (bt < 0 || t < bt || (i == 6 && t == bt)) {
       bt = t;
       best = i;
     }
@@ -147,44 +149,55 @@ template <class F> void with_wt(int M, int N, int max_ct, const F& f) {
     case 2: f(WTile<2, 2>{}); break;
     case 3: f(WTile<4, 1>{}); break;
     case 4: f(WTile<4, 2>{}); break;
-    default: f(WTile<4, 4>{}); break;
+    case 5: f(WTile<4, 4>{}); break;
+    default: f(WTile<8, 2>{}); break;
   }
 }
-// N output columns, halved for an epilogue that takes two weight rows per column (pair = 2)
+// N weight rows (WtSwiGLU: both matrices')
 template <typename T, class E>
-void launch_wt(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls = PROF_NONE, int max_ct = 4) {
-  with_wt(op.M, N, max_ct, [&](auto wt) {
+void launch_wt(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls = PROF_NONE) {
+  with_wt(op.M, N, [&](auto wt) {
     using WT = decltype(wt);
-    op.nx = N / WT::COLS;
-    launch_k(prof_cls, k_wt<T, WT, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64), 0, s, op, e);
-  });
+    if constexpr (WT::NA <= 4 || E::TALL) {
+      op.nx = N / WT::COLS;
+      launch_k(prof_cls, k_wt<T, WT, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64), 0, s, op, e);
+    }
+  }, E::TALL);
 }
-// a product with a long K whose tiles would leave half of the CUs idle: K over four waves per tile
+// a product summed in parts (a step's W_O and MLP products, M <= ROWS_MAX): four waves per 16-column tile
+// while that gives the CUs at most two such blocks each, of short rings (two to a CU); eighths always, in
+// taller and wider tiles beyond. Measured at weights from HBM, four waves against one per tile (which for
+// the down products summed one chain): M = 1, d x H = 512 x 1376: up 3.1 against 3.7 us, down 3.5 / 4.9;
+// 1024 x 2752: 5.1 / 5.8, 4.9 / 7.9; M = 64: up 9.6 / 8.0, down 5.6 / 8.2; 2048 x 5504, M = 32: up
+// 17.7 / 13.5, down 8.5 / 14.6; W_O, M = 16, d = 1024: 3.5 / 4.4. Rings of 6 to 8 stages, one block to a
+// CU: down 5.1 against 4.9 at M = 1, 9.5 against 8.5 at M = 32.
 template <typename T, class E>
-void launch_wt_long(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls = PROF_NONE) {
-  constexpr int KW = 4;
-  if (op.K < 1536 || (long)cdiv(op.M, 32) * (N / 16) > 128) {
-    launch_wt(op, N, e, s, prof_cls);
-    return;
-  }
+void launch_wt_parts(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls = PROF_NONE) {
   auto run = [&](auto wt) {
     using WT = decltype(wt);
     op.nx = N / WT::COLS;
-    launch_k(prof_cls, k_wt_ksplit<T, WT, KW, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64 * KW), 0, s, op, e);
+    launch_k(prof_cls, k_wt_ksplit<T, WT, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64 * WT_PARTS), 0, s, op, e);
   };
-  if (op.M <= 8) run(WTile<1, 1>{});
-  else if (op.M <= 16) run(WTile<2, 1>{});
-  else run(WTile<4, 1, 6>{});
+  if (op.M <= 8) return run(WTile<1, 1, 4>{});
+  if ((long)cdiv(op.M, 16) * (N / 16) < 512) return run(WTile<2, 1, 4>{});
+  if constexpr (E::SUM == WT_EIGHTHS) {
+    if ((long)cdiv(op.M, 32) * (N / 16) < 512) run(WTile<4, 1, 3>{});
+    else run(WTile<4, 2, 3>{});
+  } else {
+    launch_wt(op, N, e, s, prof_cls);
+  }
 }
 template <typename T, class E1, class E2>
 void launch_wt2(WtOp<T> op1, int N1, const E1& e1, WtOp<T> op2, int N2, const E2& e2, hipStream_t s,
                 int prof_cls = PROF_NONE) {
-  with_wt(op1.M, N1 + N2, 4, [&](auto wt) {
+  with_wt(op1.M, N1 + N2, [&](auto wt) {
     using WT = decltype(wt);
-    op1.nx = N1 / WT::COLS;
-    op2.nx = N2 / WT::COLS;
-    launch_k(prof_cls, k_wt2<T, WT, E1, E2>, dim3(op1.nx + op2.nx, cdiv(op1.M, WT::ROWS)), dim3(64), 0, s, op1, e1, op2,
-             e2);
+    if constexpr (WT::NA <= 4) {
+      op1.nx = N1 / WT::COLS;
+      op2.nx = N2 / WT::COLS;
+      launch_k(prof_cls, k_wt2<T, WT, E1, E2>, dim3(op1.nx + op2.nx, cdiv(op1.M, WT::ROWS)), dim3(64), 0, s, op1, e1,
+               op2, e2);
+    }
   });
 }
 // What rides in a decode step's refine: the W_O product in its first launch (both read o_cat), and the
@@ -323,7 +336,7 @@ void run_refine_wt(const dm_config* c, const dm_packed* w, const CellGeom& g, in
       ssq, c->h, 1.0f / (float)d, c->rms_eps};
   const WtOp<T> op1{o, d, N, d};
   if (wo != nullptr)
-    launch_wt2(op1, 4 * d, e1, op1, d, WtStore<T>{wo->W, d, wo->y, N, d}, s, PROF_SWEEP1);
+    launch_wt2(op1, 4 * d, e1, op1, d, WtStore<T, WT_EIGHTHS>{wo->W, d, wo->y, N, d}, s, PROF_SWEEP1);
   else
     launch_wt(op1, 4 * d, e1, s, PROF_SWEEP1);
   if (c->ctx_mod == DM_CTX_LINEAR) return;

@@ -456,7 +456,9 @@ int run_decode(const dm_config* c, const dm_packed* w, const float* cos, const f
     bool done = false;
     if constexpr (sizeof(T) == 2) {
       if (wt_ok<T>(B, a->o_cat, w->wo)) {
-        launch_wt(WtOp<T>{(const T*)a->o_cat, d, B, d}, d, WtStore<T>{(const T*)w->wo, d, (T*)a->y, B, d}, s);
+        const WtOp<T> op{(const T*)a->o_cat, d, B, d};
+        if (B <= ROWS_MAX) launch_wt_parts(op, d, WtStore<T, WT_EIGHTHS>{(const T*)w->wo, d, (T*)a->y, B, d}, s);
+        else launch_wt(op, d, WtStore<T, WT_CHAIN>{(const T*)w->wo, d, (T*)a->y, B, d}, s);
         done = true;
       }
     }
@@ -731,9 +733,10 @@ int dm_swiglu_rows(int32_t dtype, const void* x, const void* w1, const void* w3,
   DM_REQUIRE(aligned16(x) && aligned16(w1) && aligned16(w3) && aligned16(w2) && aligned16(act), DM_ERR_INVALID,
              "operands must be 16-byte aligned");
   hipStream_t s = S(stream);
-  launch_wt(WtOp<bf16>{(const bf16*)x, d, M, d}, 2 * H,
-            WtSwiGLU<bf16>{(const bf16*)w1, (const bf16*)w3, d, (bf16*)act, M, H}, s);
-  launch_wt_long(WtOp<bf16>{(const bf16*)act, H, M, H}, d, WtStore<bf16>{(const bf16*)w2, H, (bf16*)out, M, d}, s);
+  launch_wt_parts(WtOp<bf16>{(const bf16*)x, d, M, d}, 2 * H,
+                  WtSwiGLU<bf16>{(const bf16*)w1, (const bf16*)w3, d, (bf16*)act, M, H}, s);
+  launch_wt_parts(WtOp<bf16>{(const bf16*)act, H, M, H}, d,
+                  WtStore<bf16, WT_EIGHTHS>{(const bf16*)w2, H, (bf16*)out, M, d}, s);
   DM_HIP(hipGetLastError());
   return DM_OK;
 }

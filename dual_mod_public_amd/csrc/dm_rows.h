@@ -9,13 +9,15 @@
 // global memory (S - 1 of the 64-wide k steps in flight, no register held by a load) and waits for
 // its own loads only; there is no barrier. A load instruction moves eight whole 128-byte lines
 // (fragments loaded straight into registers, half a line per row, moved half as many bytes per clock
-// of a CU). The tile is chosen by wt_config so that the waves spread over the CUs.
+// of a CU). The tile is chosen (with_wt) so that the waves spread over the CUs.
 // Measured on MI355X (K = 1024, weights from HBM, plain store; launch alone 2.3 us):
 //   M =   8, N = 4096: 3.9 us, N = 6144: 4.3     (64 x 64 block tiles in place: 12.1, 9.5 with their epilogues)
 //   M =  64, N = 4096: 5.8;  M = 128: 6.7;  M = 256: 9.0     (64 x 128 blocks in place: 12.6, 12.6, 13.1)
 // From M = 512 on (13.6 us) sharing the operands between a block's waves wins (13.0 with its epilogue).
-// Every output still sums its k in ascending 32-wide MFMA steps, as the tiled GEMMs do, so a row's
-// result does not depend on which of the two computed it.
+// The order of an output's sum over k is fixed by the product, never by the rows of the call or the
+// tile that computes it, so a row's result is the same in every batch (WtSum): the products that larger
+// calls run on the tiled GEMMs sum as those do, one chain over ascending 32-wide MFMA steps; a step's W_O
+// and MLP products sum partial chains.
 //
 // An epilogue chooses the 16 CT weight rows of a tile (wrow), so that its items are complete inside
 // the tile (a RoPE pair, a key's candidate and gate halves), gathers its inputs ahead of the k-loop
@@ -48,19 +50,54 @@ template <int... I, class F> DM_DEV void static_steps(std::integer_sequence<int,
   (f(std::integral_constant<int, I>{}), ...);
 }
 
+// The order of the sum over k: one chain of ascending 32-wide MFMA steps; four chains over K's quarters
+// (K a multiple of 128), added in order; or eight chains, the j-th over the steps j, j + 8, ..., added in
+// order. One wave walks the quarters one after the other, the eighths as four pairs (steps j, j + 1 share
+// a 64-wide load; eight accumulators per output over an ascending walk: W_O at d = 1024 6.1 us against
+// 4.7); four waves (k_wt_ksplit) take a quarter or a pair each: the same sums.
+enum WtSum { WT_CHAIN = 0, WT_QUARTERS = 1, WT_EIGHTHS = 2 };
+constexpr int WT_PARTS = 4;   // quarters, or pairs of eighths
+template <int SUM, bool PART> struct WtWalk {   // over the 64-wide loads of one part, or of all
+  int K, k, end, part;
+  static constexpr bool PARTS = SUM != WT_CHAIN && !PART;
+  static constexpr int STRIDE = SUM == WT_EIGHTHS ? 64 * WT_PARTS : 64;
+  DM_DEV WtWalk(int K_, int part_) : K(K_), k(0), end(K_), part(part_) { set(); }
+  DM_DEV void set() {
+    if (SUM == WT_EIGHTHS) k = 64 * part;
+    if (SUM == WT_QUARTERS) {
+      k = part * (K / 4);
+      end = k + K / 4;
+    }
+  }
+  DM_DEV bool last() const { return k + STRIDE >= end; }   // of its part
+  DM_DEV void next() {
+    k += STRIDE;
+    if (PARTS && k >= end) {
+      ++part;
+      set();
+    }
+  }
+  DM_DEV int steps() const {
+    if (SUM == WT_QUARTERS) return (PARTS ? WT_PARTS : 1) * ((K / 4 + 63) / 64);
+    return SUM == WT_EIGHTHS && PART ? max(0, (K - 64 * part + STRIDE - 1) / STRIDE) : (K + 63) / 64;
+  }
+};
+
 template <typename T> struct WtOp {   // the A operand: row m at A + m lda; K a multiple of 32
   const T* A;
   long lda;
   int M, K, nx;   // nx column tiles
 };
 
-// The accumulators of one tile (column tile bx, row tile by) by one wave, over its 64-wide k steps
-// [kt0, kt0 + nk); leaves the stages free.
-template <typename T, class WT, class E>
-DM_DEV void wt_kloop(const E& e, const WtOp<T>& op, int bx, int by, int kt0, int nk, char* smem,
-                     floatx4 (&acc)[WT::RT][WT::CT]) {
+// The sums of one tile (column tile bx, row tile by) by one wave: every part of E's sum into acc[0], or
+// with PART only part `part` (its two chains of eighths apart in acc[0] and acc[1]); leaves the stages free.
+template <typename T, class WT, bool PART, class E>
+DM_DEV void wt_kloop(const E& e, const WtOp<T>& op, int bx, int by, int part, char* smem,
+                     floatx4 (&acc)[E::SUM == WT_EIGHTHS ? 2 : 1][WT::RT][WT::CT]) {
   using MF = Mfma<T>;
-  constexpr int NA = WT::NA, CT = WT::CT, RT = WT::RT, S = WT::S, L = WT::L;
+  constexpr int NA = WT::NA, CT = WT::CT, RT = WT::RT, S = WT::S, L = WT::L, SUM = E::SUM;
+  constexpr bool FLUSH = SUM != WT_CHAIN && !PART;   // chains added up on the way
+  constexpr int NC = SUM == WT_EIGHTHS ? 2 : 1;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int lr = lane >> 3, lc = (lane & 7) ^ lr;   // the lane's row of an 8-row load; its 16-byte chunk, swizzled
   const int m0 = by * WT::ROWS, K = op.K;
@@ -70,25 +107,34 @@ DM_DEV void wt_kloop(const E& e, const WtOp<T>& op, int bx, int by, int kt0, int
   for (int i = 0; i < 2 * CT; ++i) pw[i] = e.wrow(bx, WT{}, 8 * i + lr);
 #pragma unroll
   for (int i = 0; i < NA; ++i) pa[i] = op.A + (long)min(m0 + 8 * i + lr, op.M - 1) * op.lda;   // past M: row M - 1 again
-  auto issue = [&](int kt, int st) {
+  WtWalk<SUM, PART> wi(K, PART ? part : 0), wc = wi;   // of the loads issued, of the steps computed
+  auto issue = [&](int st) {
     char* b = smem + st * WT::STAGE;
-    const int k = min(64 * (kt0 + kt) + 8 * lc, K - 8);   // a half last step: chunks past K read K's last, unused
+    const int k = min(wi.k + 8 * lc, K - 8);   // a half last step: chunks past K read K's last, unused
 #pragma unroll
     for (int i = 0; i < 2 * CT; ++i)
       __builtin_amdgcn_global_load_lds((const void*)(pw[i] + k), (lds_void_t*)(b + i * 1024), 16, 0, 0);
 #pragma unroll
     for (int i = 0; i < NA; ++i)
       __builtin_amdgcn_global_load_lds((const void*)(pa[i] + k), (lds_void_t*)(b + (2 * CT + i) * 1024), 16, 0, 0);
+    wi.next();
   };
+  floatx4 chain[NC][RT][CT];   // without FLUSH: unused, the chains are acc
+  auto& run = [&]() -> auto& { if constexpr (FLUSH) return chain; else return acc; }();
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int c = 0; c < CT; ++c) acc[t][c] = zero4();
-  auto compute = [&](int kt, int st) {
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int q = 0; q < CT; ++q) {
+        acc[c][t][q] = zero4();
+        if constexpr (FLUSH) chain[c][t][q] = zero4();
+      }
+  auto compute = [&](int st) {
     const char* b = smem + st * WT::STAGE;
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
-      if (64 * (kt0 + kt) + 32 * hf >= K) break;   // uniform
+      if (wc.k + 32 * hf >= wc.end) break;   // uniform
       const int sw = ((4 * hf + g) ^ (r & 7)) << 4;
       typename MF::frag w[CT];
 #pragma unroll
@@ -99,25 +145,40 @@ DM_DEV void wt_kloop(const E& e, const WtOp<T>& op, int bx, int by, int kt0, int
         const int ar = 16 * t + ((NA & 1) && t == RT - 1 ? (r & 7) : r);
         const typename MF::frag a = *reinterpret_cast<const typename MF::frag*>(b + (WT::COLS + ar) * 128 + sw);
 #pragma unroll
-        for (int c = 0; c < CT; ++c) acc[t][c] = MF::mma(a, w[c], acc[t][c]);
+        for (int c = 0; c < CT; ++c) run[NC == 2 ? hf : 0][t][c] = MF::mma(a, w[c], run[NC == 2 ? hf : 0][t][c]);
       }
     }
+    if constexpr (FLUSH) {
+      if (wc.last()) {   // uniform
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+          for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int q = 0; q < CT; ++q) {
+              acc[0][t][q] += chain[c][t][q];
+              chain[c][t][q] = zero4();
+            }
+      }
+    }
+    wc.next();
   };
+  const int nk = wi.steps();
 #pragma unroll
   for (int s = 0; s < S; ++s)
-    if (s < nk) issue(s, s);
+    if (s < nk) issue(s);
   int kt = 0;
   for (; kt + S < nk; ++kt) {
     wait_vm_lgkm0<(S - 1) * L>();   // stage kt has landed
-    compute(kt, kt % S);
+    compute(kt % S);
     wait_vm_lgkm0<63>();            // its fragment reads are done: the stage is free
-    issue(kt + S, kt % S);
+    issue(kt % S);
   }
   static_steps(std::make_integer_sequence<int, S>{}, [&](auto ic) {
     constexpr int j = S - 1 - decltype(ic)::value;   // stages issued after this one
     if (j < nk - kt) {   // uniform
       wait_vm_lgkm0<j * L>();
-      compute(nk - 1 - j, (nk - 1 - j) % S);
+      compute((nk - 1 - j) % S);
     }
   });
   // every load has landed and one wave's LDS operations complete in order: the stages are free
@@ -139,10 +200,10 @@ template <typename T, class WT, class E>
 DM_DEV void wt_tile(const E& e, const WtOp<T>& op, int bx, int by, char* smem) {
   typename E::template Pre<WT> pre;
   e.prefetch(bx, by * WT::ROWS, pre);
-  floatx4 acc[WT::RT][WT::CT];
-  wt_kloop<T, WT>(e, op, bx, by, 0, (op.K + 63) / 64, smem, acc);
+  floatx4 acc[E::SUM == WT_EIGHTHS ? 2 : 1][WT::RT][WT::CT];
+  wt_kloop<T, WT, false>(e, op, bx, by, 0, smem, acc);
   float* tile = reinterpret_cast<float*>(smem);
-  wt_stage<WT>(acc, tile);
+  wt_stage<WT>(acc[0], tile);
   __syncthreads();
   e.apply(bx, by * WT::ROWS, tile, pre);
 }
@@ -161,20 +222,23 @@ static __global__ __launch_bounds__(64) void k_wt2(WtOp<T> op1, E1 e1, WtOp<T> o
   else wt_tile<T, WT>(e2, op2, b - op1.nx, blockIdx.y, smem);
 }
 
-// A long K in few tiles (an MLP's down product): KW waves per tile, each a quarter of the k steps with its
-// own ring, their partial tiles added in wave order. One wave alone keeps 24 KB in flight; 64 tiles
-// on 64 CUs then read K = 2752 at 34 KB/us each.
-template <typename T, class WT, int KW, class E>
-static __global__ __launch_bounds__(64 * KW) void k_wt_ksplit(WtOp<T> op, E e) {
-  __shared__ __attribute__((aligned(1024))) char smem[KW * WT::LDS];
-  const int wave = threadIdx.x >> 6, nk = (op.K + 63) / 64;
-  const int k0 = wave * nk / KW, k1 = (wave + 1) * nk / KW;
+// A product summed in parts by four waves per tile, each a part of E's sum with its own ring, their partial
+// tiles added in the sum's order: a tile's chain of k steps is a quarter as long, and four times the
+// bytes are in flight (launch_wt_parts, with what both measured).
+template <typename T, class WT, class E>
+static __global__ __launch_bounds__(64 * WT_PARTS) void k_wt_ksplit(WtOp<T> op, E e) {
+  static_assert(E::SUM != WT_CHAIN, "a sum of parts");
+  constexpr int NC = E::SUM == WT_EIGHTHS ? 2 : 1, TILE = 16 * WT::RT * WT::LDT;
+  static_assert(NC * TILE * 4 <= WT::LDS, "a wave's partial tiles fit its stages");
+  __shared__ __attribute__((aligned(1024))) char smem[WT_PARTS * WT::LDS];
+  const int wave = threadIdx.x >> 6;
   typename E::template Pre<WT> pre;
   e.prefetch(blockIdx.x, blockIdx.y * WT::ROWS, pre);
-  floatx4 acc[WT::RT][WT::CT];
+  floatx4 acc[NC][WT::RT][WT::CT];
   char* mine = smem + wave * WT::LDS;
-  wt_kloop<T, WT>(e, op, blockIdx.x, blockIdx.y, k0, k1 - k0, mine, acc);
-  wt_stage<WT>(acc, reinterpret_cast<float*>(mine));
+  wt_kloop<T, WT, true>(e, op, blockIdx.x, blockIdx.y, wave, mine, acc);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) wt_stage<WT>(acc[c], reinterpret_cast<float*>(mine) + c * TILE);
   __syncthreads();
   if (wave > 0) return;
   float* tile = reinterpret_cast<float*>(smem);
@@ -182,7 +246,8 @@ static __global__ __launch_bounds__(64 * KW) void k_wt_ksplit(WtOp<T> op, E e) {
   for (int i = threadIdx.x; i < NE; i += 64) {
     float v = tile[i];
 #pragma unroll
-    for (int w = 1; w < KW; ++w) v += reinterpret_cast<const float*>(smem + w * WT::LDS)[i];
+    for (int p = 1; p < WT_PARTS * NC; ++p)
+      v += reinterpret_cast<const float*>(smem + p / NC * WT::LDS)[p % NC * TILE + i];
     tile[i] = v;
   }
   __builtin_amdgcn_wave_barrier();   // one wave's LDS operations complete in order
@@ -191,7 +256,9 @@ static __global__ __launch_bounds__(64 * KW) void k_wt_ksplit(WtOp<T> op, E e) {
 
 // ---- epilogues ----------------------------------------------------------------------------------
 // out[M, N] = the product
-template <typename T> struct WtStore {
+template <typename T, int SUM_> struct WtStore {
+  static constexpr int SUM = SUM_;
+  static constexpr bool TALL = false;
   const T* W;
   long ldw;
   T* out;
@@ -221,6 +288,8 @@ template <typename T> struct WtStore {
 
 // act[M, H] = silu(x W1^T) (x W3^T): a tile's first half of columns from W1, the second the same from W3
 template <typename T> struct WtSwiGLU {
+  static constexpr int SUM = WT_QUARTERS;
+  static constexpr bool TALL = true;   // 64-row tiles too (with_wt)
   const T* W1;
   const T* W3;
   long ldw;
@@ -250,6 +319,8 @@ template <typename T> struct WtSwiGLU {
 
 // the projection (EpiProj without the value norm): q / k / v tiles hold 8 CT RoPE pairs of one head
 template <typename T, int DH, bool DEVPOS> struct WtProj {
+  static constexpr int SUM = WT_CHAIN;
+  static constexpr bool TALL = false;
   const T* W;   // [nseg d, d]
   EpiProj<T, DH, DEVPOS> e;
   template <class WT> struct Pre {
@@ -328,6 +399,8 @@ template <typename T, int DH, bool DEVPOS> struct WtProj {
 // same 4 CT columns of each of its four sections, a v_map / g_v tile 16 CT plain columns; an item is
 // V columns (of each section) of one row, V so that the wave's lanes are used.
 template <typename T, int DH, bool DEVPOS> struct WtSweep1 {
+  static constexpr int SUM = WT_CHAIN;
+  static constexpr bool TALL = false;
   typedef EpiSweep1<T, DH, 1, DEVPOS> Epi;
   const T* W;   // [4d, d], packed
   Epi e;
@@ -436,6 +509,8 @@ template <typename T, int DH, bool DEVPOS> struct WtSweep1 {
 
 // sweep GEMM 2 (EpiSweep2): items of V columns of one row
 template <typename T, int DH, bool DEVPOS> struct WtSweep2 {
+  static constexpr int SUM = WT_CHAIN;
+  static constexpr bool TALL = false;
   typedef EpiSweep2<T, DH, DEVPOS> Epi;
   const T* W;   // [d, d]
   Epi e;

@@ -131,6 +131,49 @@ def test_swiglu_rows_half_step(M, d, H):
     assert err < 4 * 2 ** -9, err
 
 
+# a row's MLP output is the same in every batch: the split of each product's sum follows from its sizes alone
+@pytest.mark.parametrize("d,H", [(128, 32), (512, 1376), (2048, 5504)])
+def test_swiglu_rows_equal_in_every_batch(d, H):
+    say(f"swiglu rows of 64 and of fewer, d={d} H={H}")
+    x, w1, w3, w2 = (_rand(*s, seed=i) for i, s in enumerate([(64, d), (H, d), (H, d), (d, H)]))
+    out = L.swiglu_rows(x, w1 * 0.05, w3 * 0.05, w2 * 0.05)
+    for n in (1, 8, 9, 16, 17, 32, 33, 63):
+        _same(L.swiglu_rows(x[:n].contiguous(), w1 * 0.05, w3 * 0.05, w2 * 0.05), out[:n], f"{n} rows")
+
+
+# W_O and the MLP's down product sum eight chains of 32-wide steps (step j in chain j mod 8), its up products
+# one chain per quarter of d: the rounding of these sums shows which. 2^24 swallows a 1 added to it.
+@pytest.mark.parametrize("M", [1, 9, 17, 33, 64])
+@pytest.mark.parametrize("K", [512, 1536])
+def test_row_product_sum_order(M, K):
+    say(f"order of the row products' sums, M={M} K={K}")
+    bf = dict(device=DEV, dtype=torch.bfloat16)
+    a, w = torch.zeros(K, **bf), torch.zeros(K, **bf)
+    a[0] = a[256] = w[0] = 2.0 ** 12
+    w[256] = -(2.0 ** 12)
+    a[32:256:32] = w[32:256:32] = 1.0                     # steps 1 .. 7
+    # W_O: a step without past rows returns its own value row, here x-hat itself
+    cfg = cfg_of(K, K // 64, "mult_res", 8)
+    sd = dict(_sd(cfg), **{"wv.weight": torch.eye(K, **bf), "wo.weight": w.expand(K, K).contiguous()})
+    cos, sin = (t.to(DEV) for t in build_rope_cache(8, 64, cfg.rope_theta))
+    y = StaticTape(cfg, M, 8, DEV, torch.bfloat16, sd=sd).step(a.expand(M, K).contiguous(), 0, cos, sin, with_wo=True)[1]
+    _same(y, torch.full_like(y, 7.0), "W_O")
+    # down: act = silu(64) * (a / 64)
+    d = 128
+    x, w1, w3 = torch.zeros(M, d, **bf), torch.zeros(K, d, **bf), torch.zeros(K, d, **bf)
+    x[:, 0], w1[:, 0], w3[:, 0] = 1.0, 64.0, a / 64
+    out = L.swiglu_rows(x, w1, w3, w.expand(d, K).contiguous())
+    _same(out, torch.full_like(out, 7.0), "down")
+    # up: 2^24 in the first quarter, 1 + 1 in the second, -2^24 in the third; the gate 64
+    q, H = K // 4, 128
+    x, w1, w3, w2 = (torch.zeros(*n, **bf) for n in ((M, K), (H, K), (H, K), (K, H)))
+    x[:, 0], x[:, q], x[:, q + 32], x[:, 2 * q], x[:, K - 1] = 2.0 ** 12, 1.0, 1.0, -(2.0 ** 12), 1.0
+    w3[:, 0], w3[:, q], w3[:, q + 32], w3[:, 2 * q], w1[:, K - 1] = 2.0 ** 12, 1.0, 1.0, 2.0 ** 12, 64.0
+    w2[:, 0] = 1.0
+    out = L.swiglu_rows(x, w1, w3, w2)
+    _same(out, torch.full_like(out, 128.0), "up")
+
+
 # dm_decode_step_norm against dm_decode_step and dm_residual_rmsnorm: the norm in GEMM 2's launch (bf16,
 # B <= 64, no per-head norm), and where it follows the step (linear: one refine GEMM; B = 65; v_norm; fp32)
 @pytest.mark.parametrize("dt,B,d,h,P0,kw", [

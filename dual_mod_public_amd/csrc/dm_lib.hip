@@ -343,23 +343,28 @@ DecWs carve_dec(const dm_config* c, int tape_T, void* base) {
   return w;
 }
 
-// The tape read: one launch where NS groups of a block cover it, else split
+// The tape read: one launch where a block's groups of threads cover it, else split
 // partials and their merge; the same results.
 template <typename T, int DH>
 void run_decode_read(DecodeArgs<T>& da, hipStream_t s) {
   const int BH = da.B * da.h;
-  // One launch while a (b, h)'s splits fit one block and the chip still holds the grid: with more
-  // than one split per (b, h) each block keeps its threads (256 or 512 per split) resident until the slowest is
-  // done, so from 512 (b, h) up the split grid balances better.
-  constexpr int NT = dec_threads<T, DH>(), NSMAX = 1024 / NT;
-  if (da.nsplit >= 1 && (da.nsplit == 1 || (da.nsplit <= NSMAX && BH <= 512))) {
-    if (da.nsplit == 1)
-      launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 1>, dim3(BH), dim3(NT), 0, s, da);
-    else if (da.nsplit == 2)
-      launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 2>, dim3(BH), dim3(2 * NT), 0, s, da);
-    else
-      launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, NSMAX>, dim3(BH), dim3(NSMAX * NT), 0, s, da);
+  // One launch for one split, and for two at head_dim 64 while B*h is at most 512 (with two, each block keeps
+  // its 512 threads resident until the slower is done: from 512 (b, h) up the split grid balances better).
+  // More groups do not fit the registers: a group holds its split's K rows (64 registers a lane in bf16,
+  // 128 or 256 in fp32) and their scores, a block of 1024 threads has 128 a lane, and two fp32 groups at
+  // head_dim 128 share 512. With what those spill a step took, against the split grid: bf16, head_dim 64,
+  // 1100 keys, B*h = 16 / 512: 47 / 116 us against 25 / 46; bf16, 128, 700 keys: 50 / 127 against 26 / 68; fp32,
+  // 128, 1100 keys: 299 / 1070 against 145 / 325.
+  constexpr int NT = dec_threads<T, DH>(), NSMAX = DH == 64 ? 2 : 1;
+  if (da.nsplit == 1) {
+    launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, 1>, dim3(BH), dim3(NT), 0, s, da);
     return;
+  }
+  if constexpr (NSMAX > 1) {
+    if (da.nsplit == NSMAX && BH <= 512) {
+      launch_k(PROF_DEC_READ, k_decode_direct<T, DH, DEC_SPLIT, NSMAX>, dim3(BH), dim3(NSMAX * NT), 0, s, da);
+      return;
+    }
   }
   if (da.nsplit > 0) {
     const int idx = prof_launch_begin(PROF_DEC_READ, true, da.prof_ts);

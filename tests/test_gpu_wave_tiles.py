@@ -97,20 +97,26 @@ def test_projection_rows_equal_larger_call(T, d, h):
         _same(ta[:, :, :T] if ta.dim() == 4 else ta[:, :T], tb, n)
 
 
-# splits of 512 keys: one, two and up to four in one launch; 40 batch rows (B*h > 512) take the split grid
-@pytest.mark.parametrize("P", [1, 511, 512, 513, 1024, 1025, 1600, 2048])
+# A step at a host position reads at most 512 keys (head_dim 64: 1024) in one launch, in a quarter of the passes
+# up to 128; at a device position the launch covers the whole tape, here five splits: the split grid. Keys at the
+# edges of the passes, the splits and the rule; with a window also where it cuts the first split.
+@pytest.mark.parametrize("P", [1, 127, 128, 129, 511, 512, 513, 640, 1024, 1025, 1600])
 @pytest.mark.parametrize("W", [0, 600])
-@pytest.mark.parametrize("d,h", [(1024, 16), (2048, 16)])
-def test_short_read_equals_split_read(P, W, d, h):
-    say(f"short read P={P} W={W} d={d} h={h}")
-    B, few, dh = 40, 3, d // h
-    m = DualModAttention(cfg_of(d, h, "mult_res", 2048, local_window=W)).to(DEV, torch.bfloat16)
-    q, ks, vs = (_rand(B, h, 1, dh, seed=s) for s in (1, 2, 3))
-    K, V = _rand(B, h, P, dh, seed=4), _rand(B, h, P, dh, seed=5)
-    with torch.no_grad():
-        a = m.attend_one(q, ks, vs, K, V)[0]
-        b = m.attend_one(q[:few], ks[:few], vs[:few], K[:few], V[:few])[0]
-    _same(a[:few], b, "o")
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("d,h", [(256, 4), (512, 4)])
+def test_short_read_equals_split_read(P, W, dt, d, h):
+    say(f"short read P={P} W={W} {dt} d={d} h={h}")
+    B, dh, T = 3, d // h, 2100
+    cfg = cfg_of(d, h, "mult_res", T, local_window=W)
+    sd = {k: v.to(DEV, dt) for k, v in make_state_dict(cfg, seed=5).items()}
+    cos, sin = (t.to(DEV) for t in build_rope_cache(T, dh, cfg.rope_theta))
+    tape = StaticTape(cfg, B, T, DEV, dt, sd=sd)
+    tape.K.copy_(_rand(B, h, T, dh, seed=1))
+    tape.V.copy_(_rand(B, h, T, dh, seed=2))
+    x = _rand(B, d, seed=3).to(dt)
+    host = tape.step(x, P, cos, sin)[0].clone()
+    dev = tape.step(x, torch.tensor([P], device=DEV, dtype=torch.int32), cos, sin)[0]
+    _same(host, dev, "o")
 
 
 # mlp widths whose last k step is a half one (H = 32 mod 64), rows at the tiles' edges

@@ -233,8 +233,15 @@ void run_proj_src(const dm_config* c, const dm_packed* w, const SA& sa, int M, i
                   int pos_cap = 0) {
   const int nseg = (c->ctx_mod == DM_CTX_LINEAR) ? 5 : 6;
   SrcRows<T> sb{(const T*)w->w_proj, c->d, nseg * c->d};
+  // Few rows, issued directly. Wave tiles while a wave's operands (M d of them) are few: with more, the waves
+  // of a block tile share what each of them would load; then 64-row blocks up to d = 2048, 128-row ones
+  // beyond. Measured at weights from HBM, head_dim 64, wave tiles / 64-row / 128-row blocks, us: d = 1024,
+  // M = 32 6.8 / 9.3 / -, 64 10.2 / 10.2 / 16.6, 96 15.7 / 10.1 / 18.5, 256 21.3 / 11.4 / 20.3 (256 x 256
+  // blocks 40); d = 2048, M = 32 15.7 / 16.6 / -, 48 25.9 / 17.0 / 24.9, 256 48.5 / 31.1 / 30.6; d = 4096,
+  // M = 8 42.4 / 46.6 / -, 16 49.8 / 44.4 / -, 96 104 / 65 / 55; d = 256, M = 256 5.1 / 4.8 / 13.0.
+  const bool few = sizeof(T) == 2 && M <= WT_MAX_M && launch_log() == nullptr;
   if constexpr (std::is_same<SA, SrcRows<bf16>>::value) {
-    if (wt_ok<T>(M, sa.p, w->w_proj) && v_gain(c, w) == nullptr) {
+    if (wt_ok<T>(M, sa.p, w->w_proj) && v_gain(c, w) == nullptr && (long)M * c->d <= 65536 && (M <= 8 || c->d <= 2048)) {
       const WtOp<T> op{sa.p, sa.ld, M, c->d};
       if (pos_dev != nullptr)
         launch_wt(op, nseg * c->d, WtProj<T, DH, true>{(const T*)w->w_proj,
@@ -267,13 +274,13 @@ void run_proj_src(const dm_config* c, const dm_packed* w, const SA& sa, int M, i
   // bf16, whole 256-row / 256-column tiles: 256 x 256 blocks (eight 64 x 128 wave tiles,
   // two direct-to-LDS stages); otherwise 128 x 128 with wave tiles spanning whole heads
   if constexpr (sizeof(T) == 2) {
-    if (!small_tiles && M % 256 == 0 && (nseg * c->d) % 256 == 0 && c->d % 64 == 0) {
+    if (!small_tiles && !few && M % 256 == 0 && (nseg * c->d) % 256 == 0 && c->d % 64 == 0) {
       launch_gemm<T, 256, 256, 4, 2, -2>(sa, sb, M, nseg * c->d, c->d, epi, s, PROF_PROJ);
       return;
     }
   }
-  if (M <= 64) {
-    // a decode step's few rows: 64-row blocks, one head wide (twice the blocks of 128 x 128)
+  if (M <= 64 || (few && c->d <= 2048)) {
+    // 64-row blocks, one head wide (twice the blocks of 128 x 128)
     if constexpr (DH == 64)
       launch_gemm_auto<T, 64, 64, 2, 2, 3, 4>(sa, sb, M, nseg * c->d, c->d, epi, s, PROF_PROJ);
     else

@@ -82,7 +82,7 @@ def test_refine_rows_equal_larger_call(n, mod, d, h):
 
 
 @pytest.mark.parametrize("T", [1, 8, 13, 16, 32, 40, 64, 100, 256])
-@pytest.mark.parametrize("d,h", [(256, 4), (1024, 8), (1024, 16)])
+@pytest.mark.parametrize("d,h", [(256, 4), (1024, 8), (1024, 16), (2048, 16), (2304, 36)])
 def test_projection_rows_equal_larger_call(T, d, h):
     say(f"projection rows T={T} d={d} h={h}")
     N = 512

@@ -369,12 +369,18 @@ template <typename T> bool refine_wt_ok(const dm_config* c, const dm_packed* w, 
   return wt_ok<T>(N, o, w->w_sweep) && kctx_gain(c, w) == nullptr && vctx_gain(c, w) == nullptr &&
          (c->ctx_mod == DM_CTX_LINEAR || (aligned16(vin) && aligned16(w->w_vctx)));
 }
-// Both GEMMs in wave tiles: up to 64 rows (one row of 64 x 64 blocks would use 4d / 64 CUs). With more
-// rows sweep GEMM 1's 64-wide block tiles are the faster ones: their epilogue touches each row of its
-// inputs in longer runs (M = 128 equal; 192: 16.8 against 11.0 us; 256: 15.8 against 13.1).
+// Both GEMMs in wave tiles, at most 64 rows. With more rows sweep GEMM 1's 64-wide block tiles are the faster
+// ones: their epilogue touches each row of its inputs in longer runs (d = 1024, M = 96: 11.0 against 10.3 us,
+// 192: 18.8 / 10.5).
 template <typename T> bool refine_few_rows(const dm_config* c, const dm_packed* w, int N, const T* o, const T* vin) {
   return N <= ROWS_MAX && refine_wt_ok<T>(c, w, N, o, vin);
 }
+
+// Without a W_O product riding along, sweep GEMM 1 pays in wave tiles while a wave's operands are few (as the
+// projection's): measured at weights from HBM, against 64 x 64 blocks, d = 1024, M = 64: 8.4 / 10.5 us; 2048,
+// 32: 12.6 / 15.9, 48: 17.0 / 16.2 (weights in cache 16.3 / 13.9); 3072, 16: 18.0 / 25.8, 48: 38.4 / 23.8;
+// 4096, 16: 33.3 / 35.8 (in cache 31.1 / 24.5)
+inline bool sweep1_wt_pays(int N, int d) { return (long)N * d <= 65536 && (N <= 8 || d <= 3072); }
 
 template <typename T, int DH>
 void run_refine(const dm_config* c, const dm_packed* w, const CellGeom& g, int N, const T* o, const float* ssq,
@@ -384,7 +390,8 @@ void run_refine(const dm_config* c, const dm_packed* w, const CellGeom& g, int N
                 bool wide = false, const AheadComm<T>* ahead = nullptr, const WtWo<T>* wo = nullptr) {
   if constexpr (sizeof(T) == 2) {
     // wo: only given where refine_few_rows holds
-    if (next_attend == nullptr && !wide && refine_few_rows<T>(c, w, N, o, vin)) {
+    if (next_attend == nullptr && !wide && refine_few_rows<T>(c, w, N, o, vin) &&
+        (wo != nullptr || sweep1_wt_pays(N, c->d))) {
       if (g.pos_dev != nullptr)
         run_refine_wt<T, DH, true>(c, w, g, N, o, ssq, kraw, vraw, glogx, sig, cos, sin, Kout, Vout, out_stride,
                                      out_row0, vin, gvu, save1, save2, s, wo);
@@ -424,10 +431,11 @@ void run_refine(const dm_config* c, const dm_packed* w, const CellGeom& g, int N
                                  Kout, Vout, out_stride, out_row0, vin, gvu, save1};
     launch_gemm_auto<T, 64, 64, 2, 2, SW1_STAGES, 4>(sa, sb, N, 4 * c->d, c->d, e1, s, PROF_SWEEP1);
   } else if (sizeof(T) == 2 && DM_SW1_EIGHT_WAVES && launch_log() == nullptr &&
-             cdiv(N, 64) * (4 * c->d / 128) >= 256) {
+             cdiv(N, 64) * (4 * c->d / 128) >= 192) {
     // bf16: 64 x 128 blocks of eight waves (each 256-thread half one 64-column group; d is a
-    // multiple of 128, so the direct-to-LDS k-loop always applies) where they give every CU one (fewer:
-    // 64 x 64 blocks, 12.2 against 13.1 us at 256 rows, d = 1024): the two column groups share
+    // multiple of 128, so the direct-to-LDS k-loop always applies) where they give most CUs one (fewer:
+    // 64 x 64 blocks. 128 blocks, d = 1024, 256 rows: 12.1 against 10.5 us; 192 blocks, d = 1024, 384
+    // rows: 12.2 / 12.3, d = 3072, 128 rows: 29.1 / 33.2): the two column groups share
     // the block's o rows, so a k-step moves 24 KB into a CU's LDS instead of the 32 KB of two
     // 64 x 64 blocks, still with eight waves per CU; the same per-element k order
     if constexpr (sizeof(T) == 2) {
@@ -472,12 +480,12 @@ void run_refine(const dm_config* c, const dm_packed* w, const CellGeom& g, int N
     launch_gemm_auto<T, 64, DH, 4, 1, S2, 4>(av, bv, N, c->d, c->d, e2, s, PROF_SWEEP2);
     return;
   }
-  // GEMM 2 in wave tiles where 64 x 32 blocks would not give every CU one: measured (with the sweep
-  // around it) at d = 1024 and 256 / 192 / 128 rows 6.4 / 6.0 / 4.7 us against 6.8 / 6.6 / 6.5, at d = 2048
-  // and 256 rows (256 blocks) 10.9 us in 64 x 32 blocks, 1.8 us more in wave tiles
+  // GEMM 2 in wave tiles while their operands are few; measured against 64 x 32 blocks: d = 1024, 192 rows
+  // 5.3 / 6.4 us, 256 6.5 / 6.4; d = 2048, 96 rows 8.1 / 10.0, 128 10.3 / 10.0; d = 3072, 64 rows 11.0 / 13.4, 96
+  // 19.0 / 13.6
   bool gemm2_done = false;
   if constexpr (sizeof(T) == 2) {
-    if (!linear && cdiv(N, 64) * (c->d / 32) < 256 && refine_wt_ok<T>(c, w, N, o, vin)) {
+    if (!linear && (long)N * c->d <= 196608 && refine_wt_ok<T>(c, w, N, o, vin)) {
       if (g.pos_dev != nullptr)
         launch_gemm2_wt<T, DH, true>(c, w, g, N, vraw, glogx, Vout, out_stride, out_row0, vin, gvu, save2, s);
       else

@@ -65,7 +65,8 @@ def test_exact_rows_equal_sweeps(B, T, mod, d, h, kw):
 
 # rows of the small call: edges of the 8-, 16- and 32-row tiles and of the wave-tile range
 @pytest.mark.parametrize("n", [1, 8, 9, 16, 17, 32, 33, 63, 64, 65, 130, 256])
-@pytest.mark.parametrize("mod,d,h", [("mult_res", 256, 4), ("linear", 1024, 16), ("fusion", 512, 4), ("mult", 1024, 8)])
+@pytest.mark.parametrize("mod,d,h", [("mult_res", 256, 4), ("linear", 1024, 16), ("fusion", 512, 4), ("mult", 1024, 8),
+                                     ("mult_res", 2048, 32)])
 def test_refine_rows_equal_larger_call(n, mod, d, h):
     say(f"refine rows n={n} {mod} d={d} h={h}")
     N = 320

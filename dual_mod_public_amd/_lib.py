@@ -159,6 +159,10 @@ SIGNATURES = {
     "dm_linear": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_vp]),
     "dm_embed_bwd": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_vp]),
     "dm_ce_rows": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_vp]),
+    "dm_ce_count": (ctypes.c_int, [c_vp, c_i32, c_vp, c_vp]),
+    "dm_ce_mean": (ctypes.c_int, [c_vp, c_i32, c_vp, c_vp, c_vp]),
+    "dm_rms_wgrad_workspace_bytes": (ctypes.c_size_t, [c_i32]),
+    "dm_rms_wgrad": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_vp, ctypes.c_size_t, c_vp]),
     "dm_argmax_rows": (ctypes.c_int, [c_i32, c_vp, c_i32, c_i32, ctypes.c_int64, c_vp, c_vp]),
     "dm_stack_fwd_plan_bytes": (ctypes.c_size_t, [P(dm_config), c_i32, P(dm_stack_layer), P(c_i32), c_i32, c_i32]),
     "dm_stack_fwd": (ctypes.c_int, [P(dm_config), c_i32, P(dm_stack_layer), c_fp, c_fp, P(c_i32), c_i32, c_i32,
@@ -320,17 +324,46 @@ def embed_bwd(dx, idx, g):
     check(lib().dm_embed_bwd(dtype_code(dx.dtype), ptr(dx), ptr(idx), ptr(g), M, d, g.shape[0], stream_ptr()))
 
 
-def ce_rows(logits, target, nvalid):
-    """dm_ce_rows on contiguous device tensors: the rows' cross entropies (fp32 [M], 0 for targets < 0);
-    logits [M, V] becomes the gradient of their sum / nvalid (a one-element fp32 tensor)."""
+def ce_rows(logits, target, nvalid, loss=None):
+    """dm_ce_rows on contiguous device tensors: the rows' cross entropies (fp32 [M], 0 for targets < 0; into
+    loss where given); logits [M, V] becomes the gradient of their sum / nvalid (a one-element fp32 tensor)."""
     M, V = logits.shape
     assert logits.is_contiguous() and target.is_contiguous()
     assert target.dtype == torch.int64 and target.numel() == M
     assert nvalid.dtype == torch.float32 and nvalid.numel() == 1
-    loss = torch.empty(M, device=logits.device, dtype=torch.float32)
+    if loss is None:
+        loss = torch.empty(M, device=logits.device, dtype=torch.float32)
+    assert loss.is_contiguous() and loss.dtype == torch.float32 and loss.numel() == M
     check(lib().dm_ce_rows(dtype_code(logits.dtype), ptr(logits), ptr(target), ptr(nvalid), ptr(loss), M, V,
                            stream_ptr()))
     return loss
+
+
+def ce_count(target, nvalid):
+    """dm_ce_count: nvalid (one fp32) = max(number of targets >= 0, 1); target int64, contiguous."""
+    assert target.is_contiguous() and target.dtype == torch.int64
+    assert nvalid.dtype == torch.float32 and nvalid.numel() == 1
+    check(lib().dm_ce_count(ptr(target), target.numel(), ptr(nvalid), stream_ptr()))
+    return nvalid
+
+
+def ce_mean(loss, nvalid, out):
+    """dm_ce_mean: out (one fp32) = loss.sum() / nvalid; loss fp32, contiguous."""
+    assert loss.is_contiguous() and loss.dtype == nvalid.dtype == out.dtype == torch.float32
+    assert nvalid.numel() == 1 and out.numel() == 1
+    check(lib().dm_ce_mean(ptr(loss), loss.numel(), ptr(nvalid), ptr(out), stream_ptr()))
+    return out
+
+
+def rms_wgrad(dy, x, r, dw):
+    """dm_rms_wgrad: dw (fp32 [d]) += (dy * x * r).sum(0) for dy, x [M, d] of one dtype, r fp32 [M, 1]."""
+    M, d = x.shape
+    assert dy.shape == x.shape and dy.dtype == x.dtype and dy.is_contiguous() and x.is_contiguous()
+    assert r.dtype == dw.dtype == torch.float32 and r.is_contiguous() and r.numel() == M
+    assert dw.is_contiguous() and dw.numel() == d
+    ws = torch.empty(lib().dm_rms_wgrad_workspace_bytes(d), device=x.device, dtype=torch.uint8)
+    check(lib().dm_rms_wgrad(dtype_code(x.dtype), ptr(dy), ptr(x), ptr(r), ptr(dw), M, d, ptr(ws), ws.numel(),
+                             stream_ptr()))
 
 
 MLP_ROWS = 64   # rows dm_swiglu_rows takes per call

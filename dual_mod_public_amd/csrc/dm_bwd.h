@@ -1643,6 +1643,28 @@ static __global__ __launch_bounds__(256) void k_colsum_partial(int M, int ncols,
   part[(long)blockIdx.y * ncols + col] = s;
 }
 
+// part[chunk, col] = sum over the chunk's rows of dy x r (an RMSNorm weight's gradient), as k_colsum_partial
+template <typename T>
+static __global__ __launch_bounds__(256) void k_rms_wgrad_partial(int M, int ncols, int rows_per_chunk, const T* __restrict__ dy,
+                                                                 const T* __restrict__ x, const float* __restrict__ r,
+                                                                 float* __restrict__ part) {
+  const int col = blockIdx.x * 256 + threadIdx.x;
+  if (col >= ncols) return;
+  const int r0 = blockIdx.y * rows_per_chunk, r1 = min(r0 + rows_per_chunk, M);
+  float s = 0.f;
+  for (int m0 = r0; m0 < r1; m0 += 8) {   // eight rows' loads in flight at a time
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const long m = min(m0 + k, r1 - 1);
+      v[k] = to_f(dy[m * ncols + col]) * to_f(x[m * ncols + col]) * r[m];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += (m0 + k < r1) ? v[k] : 0.f;
+  }
+  part[(long)blockIdx.y * ncols + col] = s;
+}
+
 // out[col] += sum_chunk part[chunk * ld + col], col < ncols
 // C[i] (+)= sum_z part[z * n + i], z = 0..S-1 in order (split-K slices)
 static __global__ __launch_bounds__(256) void k_sum_splits(int S, long n, const float* __restrict__ part,

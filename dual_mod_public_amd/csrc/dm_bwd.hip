@@ -1219,6 +1219,29 @@ int dm_mlp_fwd(int32_t dtype, const dm_mlp_packed* w, const void* y, void* z, co
   return DM_OK;
 }
 
+size_t dm_rms_wgrad_workspace_bytes(int32_t d) { return d > 0 ? (size_t)NCHUNK * d * 4 : 0; }
+
+int dm_rms_wgrad(int32_t dtype, const void* dy, const void* x, const float* r, float* dw, int32_t M, int32_t d,
+                 void* workspace, size_t workspace_bytes, void* stream) {
+  DM_REQUIRE(dy && x && r && dw, DM_ERR_INVALID, "null operand");
+  DM_REQUIRE(M > 0 && d > 0, DM_ERR_INVALID, "M=%d d=%d", M, d);
+  DM_REQUIRE(dtype == DM_BF16 || dtype == DM_F32, DM_ERR_INVALID, "dtype %d", dtype);
+  DM_REQUIRE(workspace && workspace_bytes >= dm_rms_wgrad_workspace_bytes(d), DM_ERR_WORKSPACE, "workspace %zu < %zu bytes",
+             workspace_bytes, dm_rms_wgrad_workspace_bytes(d));
+  hipStream_t s = S(stream);
+  const dim3 grid(cdiv(d, 256), NCHUNK);
+  const int rpc = cdiv(M, NCHUNK);
+  float* part = (float*)workspace;
+  if (dtype == DM_BF16)
+    hipLaunchKernelGGL(k_rms_wgrad_partial<bf16>, grid, dim3(256), 0, s, M, d, rpc, (const bf16*)dy, (const bf16*)x, r, part);
+  else
+    hipLaunchKernelGGL(k_rms_wgrad_partial<float>, grid, dim3(256), 0, s, M, d, rpc, (const float*)dy, (const float*)x, r, part);
+  hipLaunchKernelGGL(k_sum_rows_add, dim3(cdiv(d, 64)), dim3(256), 0, s, NCHUNK, d, d, part, dw, (float*)nullptr,
+                     (float*)nullptr, d);
+  DM_HIP(hipGetLastError());
+  return DM_OK;
+}
+
 size_t dm_mlp_workspace_bytes(int32_t dtype, int32_t M, int32_t d, int32_t H) {
   if ((dtype != DM_F32 && dtype != DM_BF16) || M <= 0 || d <= 0 || H <= 0 || d % 128 || H % 128) return 0;
   return carve_mlp(M, d, H, nullptr).bytes;

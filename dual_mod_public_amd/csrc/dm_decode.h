@@ -502,6 +502,37 @@ __global__ __launch_bounds__(256) void k_ce_rows(T* x, const int64_t* target, co
   }
 }
 
+// The sums around k_ce_rows by one block each, in a fixed order and without state to clear: the library's sums
+// split such a column over blocks and clear their counters by a memset, which a captured step would hold as
+// a node. 16384 tokens: 8 us each (the library's passes 24 and 15).
+// nvalid = max(number of targets >= 0, 1)
+static __global__ __launch_bounds__(1024) void k_ce_count(const int64_t* target, int M, float* nvalid) {
+  __shared__ int red[16];
+  int c = 0;
+#pragma unroll 8
+  for (int m = threadIdx.x; m < M; m += 1024) c += target[m] >= 0;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) c += __shfl_xor(c, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x > 0) return;
+  for (int w = 1; w < 16; ++w) c += red[w];
+  *nvalid = (float)max(c, 1);
+}
+// out = (sum of x[0 .. M)) / nvalid
+static __global__ __launch_bounds__(1024) void k_ce_mean(const float* x, int M, const float* nvalid, float* out) {
+  __shared__ float red[16];
+  float v = 0.f;
+#pragma unroll 8
+  for (int m = threadIdx.x; m < M; m += 1024) v += x[m];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x > 0) return;
+  for (int w = 1; w < 16; ++w) v += red[w];
+  *out = v / *nvalid;
+}
+
 // k_argmax_rows for 16-byte aligned rows (ld a multiple of the vector width): 1024 threads per row,
 // 16-byte loads. A lane visits its columns in increasing order (its vectors, then the tail columns,
 // which come last in the row), so a strict > keeps its first maximum; lanes and waves then merge

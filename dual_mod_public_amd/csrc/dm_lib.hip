@@ -800,6 +800,22 @@ int dm_ce_rows(int32_t dtype, void* logits, const int64_t* target, const float* 
   return DM_OK;
 }
 
+int dm_ce_count(const int64_t* target, int32_t M, float* nvalid, void* stream) {
+  DM_REQUIRE(target && nvalid, DM_ERR_INVALID, "null operand");
+  DM_REQUIRE(M > 0, DM_ERR_INVALID, "M=%d", M);
+  hipLaunchKernelGGL(k_ce_count, dim3(1), dim3(1024), 0, S(stream), target, M, nvalid);
+  DM_HIP(hipGetLastError());
+  return DM_OK;
+}
+
+int dm_ce_mean(const float* loss, int32_t M, const float* nvalid, float* out, void* stream) {
+  DM_REQUIRE(loss && nvalid && out, DM_ERR_INVALID, "null operand");
+  DM_REQUIRE(M > 0, DM_ERR_INVALID, "M=%d", M);
+  hipLaunchKernelGGL(k_ce_mean, dim3(1), dim3(1024), 0, S(stream), loss, M, nvalid, out);
+  DM_HIP(hipGetLastError());
+  return DM_OK;
+}
+
 int dm_argmax_rows(int32_t dtype, const void* x, int32_t rows, int32_t cols, int64_t ld, int64_t* out,
                    void* stream) {
   DM_REQUIRE(x && out, DM_ERR_INVALID, "null operand");

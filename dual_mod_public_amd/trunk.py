@@ -51,7 +51,7 @@ def _rms_vjp(dy, x, r, w, dw):
     """VJP of y = x r w with r = rsqrt(mean x^2 + eps): returns dx (fp32) and adds sum_rows dy x r
     into dw (fp32)."""
     xf, g = x.float(), dy.float()
-    dw.add_((g * xf * r).sum(0))
+    L.rms_wgrad(dy, x, r, dw)
     gw = g * w.float()
     return r * gw - xf * (r * r * r) * (gw * xf).mean(-1, keepdim=True)
 
@@ -316,26 +316,29 @@ class HipTrunk:
     def _head(self):
         """norm_f, the tied head and the mean cross entropy (ignore_index -1, model.py:279-281), with
         its gradient: the loss's softmax gradient needs nothing but the logits, so the head's VJP runs
-        with its forward, chunk by chunk of rows (the reference's loss_chunk, graphs.py:322-341)."""
+        with its forward, chunk by chunk of rows (the reference's loss_chunk, graphs.py:322-341). The sums
+        over rows are the library's own (libdm_hip.so): torch's
+        split a long column over blocks and clear their counters with memsets, which a captured step
+        would hold as nodes."""
         m = self.m
         M, d = self.B * self.T, self.cfg.d_model
         x = self.xs[-1].view(M, d)
         tg = self.targets.view(M)
-        nvalid = (tg >= 0).sum().clamp_min(1).float()
+        nvalid = L.ce_count(tg, torch.empty((), device=self.dev, dtype=torch.float32))
         gw = self.grad["tok_emb.weight"]
         gnf = self.grad["norm_f.weight"]
-        loss = torch.zeros((), device=self.dev, dtype=torch.float32)
+        loss = torch.empty(M, device=self.dev, dtype=torch.float32)
         dxl = self.dxs[-1].view(M, d)
         for r0 in range(0, M, self.loss_chunk):
             r1 = min(r0 + self.loss_chunk, M)
             xc, t = x[r0:r1], tg[r0:r1]
             hf, r = _rms(xc, m.norm_f.weight, m.norm_f.eps)
             dl = hf @ self.w_emb.t()
-            loss = loss + L.ce_rows(dl, t, nvalid).sum()   # dl: the logits, then their gradient
+            L.ce_rows(dl, t, nvalid, loss[r0:r1])   # dl: the logits, then their gradient
             gw.add_(_mm32(dl.t(), hf))
             dhf = dl @ self.w_emb
             dxl[r0:r1].copy_(_rms_vjp(dhf, xc, r, m.norm_f.weight, gnf))
-        self.loss.copy_(loss / nvalid)
+        L.ce_mean(loss, nvalid, self.loss)
 
     def _embed_bwd(self):
         M, d = self.B * self.T, self.cfg.d_model
@@ -386,7 +389,8 @@ class HipTrunk:
         return self
 
     def train_step(self, idx, targets):
-        """Forward + backward of the batch (idx, targets [B, T] token ids; targets -1 are ignored).
+        """Forward + backward of the batch (idx, targets [B, T] token ids; targets -1 are ignored, one >=
+        vocab_size makes the loss NaN; an id outside the table is left out of the embedding gradient).
         Returns the loss (a static device scalar, overwritten by the next step); the gradients are
         the views ``grad[name]`` of the flat buffer ``flat`` (``to_param_grads`` copies them into
         the parameters' .grad)."""

@@ -509,6 +509,19 @@ int dm_embed_bwd(int32_t dtype, const void* dx, const int64_t* idx, float* g, in
 int dm_ce_rows(int32_t dtype, void* logits, const int64_t* target, const float* nvalid, float* loss, int32_t rows,
                int32_t cols, void* stream);
 
+/* nvalid (one fp32) = max(number of targets >= 0, 1); out (one fp32) = the sum of the M loss rows / nvalid: the
+ * sums around dm_ce_rows, one block each in a fixed order, nothing to clear (they may be captured). */
+int dm_ce_count(const int64_t* target, int32_t M, float* nvalid, void* stream);
+int dm_ce_mean(const float* loss, int32_t M, const float* nvalid, float* out, void* stream);
+
+/* ---- RMSNorm weight gradient -----------------------------------------------------------
+ * dw [d] fp32 += sum over the M rows of dy x r (dy, x [M, d] storage dtype, r [M] fp32 the rows' scales
+ * rsqrt(mean x^2 + eps)): attention.py:74-83's weight, summed in a fixed order over 64 chunks of rows.
+ * Nothing to clear. */
+size_t dm_rms_wgrad_workspace_bytes(int32_t d);
+int dm_rms_wgrad(int32_t dtype, const void* dy, const void* x, const float* r, float* dw, int32_t M, int32_t d,
+                 void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- row argmax ------------------------------------------------------------------
  * out[r] = the first index of the maximum of x[r, 0:cols) (row stride ld elements),
  * storage dtype bf16 or fp32: the greedy pick of lm/eval/graph_decode.py:62

@@ -57,6 +57,64 @@ def _model(cfg, dtype, seed=7):
     return m, sd
 
 
+def _memsets(run):
+    """The memset nodes of the graph that ``run`` records; the graph is not replayed."""
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so")
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        run()
+    raw, n = ctypes.c_void_p(g.raw_cuda_graph()), ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0 and n.value > 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    kinds = []
+    for node in nodes:
+        k = ctypes.c_int()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(k)) == 0
+        kinds.append(k.value)
+    return kinds.count(2)   # hipGraphNodeTypeMemset
+
+
+@pytest.mark.parametrize("wavefront", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_captured_step_records_no_memset(dtype, wavefront):
+    """A recorded memset has not taken effect on later replays, so a step records none, also at token counts
+    where a library's sum over all of them clears counters (the first line: such a sum is seen)."""
+    say(f"nodes of a captured 16384-token step, {dtype} wavefront={wavefront}")
+    x = torch.zeros(1 << 22, device=DEV)
+    assert _memsets(lambda: x.sum()) > 0
+    cfg = _cfg(n_layers=1, max_seq_len=1024)
+    m, _ = _model(cfg, dtype)
+    tr = HipTrunk(m, 16, 1024, schedule=uniform_chunks(1024, 64, 1), wavefront=wavefront)
+    idx, tg = (t.to(DEV) for t in _batch(cfg, 16, 1024))
+    tr.train_step(idx, tg)
+    torch.cuda.synchronize()
+    assert _memsets(tr._run) == 0
+
+
+# sums of one block's rows and of many, columns at the edge of a block; the gradient is added
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,d", [(1, 64), (65, 300), (4097, 256)])
+def test_head_sums(M, d, dtype):
+    say(f"head sums M={M} d={d} {dtype}")
+    g = torch.Generator(device=DEV).manual_seed(M)
+    dy, x = (torch.randn(M, d, generator=g, device=DEV).to(dtype) for _ in range(2))
+    r, dw = torch.rand(M, 1, generator=g, device=DEV) + 0.5, torch.randn(d, generator=g, device=DEV)
+    t = torch.randint(-1, 3, (M,), generator=g, device=DEV)
+    prod = dy.double().cpu() * x.double().cpu() * r.double().cpu()
+    ref, mag = dw.double().cpu() + prod.sum(0), dw.double().cpu().abs() + prod.abs().sum(0)
+    L.rms_wgrad(dy, x, r, dw)
+    nv = L.ce_count(t, torch.empty((), device=DEV))
+    mean = L.ce_mean(r.view(M), nv, torch.empty((), device=DEV))
+    torch.cuda.synchronize()
+    # each product rounded twice, chains of M / 64 rows, of 16 chunks and 4 more
+    assert ((dw.double().cpu() - ref).abs() <= (M / 64 + 24) * 2 ** -24 * mag).all()
+    assert nv.item() == max((t >= 0).sum().item(), 1)
+    want = r.double().sum().item() / nv.item()
+    assert abs(mean.item() - want) <= (M / 1024 + 24) * 2 ** -24 * want   # chains of M / 1024 rows, 6 + 16 more
+
+
 def _batch(cfg, B, T, seed=3):
     g = torch.Generator().manual_seed(seed)
     idx = torch.randint(0, cfg.vocab_size, (B, T), generator=g)

@@ -108,9 +108,9 @@ DM_DEV void wt_kloop(const E& e, const WtOp<T>& op, int bx, int by, int part, ch
 #pragma unroll
   for (int i = 0; i < NA; ++i) pa[i] = op.A + (long)min(m0 + 8 * i + lr, op.M - 1) * op.lda;   // past M: row M - 1 again
   WtWalk<SUM, PART> wi(K, PART ? part : 0), wc = wi;   // of the loads issued, of the steps computed
-  auto issue = [&](int st) {
+  auto issue = [&](int kt, int st) {
     char* b = smem + st * WT::STAGE;
-    const int k = min(wi.k + 8 * lc, K - 8);   // a half last step: chunks past K read K's last, unused
+    const int k = min((SUM == WT_CHAIN ? 64 * kt : wi.k) + 8 * lc, K - 8);   // a half last step: chunks past K read K's last, unused
 #pragma unroll
     for (int i = 0; i < 2 * CT; ++i)
       __builtin_amdgcn_global_load_lds((const void*)(pw[i] + k), (lds_void_t*)(b + i * 1024), 16, 0, 0);
@@ -130,11 +130,12 @@ DM_DEV void wt_kloop(const E& e, const WtOp<T>& op, int bx, int by, int part, ch
         acc[c][t][q] = zero4();
         if constexpr (FLUSH) chain[c][t][q] = zero4();
       }
-  auto compute = [&](int st) {
+  auto compute = [&](int kt, int st) {
     const char* b = smem + st * WT::STAGE;
+    const int kc = SUM == WT_CHAIN ? 64 * kt : wc.k, kend = SUM == WT_CHAIN ? K : wc.end;
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
-      if (wc.k + 32 * hf >= wc.end) break;   // uniform
+      if (kc + 32 * hf >= kend) break;   // uniform
       const int sw = ((4 * hf + g) ^ (r & 7)) << 4;
       typename MF::frag w[CT];
 #pragma unroll
@@ -166,19 +167,19 @@ DM_DEV void wt_kloop(const E& e, const WtOp<T>& op, int bx, int by, int part, ch
   const int nk = wi.steps();
 #pragma unroll
   for (int s = 0; s < S; ++s)
-    if (s < nk) issue(s);
+    if (s < nk) issue(s, s);
   int kt = 0;
   for (; kt + S < nk; ++kt) {
     wait_vm_lgkm0<(S - 1) * L>();   // stage kt has landed
-    compute(kt % S);
+    compute(kt, kt % S);
     wait_vm_lgkm0<63>();            // its fragment reads are done: the stage is free
-    issue(kt % S);
+    issue(kt + S, kt % S);
   }
   static_steps(std::make_integer_sequence<int, S>{}, [&](auto ic) {
     constexpr int j = S - 1 - decltype(ic)::value;   // stages issued after this one
     if (j < nk - kt) {   // uniform
       wait_vm_lgkm0<j * L>();
-      compute((nk - 1 - j) % S);
+      compute(nk - 1 - j, (nk - 1 - j) % S);
     }
   });
   // every load has landed and one wave's LDS operations complete in order: the stages are free

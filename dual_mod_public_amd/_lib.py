@@ -158,6 +158,8 @@ SIGNATURES = {
                                     c_vp, ctypes.c_size_t, c_vp]),
     "dm_linear": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_vp]),
     "dm_embed_bwd": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_vp]),
+    "dm_embed_bwd_workspace_bytes": (ctypes.c_size_t, [c_i32, c_i32, c_i32]),
+    "dm_embed_bwd_lists": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_vp, ctypes.c_size_t, c_vp]),
     "dm_ce_rows": (ctypes.c_int, [c_i32, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_vp]),
     "dm_ce_count": (ctypes.c_int, [c_vp, c_i32, c_vp, c_vp]),
     "dm_ce_mean": (ctypes.c_int, [c_vp, c_i32, c_vp, c_vp, c_vp]),
@@ -317,11 +319,18 @@ def residual_rmsnorm(x, delta=None, w=None, dtype=torch.bfloat16, y=None, eps=1e
 
 
 def embed_bwd(dx, idx, g):
-    """dm_embed_bwd on contiguous device tensors: g[idx[m]] += dx[m] (g fp32 [n, d], idx int64 [M], dx [M, d])."""
+    """dm_embed_bwd / dm_embed_bwd_lists on contiguous device tensors: g[idx[m]] += dx[m] (g fp32 [n, d], idx
+    int64 [M], dx [M, d]); ids outside [0, n) are left out."""
     M, d = dx.shape
     assert dx.is_contiguous() and idx.is_contiguous() and g.is_contiguous()
     assert idx.dtype == torch.int64 and idx.numel() == M and g.dtype == torch.float32 and g.shape[1] == d
-    check(lib().dm_embed_bwd(dtype_code(dx.dtype), ptr(dx), ptr(idx), ptr(g), M, d, g.shape[0], stream_ptr()))
+    args = (dtype_code(dx.dtype), ptr(dx), ptr(idx), ptr(g), M, d, g.shape[0])
+    nb = lib().dm_embed_bwd_workspace_bytes(M, d, g.shape[0])
+    if nb == 0:
+        check(lib().dm_embed_bwd(*args, stream_ptr()))
+        return
+    ws = torch.empty(nb, device=dx.device, dtype=torch.uint8)
+    check(lib().dm_embed_bwd_lists(*args, ptr(ws), nb, stream_ptr()))
 
 
 def ce_rows(logits, target, nvalid, loss=None):

@@ -379,23 +379,89 @@ __global__ __launch_bounds__(256) void k_residual_rmsnorm_reg(float* x, const T*
   residual_rmsnorm_row<T, NPT>(blockIdx.x, x, delta, w, y, d, eps, red);
 }
 
-// Embedding backward: g[idx[m]] += sum of the rows dx[m'] with idx[m'] = idx[m], in ascending order (fp32),
-// by the block of the id's first token; the blocks of its later tokens find it and end. No sort and nothing
-// to clear, so it may be captured. Each block reads the ids (32 KB at 4096 tokens, from L2). Bound by
-// reading dx and updating the touched rows of g; above some 10000 tokens by the ids (M^2 of them read). A
-// frequent id's rows are one block's chain, so eight rows are in flight, which the unconditional loads
-// (column d - 1 again past d) let the compiler hoist over the sums: 4096 x 1024 bf16, half of the ids one
-// padding id, 2022 -> 171 us (distinct ids 18 -> 19 us). d in passes of 256 * EMB_COLS columns: 8 a thread
-// would keep 2048 columns in one pass (16384 distinct rows: 198 us against 281) but hold too many loads
-// for eight rows. An id outside [0, n) is left out.
-constexpr int EMB_COLS = 4;
-template <typename T>
+// ---- embedding backward --------------------------------------------------------------------------
+// g[idx[m]] += the sum of the rows dx[m'] with idx[m'] = idx[m], in ascending order in fp32, added up by
+// chains of EMB_CHAIN rows (a frequent id's error is that of two short chains, not of one over thousands of
+// rows). No sort and nothing cleared by a memset node, so it may be captured. An id outside [0, n) is left out.
+constexpr int EMB_CHAIN = 64;   // rows per chain
+constexpr int EMB_VEC = 4;      // columns per thread and pass of 256 threads
+
+// acc[e] += the chained sum of the rows rows[0 .. count) (ascending; LDS) at the thread's columns of the pass
+// from c0. VEC: four adjacent columns by vector loads (d a multiple of 4, aligned rows), else every 256th.
+// Eight rows in flight: the loads are unconditional (the last column again past d), so that they are hoisted
+// over the sums (16 rows took more registers, fewer blocks: 4096 distinct rows 26 us against 20).
+template <typename T, bool VEC>
+DM_DEV void emb_sum_rows(const T* dx, const int* rows, int count, int d, int c0, float (&acc)[EMB_VEC]) {
+  const int cv = min(c0 + EMB_VEC * (int)threadIdx.x, d - EMB_VEC);
+  for (int q0 = 0; q0 < count; q0 += EMB_CHAIN) {
+    const int q1 = min(q0 + EMB_CHAIN, count);
+    float ch[EMB_VEC];
+#pragma unroll
+    for (int e = 0; e < EMB_VEC; ++e) ch[e] = 0.f;
+#pragma unroll 8
+    for (int q = q0; q < q1; ++q) {
+      const T* row = dx + (long)rows[q] * d;
+      if constexpr (VEC) {
+        float v[EMB_VEC];
+        unpackv<T, EMB_VEC>(*reinterpret_cast<const typename RawV<T, EMB_VEC>::type*>(row + cv), v);
+#pragma unroll
+        for (int e = 0; e < EMB_VEC; ++e) ch[e] += v[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < EMB_VEC; ++e) ch[e] += to_f(row[min(c0 + (int)threadIdx.x + 256 * e, d - 1)]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < EMB_VEC; ++e) acc[e] += ch[e];
+  }
+}
+// dst[columns] (+)= acc
+template <bool VEC, bool ADD>
+DM_DEV void emb_store(float* dst, int d, int c0, const float (&acc)[EMB_VEC]) {
+  if constexpr (VEC) {
+    const int c = c0 + EMB_VEC * threadIdx.x;
+    if (c >= d) return;
+    floatx4* p = reinterpret_cast<floatx4*>(dst + c);
+    const floatx4 v = {acc[0], acc[1], acc[2], acc[3]};
+    *p = ADD ? *p + v : v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < EMB_VEC; ++e) {
+      const int c = c0 + threadIdx.x + 256 * e;
+      if (c < d) dst[c] = ADD ? dst[c] + acc[e] : acc[e];
+    }
+  }
+}
+// The tokens of ids[j0, j0 + 256) with this id, ascending, into hits; returns their number (block-wide)
+template <typename I> DM_DEV int emb_hits(const I* ids, int j0, int M, I id, int* hits, int* wcount) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = j0 + threadIdx.x;
+  const bool hit = j < M && ids[j] == id;
+  const unsigned long long mask = __ballot(hit);
+  if (lane == 0) wcount[wave] = __popcll(mask);
+  __syncthreads();
+  int base = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (w < wave) base += wcount[w];
+    total += wcount[w];
+  }
+  if (hit) hits[base + __popcll(mask & ((1ull << lane) - 1))] = j;
+  __syncthreads();
+  return total;
+}
+
+// Few tokens (EMB_ONE): one launch, the block of an id's first token sums its rows; the blocks of its later
+// tokens find that one and end. Every block reads the ids (M^2 of them, from L2), and one block sums a frequent
+// id's rows. bf16, us, distinct ids / half of them one padding id: 2048 x 1024 9.7 / 63 (lists: 22 / 56), 4096
+// 16 / 158 (24 / 77), 6144 30 / 236 (28 / 95).
+constexpr int EMB_ONE = 4096;
+template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void k_embed_bwd(const T* dx, const int64_t* idx, float* g, int M, int d, int n) {
   __shared__ int hits[256];
   __shared__ int wcount[4];
   __shared__ int seen;
-  const int m = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long id = idx[m];
+  const int m = blockIdx.x;
+  const int64_t id = idx[m];
   if (id < 0 || id >= n) return;   // uniform
   if (threadIdx.x == 0) seen = 0;
   __syncthreads();
@@ -404,40 +470,146 @@ __global__ __launch_bounds__(256) void k_embed_bwd(const T* dx, const int64_t* i
   if (any) seen = 1;
   __syncthreads();
   if (seen) return;   // uniform
-  float* gr = g + id * (long)d;
-  for (int c0 = 0; c0 < d; c0 += 256 * EMB_COLS) {
-    float acc[EMB_COLS];
-#pragma unroll
-    for (int e = 0; e < EMB_COLS; ++e) acc[e] = 0.f;
+  for (int c0 = 0; c0 < d; c0 += 256 * EMB_VEC) {
+    float acc[EMB_VEC] = {0.f, 0.f, 0.f, 0.f};
     for (int j0 = m; j0 < M; j0 += 256) {
-      // the block's 256 tokens with this id, in order
-      const int j = j0 + threadIdx.x;
-      const bool hit = j < M && idx[j] == id;
-      const unsigned long long mask = __ballot(hit);
-      if (lane == 0) wcount[wave] = __popcll(mask);
-      __syncthreads();
-      int base = 0, total = 0;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        if (w < wave) base += wcount[w];
-        total += wcount[w];
-      }
-      if (hit) hits[base + __popcll(mask & ((1ull << lane) - 1))] = j;
-      __syncthreads();
-#pragma unroll 8
-      for (int q = 0; q < total; ++q) {
-        const T* row = dx + (long)hits[q] * d;
-#pragma unroll
-        for (int e = 0; e < EMB_COLS; ++e) acc[e] += to_f(row[min(c0 + (int)threadIdx.x + 256 * e, d - 1)]);
-      }
+      const int total = emb_hits<int64_t>(idx, j0, M, id, hits, wcount);
+      emb_sum_rows<T, VEC>(dx, hits, total, d, c0, acc);
       __syncthreads();
     }
-#pragma unroll
-    for (int e = 0; e < EMB_COLS; ++e) {
-      const int c = c0 + threadIdx.x + 256 * e;
-      if (c < d) gr[c] += acc[e];
-    }
+    emb_store<VEC, true>(g + id * (long)d, d, c0, acc);
   }
+}
+
+// Many tokens: the ids' row lists are found once. An id of at most EMB_LIST tokens gets a list (filled in any
+// order, sorted by the block that sums it); a more frequent one is summed in pieces of `plen` tokens by the
+// blocks of its first token in each, the pieces added up in order by a last launch. Bound by reading dx and
+// updating g; a frequent id by its pieces' chains. bf16, us, against the library's sort and sums with their add
+// into g: 16384 x 1024 distinct 42 / 268, half one padding id 174 / 442; 16384 x 2048 Zipf 80 / 451; 65536 x
+// 1024 Zipf 151 / 615.
+constexpr int EMB_LIST = 256, EMB_PASS = 1024, EMB_PIECES = 64, EMB_NONE = 0x7fffffff;
+struct EmbWs {
+  int* cnt;     // [n] tokens of an id
+  int* start;   // [n] its list, or -1 - its number among the frequent ids
+  int* slot;    // [M] a token's place among its id's tokens
+  int* list;    // [M]
+  int* fid;     // [frequent] the id
+  int* first;   // [frequent, pieces] its first token in the piece, EMB_NONE without
+  int* cursor;  // list entries and frequent ids handed out
+  float* part;  // [frequent, pieces, d]
+  int pieces, plen, frequent;
+  size_t bytes;
+};
+static __global__ __launch_bounds__(256) void k_emb_clear(EmbWs w, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) w.cnt[i] = 0;
+  if (i < w.frequent * w.pieces) w.first[i] = EMB_NONE;
+  if (i < 2) w.cursor[i] = 0;
+}
+// one atomic per wave and id: a wave of one padding id would queue 64 at one address
+static __global__ __launch_bounds__(256) void k_emb_count(EmbWs w, const int64_t* idx, int M, int n) {
+  const int m = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+  const int64_t id64 = m < M ? idx[m] : -1;
+  const bool ok = id64 >= 0 && id64 < n;
+  const int id = ok ? (int)id64 : -1;
+  unsigned long long left = __ballot(ok), mine = 0;
+  while (left != 0) {   // uniform
+    const int lead = __ffsll((long long)left) - 1;
+    const unsigned long long same = __ballot(id == __shfl(id, lead, 64)) & left;
+    if ((same >> lane) & 1) mine = same;
+    left &= ~same;
+  }
+  const int lead = ok ? __ffsll((long long)mine) - 1 : lane;
+  int base = 0;
+  if (ok && lead == lane) base = atomicAdd(w.cnt + id, (int)__popcll(mine));
+  base = __shfl(base, lead, 64);
+  if (ok) w.slot[m] = base + (int)__popcll(mine & ((1ull << lane) - 1));
+}
+static __global__ __launch_bounds__(256) void k_emb_start(EmbWs w, const int64_t* idx, int M, int n) {
+  const int m = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+  const int64_t id = m < M ? idx[m] : -1;
+  const bool own = id >= 0 && id < n && w.slot[m] == 0;
+  const int c = own ? w.cnt[id] : 0;
+  const int need = c > 1 && c <= EMB_LIST ? c : 0;
+  int sum = need;   // inclusive over the wave
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(sum, o, 64);
+    if (lane >= o) sum += v;
+  }
+  const int total = __shfl(sum, 63, 64);
+  int base = 0;
+  if (lane == 0 && total > 0) base = atomicAdd(w.cursor, total);
+  base = __shfl(base, 0, 64);
+  if (need > 0) w.start[id] = base + sum - need;
+  if (c > EMB_LIST) {
+    const int f = atomicAdd(w.cursor + 1, 1);
+    w.fid[f] = (int)id;
+    w.start[id] = -1 - f;
+  }
+}
+static __global__ __launch_bounds__(256) void k_emb_place(EmbWs w, const int64_t* idx, int M, int n) {
+  const int m = blockIdx.x * 256 + threadIdx.x;
+  if (m >= M) return;
+  const int64_t id = idx[m];
+  if (id < 0 || id >= n) return;
+  const int c = w.cnt[id];
+  if (c > EMB_LIST) atomicMin(w.first + (-1 - w.start[id]) * w.pieces + m / w.plen, m);
+  else if (c > 1) w.list[w.start[id] + w.slot[m]] = m;
+}
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void k_emb_sum(EmbWs w, const T* dx, const int64_t* idx, float* g, int M, int d, int n) {
+  __shared__ int raw[EMB_LIST], rows[EMB_PASS];
+  __shared__ int wcount[4];
+  const int m = blockIdx.x;
+  const int64_t id = idx[m];
+  if (id < 0 || id >= n) return;   // uniform, as every branch below
+  const int c = w.cnt[id];
+  if (c > EMB_LIST) {
+    const int p = m / w.plen, slot = (-1 - w.start[id]) * w.pieces + p;
+    if (w.first[slot] != m) return;
+    const int j1 = min((p + 1) * w.plen, M);
+    for (int c0 = 0; c0 < d; c0 += 256 * EMB_VEC) {
+      float acc[EMB_VEC] = {0.f, 0.f, 0.f, 0.f};
+      for (int j0 = m; j0 < j1; j0 += EMB_PASS) {
+        int count = 0;
+        for (int j = j0; j < min(j0 + EMB_PASS, j1); j += 256)
+          count += emb_hits<int64_t>(idx, j, j1, id, rows + count, wcount);
+        emb_sum_rows<T, VEC>(dx, rows, count, d, c0, acc);
+        __syncthreads();
+      }
+      emb_store<VEC, false>(w.part + (long)slot * d, d, c0, acc);
+    }
+    return;
+  }
+  if (c == 1) {
+    if (threadIdx.x == 0) rows[0] = m;
+    __syncthreads();
+  } else {
+    static_assert(EMB_LIST == 256, "an entry per thread");
+    const int e = (int)threadIdx.x < c ? w.list[w.start[id] + threadIdx.x] : EMB_NONE;
+    raw[threadIdx.x] = e;
+    __syncthreads();
+    int rank = 0;
+    for (int i = 0; i < c; ++i) rank += raw[i] < e;
+    if ((int)threadIdx.x < c) rows[rank] = e;
+    __syncthreads();
+    if (rows[0] != m) return;
+  }
+  for (int c0 = 0; c0 < d; c0 += 256 * EMB_VEC) {
+    float acc[EMB_VEC] = {0.f, 0.f, 0.f, 0.f};
+    emb_sum_rows<T, VEC>(dx, rows, c, d, c0, acc);
+    emb_store<VEC, true>(g + id * (long)d, d, c0, acc);
+  }
+}
+// block (f, x): the pieces of frequent id f in order, columns [256 x, 256 (x + 1))
+static __global__ __launch_bounds__(256) void k_emb_pieces(EmbWs w, float* g, int d) {
+  const int f = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
+  if (f >= w.cursor[1] || c >= d) return;
+  float acc = 0.f;
+  for (int p = 0; p < w.pieces; ++p)
+    if (w.first[f * w.pieces + p] != EMB_NONE) acc += w.part[((long)f * w.pieces + p) * d + c];
+  g[w.fid[f] * (long)d + c] += acc;
 }
 
 // Cross entropy of one row of logits per block, with its gradient in place: loss[row] = lse - x[t] and

@@ -374,6 +374,58 @@ void run_decode_read(DecodeArgs<T>& da, hipStream_t s) {
   launch_k(PROF_DEC_MERGE, k_decode_merge<T, DH>, dim3(BH), dim3(64), 0, s, da);
 }
 
+EmbWs carve_emb(int M, int d, int n, void* base) {
+  EmbWs w{};
+  Carver cv(base);
+  w.pieces = std::min(EMB_PIECES, cdiv(M, EMB_PASS));
+  w.plen = cdiv(cdiv(M, w.pieces), EMB_PASS) * EMB_PASS;
+  w.pieces = cdiv(M, w.plen);
+  w.frequent = M / (EMB_LIST + 1);
+  w.cnt = cv.take<int>((size_t)n * 4);
+  w.start = cv.take<int>((size_t)n * 4);
+  w.slot = cv.take<int>((size_t)M * 4);
+  w.list = cv.take<int>((size_t)M * 4);
+  w.fid = cv.take<int>((size_t)w.frequent * 4);
+  w.first = cv.take<int>((size_t)w.frequent * w.pieces * 4);
+  w.cursor = cv.take<int>(8);
+  w.part = cv.take<float>((size_t)w.frequent * w.pieces * d * 4);
+  w.bytes = cv.off;
+  return w;
+}
+
+// w nullptr: in one launch
+template <typename T, bool VEC>
+void run_embed_bwd(const T* dx, const int64_t* idx, float* g, int M, int d, int n, const EmbWs* w, hipStream_t s) {
+  if (w == nullptr) {
+    hipLaunchKernelGGL((k_embed_bwd<T, VEC>), dim3(M), dim3(256), 0, s, dx, idx, g, M, d, n);
+    return;
+  }
+  const int nb = cdiv(M, 256);
+  hipLaunchKernelGGL(k_emb_clear, dim3(cdiv(std::max({n, w->frequent * w->pieces, 2}), 256)), dim3(256), 0, s, *w, n);
+  hipLaunchKernelGGL(k_emb_count, dim3(nb), dim3(256), 0, s, *w, idx, M, n);
+  hipLaunchKernelGGL(k_emb_start, dim3(nb), dim3(256), 0, s, *w, idx, M, n);
+  hipLaunchKernelGGL(k_emb_place, dim3(nb), dim3(256), 0, s, *w, idx, M, n);
+  hipLaunchKernelGGL((k_emb_sum<T, VEC>), dim3(M), dim3(256), 0, s, *w, dx, idx, g, M, d, n);
+  if (w->frequent > 0) hipLaunchKernelGGL(k_emb_pieces, dim3(w->frequent, cdiv(d, 256)), dim3(256), 0, s, *w, g, d);
+}
+int embed_bwd(int dtype, const void* dx, const int64_t* idx, float* g, int M, int d, int n, const EmbWs* w, void* stream) {
+  DM_REQUIRE(dx && idx && g, DM_ERR_INVALID, "null operand");
+  DM_REQUIRE(M > 0 && d > 0 && n > 0, DM_ERR_INVALID, "M=%d d=%d n=%d", M, d, n);
+  DM_REQUIRE(dtype == DM_BF16 || dtype == DM_F32, DM_ERR_INVALID, "dtype %d", dtype);
+  hipStream_t s = S(stream);
+  auto run = [&](auto tag) {
+    using T = decltype(tag);
+    // four columns at a time: whole vectors in every row
+    const bool vec = d % EMB_VEC == 0 && aligned16(g) && reinterpret_cast<uintptr_t>(dx) % (EMB_VEC * sizeof(T)) == 0;
+    if (vec) run_embed_bwd<T, true>((const T*)dx, idx, g, M, d, n, w, s);
+    else run_embed_bwd<T, false>((const T*)dx, idx, g, M, d, n, w, s);
+  };
+  if (dtype == DM_BF16) run(bf16{});
+  else run(float{});
+  DM_HIP(hipGetLastError());
+  return DM_OK;
+}
+
 // the residual norm after a step (dm_decode_step_norm); x nullptr: none
 struct StepNorm {
   float* x = nullptr;
@@ -770,14 +822,20 @@ int dm_residual_rmsnorm(int32_t dtype, float* x, const void* delta, const float*
 
 int dm_embed_bwd(int32_t dtype, const void* dx, const int64_t* idx, float* g, int32_t M, int32_t d, int32_t n,
                  void* stream) {
-  DM_REQUIRE(dx && idx && g, DM_ERR_INVALID, "null operand");
+  return embed_bwd(dtype, dx, idx, g, M, d, n, nullptr, stream);
+}
+
+size_t dm_embed_bwd_workspace_bytes(int32_t M, int32_t d, int32_t n) {
+  return M > EMB_ONE && d > 0 && n > 0 ? carve_emb(M, d, n, nullptr).bytes : 0;
+}
+
+int dm_embed_bwd_lists(int32_t dtype, const void* dx, const int64_t* idx, float* g, int32_t M, int32_t d, int32_t n,
+                       void* workspace, size_t workspace_bytes, void* stream) {
   DM_REQUIRE(M > 0 && d > 0 && n > 0, DM_ERR_INVALID, "M=%d d=%d n=%d", M, d, n);
-  DM_REQUIRE(dtype == DM_BF16 || dtype == DM_F32, DM_ERR_INVALID, "dtype %d", dtype);
-  hipStream_t s = S(stream);
-  if (dtype == DM_BF16) hipLaunchKernelGGL(k_embed_bwd<bf16>, dim3(M), dim3(256), 0, s, (const bf16*)dx, idx, g, M, d, n);
-  else hipLaunchKernelGGL(k_embed_bwd<float>, dim3(M), dim3(256), 0, s, (const float*)dx, idx, g, M, d, n);
-  DM_HIP(hipGetLastError());
-  return DM_OK;
+  const EmbWs w = carve_emb(M, d, n, workspace);
+  DM_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= w.bytes, DM_ERR_WORKSPACE, "workspace %zu < %zu bytes",
+             workspace_bytes, w.bytes);
+  return embed_bwd(dtype, dx, idx, g, M, d, n, &w, stream);
 }
 
 int dm_ce_rows(int32_t dtype, void* logits, const int64_t* target, const float* nvalid, float* loss, int32_t rows,

@@ -497,9 +497,16 @@ int dm_swiglu_rows(int32_t dtype, const void* x, const void* w1, const void* w3,
 
 /* ---- embedding backward ----------------------------------------------------------------
  * g [n, d] fp32: g[idx[m]] += dx[m] for the M rows of dx [M, d] (storage dtype bf16 or fp32), the rows of
- * an id summed in ascending order in fp32 (graphs.py:503). No library sort, nothing to clear. */
+ * an id summed in ascending order in fp32, in chains of 64 (graphs.py:503). No library sort, no memset. An
+ * id outside [0, n) is left out. dm_embed_bwd: one launch, each row's block reads the ids.
+ * dm_embed_bwd_lists: the ids' rows found once, a frequent id's summed by several blocks; for more rows,
+ * where dm_embed_bwd_workspace_bytes is not 0. */
 int dm_embed_bwd(int32_t dtype, const void* dx, const int64_t* idx, float* g, int32_t M, int32_t d, int32_t n,
                  void* stream);
+
+size_t dm_embed_bwd_workspace_bytes(int32_t M, int32_t d, int32_t n);
+int dm_embed_bwd_lists(int32_t dtype, const void* dx, const int64_t* idx, float* g, int32_t M, int32_t d, int32_t n,
+                       void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- cross entropy of logit rows, with its gradient -----------------------------------
  * logits [rows, cols] (contiguous, storage dtype bf16 or fp32), target [rows] int64 (< 0: ignored),

@@ -132,7 +132,7 @@ DM_DEV void store_kv(const KVRegs<T, DH, NT>& r, T* Ks, T* Vs) {
 
 // One 64-key tile: S = Q K^T * scale, mask, online softmax update, O += P V.
 // mask(q, key) -> true if the score is kept; q is the wave-relative row + 16*wave.
-template <typename T, int DH, class MASK>
+template <typename T, int DH, bool SHUFFLE = false, class MASK>
 DM_DEV void flash_tile(const typename Mfma<T>::frag* qf, const T* Ks, const T* Vs, T* Pw,
                        float scale, const MASK& keep, FlashState<T, DH>& st) {
   using C = AttnCfg<T, DH>;
@@ -161,7 +161,7 @@ DM_DEV void flash_tile(const typename Mfma<T>::frag* qf, const T* Ks, const T* V
       S[t][r] = s;
       mx = fmaxf(mx, s);
     }
-    mx = group16_max(mx);
+    mx = group16_max<SHUFFLE>(mx);
     const float mnew = fmaxf(st.m[r], mx);
     const float alpha = (st.m[r] == NEG_INF) ? 0.f : __expf(st.m[r] - mnew);
     st.m[r] = mnew;

@@ -354,9 +354,28 @@ DM_DEV float wave_sum(float v) {
   return xor_sum<1>(xor_sum<2>(xor_sum<4>(xor_sum<8>(xor_sum<16>(xor_sum<32>(v))))));
 }
 DM_DEV float wave_max(float v) { return lanes_max<1, 32>(v); }
-// reduce across the 16 lanes that share lane>>4 (xor over the low 4 bits)
-DM_DEV float group16_max(float v) { return lanes_max<1, 8>(v); }
-DM_DEV float group16_sum(float v) { return xor_sum<1>(xor_sum<2>(xor_sum<4>(xor_sum<8>(v)))); }
+// reduce across the 16 lanes that share lane>>4 (xor over the low 4 bits). SHUFFLE: through the LDS crossbar,
+// for kernels whose registers are full (regs_full): the DPP moves' partners are live registers, more of which
+// then go through scratch. The same values.
+template <typename T, int DH> constexpr bool regs_full() { return sizeof(T) == 4 && DH == 128; }
+template <bool SHUFFLE = false> DM_DEV float group16_max(float v) {
+  if constexpr (SHUFFLE) {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    return v;
+  } else {
+    return lanes_max<1, 8>(v);
+  }
+}
+template <bool SHUFFLE = false> DM_DEV float group16_sum(float v) {
+  if constexpr (SHUFFLE) {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+  } else {
+    return xor_sum<1>(xor_sum<2>(xor_sum<4>(xor_sum<8>(v))));
+  }
+}
 
 // ---- MFMA traits -------------------------------------------------------------
 // 16x16 output tile; lane l holds D[4*(l>>4) + r][l & 15], r = 0..3.

@@ -756,7 +756,7 @@ DM_DEV void attend_rows(const AttendArgs<T>& a, int bh, int q0, T* lds) {
       if constexpr (!PREV_EARLY) load_kv<T, DH, 64 * NW>(a.Kc + pb, a.Vc + pb, DH, g.pos0 - a.prev_lo, pk);
       store_kv<T, DH, 64 * NW>(pk, Ks, Vs);
       __syncthreads();
-      flash_tile<T, DH>(qf, Ks, Vs, Ps + wave * 16 * C::LDP, a.scale,
+      flash_tile<T, DH, regs_full<T, DH>()>(qf, Ks, Vs, Ps + wave * 16 * C::LDP, a.scale,
                         KeyWindow{g.pos0 - a.prev_lo, a.prev_lo, lo0 == NO_WINDOW_LO ? lo0 : lo0 + q0}, st);
       __syncthreads();   // Ks / Vs are free for the intra rows
       store_merged = true;
@@ -766,7 +766,7 @@ DM_DEV void attend_rows(const AttendArgs<T>& a, int bh, int q0, T* lds) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int q = wq + 4 * g4 + r;
-      const float zt = group16_sum(st.z[r]);
+      const float zt = group16_sum<regs_full<T, DH>()>(st.z[r]);
       if (q < g.c) {
         const long o = (long)bh * g.c + q;
 #pragma unroll
@@ -798,12 +798,12 @@ DM_DEV void attend_rows(const AttendArgs<T>& a, int bh, int q0, T* lds) {
   if constexpr (V_STAGED) store_k<T, DH, 64 * NW>(kv, Ks);
   else store_kv<T, DH, 64 * NW>(kv, Ks, Vs);
   __syncthreads();
-  flash_tile<T, DH>(qf, Ks, Vs, Ps + wave * 16 * C::LDP, a.scale, KeyStrictLower{q0, intra_wlim(g.window)}, st);
+  flash_tile<T, DH, regs_full<T, DH>()>(qf, Ks, Vs, Ps + wave * 16 * C::LDP, a.scale, KeyStrictLower{q0, intra_wlim(g.window)}, st);
 
   // raw self column: s_self = scale * <q_r, k_self_r> (fp32), value v_raw
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const float ss = group16_sum(sdot[r]) * a.scale;
+    const float ss = group16_sum<regs_full<T, DH>()>(sdot[r]) * a.scale;
     const float mnew = fmaxf(st.m[r], ss);
     const float alpha = (st.m[r] == NEG_INF) ? 0.f : __expf(st.m[r] - mnew);
     const float es = __expf(ss - mnew);
@@ -815,7 +815,7 @@ DM_DEV void attend_rows(const AttendArgs<T>& a, int bh, int q0, T* lds) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int q = wq + 4 * g4 + r;
-    const float zt = group16_sum(st.z[r]);
+    const float zt = group16_sum<regs_full<T, DH>()>(st.z[r]);
     const float inv = 1.0f / zt;
     float sq = 0.f;
     float ov[C::NDT];
@@ -824,7 +824,7 @@ DM_DEV void attend_rows(const AttendArgs<T>& a, int bh, int q0, T* lds) {
       ov[dt] = to_f(from_f<T>(st.O[dt][r] * inv));   // the stored (rounded) value
       sq += ov[dt] * ov[dt];
     }
-    sq = group16_sum(sq);
+    sq = group16_sum<regs_full<T, DH>()>(sq);
     if (q < g.c) {
       const long n = (long)b * g.c + q;
       T* orow = a.o + n * g.d + hh * DH;

@@ -160,7 +160,8 @@ void gemm_tn(const T* A, long lda, const T* Bm, long ldb, float* C, int M, int N
   // the register ring (2-byte LDS stores of both operands), 70 + 25 us so.
   if constexpr (sizeof(T) == 2) {
     const int Kt = K / 64 * 64;
-    if (Kt > 0 && Kt < K && M % 128 == 0 && N % 128 == 0) {
+    // (rows of any alignment are taken: the direct loads want 16-byte rows, the register ring does not)
+    if (Kt > 0 && Kt < K && M % 128 == 0 && N % 128 == 0 && aligned16(A) && aligned16(Bm) && lda % 8 == 0 && ldb % 8 == 0) {
       gemm_tn<T>(A, lda, Bm, ldb, C, M, N, Kt, accumulate, part, s);
       SrcKMajor<T> sa{A + (long)Kt * lda, lda, M}, sb{Bm + (long)Kt * ldb, ldb, N};
       sa.kmax = sb.kmax = K - Kt;

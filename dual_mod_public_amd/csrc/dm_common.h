@@ -141,6 +141,12 @@ template <typename V, typename P> DM_DEV V ld_global(const P* p) {
   return *(const __attribute__((address_space(1))) V*)(p);
 }
 
+// the same where p is known to be aligned to A bytes only (global loads need no more than 4; the type says so)
+template <typename V, int A, typename P> DM_DEV V ld_global_a(const P* p) {
+  typedef V VA __attribute__((aligned(A < (int)sizeof(V) ? A : (int)sizeof(V))));
+  return *(const __attribute__((address_space(1))) VA*)(p);
+}
+
 // 4 consecutive storage elements as one load / store: 8 bytes of bf16, 16 of fp32
 template <typename T> struct Raw4 { typedef u32x4 type; };
 template <> struct Raw4<bf16> { typedef u32x2 type; };

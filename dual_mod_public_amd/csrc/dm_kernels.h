@@ -1151,7 +1151,8 @@ template <typename T, int DH, int NG = 1, bool DEVPOS = false, bool SPLIT = fals
     typedef typename RawV<T, V>::type R;
     int m, b, p, t;
     row_of(row, m, b, p, t);
-    return MPre<V>{ld_global<R>(sig + ((long)b * g.Tbuf + t) * g.d + col), ld_global<R>(o + (long)m * g.d + col),
+    // sig is the caller's: aligned to four elements, whatever V
+    return MPre<V>{ld_global_a<R, 4 * sizeof(T)>(sig + ((long)b * g.Tbuf + t) * g.d + col), ld_global<R>(o + (long)m * g.d + col),
                    ld_global<R>(normw + col)};
   }
   template <int V> DM_DEV void m_settle(const MPre<V>& pr) const { settle_item(pr.sg); settle_item(pr.ov); settle_item(pr.nw); }

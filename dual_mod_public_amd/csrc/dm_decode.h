@@ -661,7 +661,15 @@ __global__ __launch_bounds__(256) void k_ce_rows(T* x, const int64_t* target, co
   float Z = 0.f;
 #pragma unroll
   for (int w = 0; w < 4; ++w) Z += red[4 + w] * expf(red[w] - M);
-  const float lse = M == __builtin_inff() ? M : M + logf(Z);
+  float lse = M + logf(Z);
+  if (M == __builtin_inff()) {   // uniform: Z is NaN (inf - inf) whether or not the row holds one
+    int bad = 0;
+    for (int i = threadIdx.x; i < n; i += 256) {
+      const float v = to_f(xr[i]);
+      bad |= v != v;
+    }
+    lse = __syncthreads_or(bad) ? __builtin_nanf("") : M;
+  }
   if (threadIdx.x == 0) loss[blockIdx.x] = valid ? lse - xt : 0.f;
   const float sc = valid ? 1.f / *nvalid : 0.f;
 #pragma unroll 4

@@ -273,6 +273,28 @@ def test_ce_rows(dt, M, V):
     assert (d <= leaf.grad.abs() * (rnd + tol + 2 ** -18) + 2 ** -22 / nv.item()).all(), d.max()
 
 
+# infinities, NaN and both in a row: the loss and the gradient that torch gives
+@pytest.mark.parametrize("V", [5, 2048, 2049])
+def test_ce_rows_not_finite(V):
+    say(f"cross entropy rows that are not finite, V={V}")
+    inf, nan = float("inf"), float("nan")
+    x = _rand(6, V, seed=1).float()
+    x[0, 1], x[1, 1], x[2, 1] = inf, nan, -inf
+    x[3, 1], x[3, V - 1] = inf, nan
+    x[4, 1], x[4, 0] = nan, inf
+    x[5] = -inf
+    t = torch.full((6,), 2, device=DEV)
+    leaf = x.double().cpu().requires_grad_(True)
+    lse = torch.logsumexp(leaf, -1)
+    ref = lse - leaf[:, 2]
+    p = torch.exp(leaf - lse[:, None]).detach()
+    p[:, 2] -= 1
+    loss = L.ce_rows(x, t, torch.ones((), device=DEV))
+    torch.cuda.synchronize()
+    torch.testing.assert_close(loss.double().cpu(), ref.detach(), rtol=1e-5, atol=1e-5, equal_nan=True)
+    torch.testing.assert_close(x.double().cpu(), p, rtol=1e-4, atol=1e-6, equal_nan=True)
+
+
 # Embedding backward: repeated ids across the block's 256-token passes, one id for all, d beyond one pass and no
 # multiple of the vector; above 4096 tokens by lists: ids of 1 to 256 tokens, frequent ones in pieces of 1024 and
 # (70000 tokens) of 2048. Equal rows that no fp32 sum holds show how deep the sums are: one chain over the 4096

@@ -125,20 +125,22 @@ template <typename T> bool wt_ok(int M, const void* A, const void* W) {
 }
 // f(WTile) with the tile of least expected time for M x N outputs (N a multiple of 64): a wave's
 // own time goes with its operand rows (8 NA + 16 CT; 57 ns each per 1024 of k), a CU's with the sum
-// over its waves (35 ns per row); fitted to 30 measured (M, N, tile) times, K = 512 .. 2048, M = 1 ..
-// 256, all within 15% of the best tile. tall: also 64 rows x 32 columns, which read the weights once
-// where shorter tiles read them twice (a tie goes to it: M = 33, N = 11008, K = 2048 17.0 us against
-// 18.5 and 21.8; N = 21888, K = 4096 55.4 against 63.9).
-template <class F> void with_wt(int M, int N, const F& f, bool tall = false) {
+// over its waves (35 ns per row); fitted to 30 measured (M, N, tile) times, K = 512 .. 2048, within 15% of
+// the best tile where the products take wave tiles. Of the first TILES forms, the ones a product's sizes can
+// reach: GEMM 2 (M N <= 262144) three, the projection and GEMM 1 alone (M d <= 65536) four, a store or GEMM 1
+// with W_O five; the MLP's up products all: 64 rows x 32 columns read the weights once where shorter tiles
+// read them twice (a tie goes to it: M = 33, N = 11008, K = 2048 17.0 us against 18.5 and 21.8; N = 21888, K =
+// 4096 55.4 against 63.9). 32 rows x 16 columns is never the least: 16 x 32 has as many rows and no more waves.
+template <int TILES, class F> void with_wt(int M, int N, const F& f) {
   struct C { int na, ct; };
-  constexpr C cand[] = {{1, 1}, {2, 1}, {2, 2}, {4, 1}, {4, 2}, {4, 4}, {8, 2}};
+  constexpr C cand[] = {{1, 1}, {2, 1}, {2, 2}, {4, 2}, {4, 4}, {8, 2}};
   int best = 0;
   long bt = -1;
-  for (int i = 0; i < (tall ? 7 : 6); ++i) {
+  for (int i = 0; i < TILES; ++i) {
     if (i > 0 && M <= 8 * cand[i - 1].na && cand[i].na > cand[i - 1].na) continue;
     const long rows = 8 * cand[i].na + 16 * cand[i].ct, waves = (long)cdiv(M, 8 * cand[i].na) * (N / (16 * cand[i].ct));
     const long t = std::max<long>(57 * rows, 35 * rows * cdiv(waves, 256));
-    if (bt < 0 || t < bt || (i == 6 && t == bt)) {
+    if (bt < 0 || t < bt || (i == 5 && t == bt)) {
       bt = t;
       best = i;
     }
@@ -147,22 +149,25 @@ template <class F> void with_wt(int M, int N, const F& f, bool tall = false) {
     case 0: f(WTile<1, 1>{}); break;
     case 1: f(WTile<2, 1>{}); break;
     case 2: f(WTile<2, 2>{}); break;
-    case 3: f(WTile<4, 1>{}); break;
-    case 4: f(WTile<4, 2>{}); break;
-    case 5: f(WTile<4, 4>{}); break;
-    default: f(WTile<8, 2>{}); break;
+    case 3:
+      if constexpr (TILES > 3) f(WTile<4, 2>{});
+      break;
+    case 4:
+      if constexpr (TILES > 4) f(WTile<4, 4>{});
+      break;
+    default:
+      if constexpr (TILES > 5) f(WTile<8, 2>{});
+      break;
   }
 }
 // N weight rows (WtSwiGLU: both matrices')
 template <typename T, class E>
 void launch_wt(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls = PROF_NONE) {
-  with_wt(op.M, N, [&](auto wt) {
+  with_wt<E::TILES>(op.M, N, [&](auto wt) {
     using WT = decltype(wt);
-    if constexpr (WT::NA <= 4 || E::TALL) {
-      op.nx = N / WT::COLS;
-      launch_k(prof_cls, k_wt<T, WT, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64), 0, s, op, e);
-    }
-  }, E::TALL);
+    op.nx = N / WT::COLS;
+    launch_k(prof_cls, k_wt<T, WT, E>, dim3(op.nx, cdiv(op.M, WT::ROWS)), dim3(64), 0, s, op, e);
+  });
 }
 // a product summed in parts (a step's W_O and MLP products, M <= ROWS_MAX): four waves per 16-column tile
 // while that gives the CUs at most two such blocks each, of short rings (two to a CU); eighths always, in
@@ -190,14 +195,12 @@ void launch_wt_parts(WtOp<T> op, int N, const E& e, hipStream_t s, int prof_cls 
 template <typename T, class E1, class E2>
 void launch_wt2(WtOp<T> op1, int N1, const E1& e1, WtOp<T> op2, int N2, const E2& e2, hipStream_t s,
                 int prof_cls = PROF_NONE) {
-  with_wt(op1.M, N1 + N2, [&](auto wt) {
+  with_wt<5>(op1.M, N1 + N2, [&](auto wt) {
     using WT = decltype(wt);
-    if constexpr (WT::NA <= 4) {
-      op1.nx = N1 / WT::COLS;
-      op2.nx = N2 / WT::COLS;
-      launch_k(prof_cls, k_wt2<T, WT, E1, E2>, dim3(op1.nx + op2.nx, cdiv(op1.M, WT::ROWS)), dim3(64), 0, s, op1, e1,
-               op2, e2);
-    }
+    op1.nx = N1 / WT::COLS;
+    op2.nx = N2 / WT::COLS;
+    launch_k(prof_cls, k_wt2<T, WT, E1, E2>, dim3(op1.nx + op2.nx, cdiv(op1.M, WT::ROWS)), dim3(64), 0, s, op1, e1, op2,
+             e2);
   });
 }
 // What rides in a decode step's refine: the W_O product in its first launch (both read o_cat), and the

@@ -259,7 +259,7 @@ static __global__ __launch_bounds__(64 * WT_PARTS) void k_wt_ksplit(WtOp<T> op, 
 // out[M, N] = the product
 template <typename T, int SUM_> struct WtStore {
   static constexpr int SUM = SUM_;
-  static constexpr bool TALL = false;
+  static constexpr int TILES = 5;   // forms with_wt may choose
   const T* W;
   long ldw;
   T* out;
@@ -290,7 +290,7 @@ template <typename T, int SUM_> struct WtStore {
 // act[M, H] = silu(x W1^T) (x W3^T): a tile's first half of columns from W1, the second the same from W3
 template <typename T> struct WtSwiGLU {
   static constexpr int SUM = WT_QUARTERS;
-  static constexpr bool TALL = true;   // 64-row tiles too (with_wt)
+  static constexpr int TILES = 6;
   const T* W1;
   const T* W3;
   long ldw;
@@ -321,7 +321,7 @@ template <typename T> struct WtSwiGLU {
 // the projection (EpiProj without the value norm): q / k / v tiles hold 8 CT RoPE pairs of one head
 template <typename T, int DH, bool DEVPOS> struct WtProj {
   static constexpr int SUM = WT_CHAIN;
-  static constexpr bool TALL = false;
+  static constexpr int TILES = 4;
   const T* W;   // [nseg d, d]
   EpiProj<T, DH, DEVPOS> e;
   template <class WT> struct Pre {
@@ -401,7 +401,7 @@ template <typename T, int DH, bool DEVPOS> struct WtProj {
 // V columns (of each section) of one row, V so that the wave's lanes are used.
 template <typename T, int DH, bool DEVPOS> struct WtSweep1 {
   static constexpr int SUM = WT_CHAIN;
-  static constexpr bool TALL = false;
+  static constexpr int TILES = 4;
   typedef EpiSweep1<T, DH, 1, DEVPOS> Epi;
   const T* W;   // [4d, d], packed
   Epi e;
@@ -511,7 +511,7 @@ template <typename T, int DH, bool DEVPOS> struct WtSweep1 {
 // sweep GEMM 2 (EpiSweep2): items of V columns of one row
 template <typename T, int DH, bool DEVPOS> struct WtSweep2 {
   static constexpr int SUM = WT_CHAIN;
-  static constexpr bool TALL = false;
+  static constexpr int TILES = 3;
   typedef EpiSweep2<T, DH, DEVPOS> Epi;
   const T* W;   // [d, d]
   Epi e;

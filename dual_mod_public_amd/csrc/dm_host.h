@@ -308,8 +308,9 @@ void launch_gemm_auto(const SA& sa, const SB& sb, int M, int N, int K, const EPI
 
 // 128 x 128 blocks of four waves. With more blocks than CUs (a layer-batched launch always) two 32 KB
 // direct-to-LDS stages, so that two blocks share a CU and one's loads and LDS reads run under the
-// other's MFMAs; else three, one block's loads further ahead. M x N x K = 3072 x 5120 x 1024 (960 blocks):
-// 55.7 us with three stages, 41.7 with two.
+// other's MFMAs; else three, one block's loads further ahead. Three stages / two, us, M x N x K: 3072 x 5120 x
+// 1024 (960 blocks) 55.7 / 41.7; 3000 x 2048 x 2048 (384) 43.5 / 33.0; 8200 x 1024 x 2816 (520) 85 / 81; 2000 x
+// 2944 x 512 (368) 17.0 / 13.7.
 inline bool two_stages_128(long blocks) { return launch_log() != nullptr || blocks > 256; }
 template <typename T, int WM, int WN, class SA, class SB, class EPI>
 void launch_gemm_128(const SA& sa, const SB& sb, int M, int N, int K, const EPI& epi, hipStream_t s,

@@ -12,12 +12,12 @@
 // of a CU). The tile is chosen (with_wt) so that the waves spread over the CUs.
 // Measured on MI355X (K = 1024, weights from HBM, plain store; launch alone 2.3 us):
 //   M =   8, N = 4096: 3.9 us, N = 6144: 4.3     (64 x 64 block tiles in place: 12.1, 9.5 with their epilogues)
-//   M =  64, N = 4096: 5.8;  M = 128: 6.7;  M = 256: 9.0     (64 x 128 blocks in place: 12.6, 12.6, 13.1)
-// From M = 512 on (13.6 us) sharing the operands between a block's waves wins (13.0 with its epilogue).
-// The order of an output's sum over k is fixed by the product, never by the rows of the call or the
-// tile that computes it, so a row's result is the same in every batch (WtSum): the products that larger
-// calls run on the tiled GEMMs sum as those do, one chain over ascending 32-wide MFMA steps; a step's W_O
-// and MLP products sum partial chains.
+//   M =  64, N = 4096: 5.8;  M = 128: 6.7;  M = 256: 9.0
+// With more rows or wider operands sharing them between a block's waves wins; each product's rule says where.
+// The order of an output's sum over k is fixed by the product, not by the tile that computes it (WtSum): the
+// products that larger calls run on the tiled GEMMs sum as those do, one chain over ascending 32-wide MFMA
+// steps; a step's W_O and MLP products, of 1 to ROWS_MAX rows, sum partial chains (a W_O of more rows one
+// chain). So a row's result is the same in every batch of either kind.
 //
 // An epilogue chooses the 16 CT weight rows of a tile (wrow), so that its items are complete inside
 // the tile (a RoPE pair, a key's candidate and gate halves), gathers its inputs ahead of the k-loop

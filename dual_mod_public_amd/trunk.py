@@ -19,9 +19,10 @@ whole step can be captured as one HIP graph and replayed (graphs.py:513-576 capt
 Numerics follow the reference's bf16 engine (autocast): the residual stream and every matrix
 product in the compute dtype with fp32 accumulation, RMSNorm statistics, softmax and the loss in
 fp32, weight gradients accumulated in fp32. The DM attention and the SwiGLU MLP sublayer run in
-libdm_hip.so (dm_layer_fwd / dm_layer_bwd, dm_mlp_fwd / dm_mlp_bwd); the embedding gather, the
-tied head's products (hipBLASLt through torch, the weight gradient with fp32 outputs) and the loss
-in torch. With ``dtype=torch.float32`` the whole step is fp32 (the parity tests).
+libdm_hip.so (dm_layer_fwd / dm_layer_bwd, dm_mlp_fwd / dm_mlp_bwd), as do the loss rows with their
+gradient, the sums over rows and the embedding's gradient; the embedding gather, the tied head's
+products (hipBLASLt through torch, the weight gradient with fp32 outputs) and norm_f's rows in torch.
+With ``dtype=torch.float32`` the whole step is fp32 (the parity tests).
 
 Layer by layer (default), each layer's forward keeps its cells' sweep states in an HBM tape while
 ``tape_budget`` bytes allow (the backward then skips the recompute), the remaining layers recompute
@@ -317,9 +318,8 @@ class HipTrunk:
         """norm_f, the tied head and the mean cross entropy (ignore_index -1, model.py:279-281), with
         its gradient: the loss's softmax gradient needs nothing but the logits, so the head's VJP runs
         with its forward, chunk by chunk of rows (the reference's loss_chunk, graphs.py:322-341). The sums
-        over rows are the library's own (libdm_hip.so): torch's
-        split a long column over blocks and clear their counters with memsets, which a captured step
-        would hold as nodes."""
+        over rows run in libdm_hip.so: torch's split a long column over blocks and clear their counters
+        with memsets, which a captured step would hold as nodes."""
         m = self.m
         M, d = self.B * self.T, self.cfg.d_model
         x = self.xs[-1].view(M, d)
@@ -389,8 +389,8 @@ class HipTrunk:
         return self
 
     def train_step(self, idx, targets):
-        """Forward + backward of the batch (idx, targets [B, T] token ids; targets -1 are ignored, one >=
-        vocab_size makes the loss NaN; an id outside the table is left out of the embedding gradient).
+        """Forward + backward of the batch (idx [B, T] token ids of the table; targets [B, T], of which
+        -1 is ignored and one >= vocab_size makes the loss NaN).
         Returns the loss (a static device scalar, overwritten by the next step); the gradients are
         the views ``grad[name]`` of the flat buffer ``flat`` (``to_param_grads`` copies them into
         the parameters' .grad)."""
